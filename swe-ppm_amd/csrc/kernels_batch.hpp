@@ -321,9 +321,10 @@ __device__ __forceinline__ TileLanes tile_lanes(const BatchBlockDesc& d, int til
 // Same edge order and arithmetic as the single-block strip sweep: the lanes
 // of a group own rows 62*yt+1 .. 62*yt+62 (rows r = 1..62; r = 0 and the
 // group's top lane are halo) and march over columns 1+xs*XS .. xs*XS+n.
-template <int S, int XS>
-__device__ __forceinline__ float strip_sums(const BatchSolver<S>& solver, const StateView& v, const SumsView& sums,
-                                            const TileLanes& t) {
+template <int S, int XS, bool N>
+__device__ __forceinline__ bool strip_sums(const BatchSolver<S>& solver, const StateView& v, const SumsView& sums,
+                                           const TileLanes& t, unsigned* smax) {
+    using A = CellMath<N>;
     const int y = kStripRows * t.yt + t.r;
     const bool rowValid = y <= v.ny + 1;
     const int yc = rowValid ? y : v.ny + 1;
@@ -332,36 +333,44 @@ __device__ __forceinline__ float strip_sums(const BatchSolver<S>& solver, const 
     const bool hEdgeValid = (t.r <= kStripRows) && (y <= v.ny);
     const int x0 = 1 + t.xs0 * XS;  // the item's first column; packed groups add a per-lane offset
     const int n = tile_columns(t, v.nx, XS);
-    const size_t colOff = (size_t)(t.xs - t.xs0) * XS * v.pitch;
-    size_t o = idx(v, x0 - 1, yc) + colOff;
-    CellQ cq = cell_q(v.h[o], v.hu[o], v.hv[o], v.b[o]);
-    o += v.pitch;
-    CellQ nq = cell_q(v.h[o], v.hu[o], v.hv[o], v.b[o]);
-    const dev::EdgeOut e = solver.solve(cq.xside(), nq.xside());
+    const int colOff = (t.xs - t.xs0) * XS * v.pitch;
+    auto load = [&](int x) -> CellQ {
+        const size_t c = (size_t)x * v.pitch;
+        const unsigned ro = lane_bytes(yc + colOff);
+        return cell_q<A>(col_get(v.h, c, ro), col_get(v.hu, c, ro), col_get(v.hv, c, ro), col_get(v.b, c, ro));
+    };
+    CellQ cq = load(x0 - 1);
+    CellQ nq = load(x0);
+    bool outside = outside_range<N>(cq) || outside_range<N>(nq);
+    const dev::EdgeOut e = solver.template solve<A>(cq.xside(), nq.xside());
     float carryH = e.hR, carryHu = e.huR;
     float smaxv = rowInterior ? e.speed : 0.f;
     for (int k = 0; k < n; ++k) {
         const int x = x0 + k;
         cq = nq;
-        o += v.pitch;
-        nq = cell_q(v.h[o], v.hu[o], v.hv[o], v.b[o]);
-        const dev::EdgeOut ev = solver.solve(cq.xside(), nq.xside());
+        nq = load(x + 1);
+        outside = outside || outside_range<N>(nq);
+        const dev::EdgeOut ev = solver.template solve<A>(cq.xside(), nq.xside());
         if (rowInterior) smaxv = dev::smax(smaxv, ev.speed);
-        const dev::EdgeOut eh = solver.solve(cq.yside(), cq.yside_from_lane_above());
+        const dev::EdgeOut eh = solver.template solve<A>(cq.yside(), cq.yside_from_lane_above());
         if (hEdgeValid) smaxv = dev::smax(smaxv, eh.speed);
         const float aH = __shfl_up(eh.hR, 1, 64);
         const float aHv = __shfl_up(eh.huR, 1, 64);
         if (owned) {
-            const size_t c = idx(v, x, y) + colOff;
-            sums.sx[c] = carryH + ev.hL;
-            sums.su[c] = carryHu + ev.huL;
-            sums.sy[c] = aH + eh.hL;
-            sums.sv[c] = aHv + eh.huL;
+            const size_t c = (size_t)x * v.pitch;
+            const unsigned ro = lane_bytes(y + colOff);
+            col_set(sums.sx, c, ro, carryH + ev.hL);
+            col_set(sums.su, c, ro, carryHu + ev.huL);
+            col_set(sums.sy, c, ro, aH + eh.hL);
+            col_set(sums.sv, c, ro, aHv + eh.huL);
         }
         carryH = ev.hR;
         carryHu = ev.huR;
     }
-    return wave_max(smaxv);
+    if (N && __any(outside)) return false;
+    smaxv = wave_max(smaxv);
+    if ((threadIdx.x & 63) == 0) atomicMax(smax, __float_as_uint(smaxv));
+    return true;
 }
 
 template <int S, int XS>
@@ -381,9 +390,11 @@ __global__ __launch_bounds__(256) void batch_sweep_kernel(BatchArena A, const Ba
         const int blk = code >> kTileBits;
         const int tile = code & ((1 << kTileBits) - 1);
         const BatchBlockDesc& d = D[blk];
-        const StateView v = batch_view(A, d, st[blk].cur);
-        const float m = strip_sums<S, XS>(solver, v, batch_sums(A, d, 0), tile_lanes(d, tile, lane));
-        if (lane == 0) atomicMax(&st[blk].smax, __float_as_uint(m));
+        const StateView v = batch_view(A, d, __builtin_amdgcn_readfirstlane(st[blk].cur));
+        const SumsView sums = batch_sums(A, d, 0);
+        run_tile<BatchSolver<S>, 0>(lane, [&](auto form, int l) {
+            return strip_sums<S, XS, decltype(form)::value>(solver, v, sums, tile_lanes(d, tile, l), &st[blk].smax);
+        });
     }
 }
 
@@ -444,66 +455,16 @@ __global__ __launch_bounds__(256) void batch_apply_kernel(BatchArena A, const Ba
 // arithmetic as the single-block fused kernel, so sums and maxima equal the
 // sweep + apply pair.
 template <int S, int XS>
-__device__ __forceinline__ float fused_tile(const BatchSolver<S>& solver, const StateView& v, const StateView& o,
-                                            const SumsView& sIn, const SumsView& sOut, bool pend, float dt,
-                                            const int* bnd, const TileLanes& t, int blk, uint2* deferQ,
-                                            unsigned* deferCount, const BatchArena& A, const GhostJob* jb,
-                                            const GhostGeom* gg) {
+__device__ __forceinline__ void fused_tile(const BatchSolver<S>& solver, const StateView& v, const StateView& o,
+                                           const SumsView& sIn, const SumsView& sOut, bool pend, float dt,
+                                           const BatchBlockDesc& d, int tile, int blk, uint2* deferQ,
+                                           unsigned* deferCount, const BatchArena& A, const GhostJob* jb,
+                                           const GhostGeom* gg, unsigned* smax) {
     const int nx = v.nx, ny = v.ny;
     const float dtdx = dt / v.dx;
     const float dtdy = dt / v.dy;
-    const int y = kStripRows * t.yt + t.r;
-    const bool rowValid = y <= ny + 1;
-    const int yc = rowValid ? y : ny + 1;
-    const bool owned = (t.r >= 1) && (t.r <= kStripRows) && (y <= ny);
-    const bool rowInterior = (y >= 1) && (y <= ny);
-    const bool hEdgeValid = (t.r <= kStripRows) && (y <= ny);
-    const bool rowBottom = (y == 0);
-    const bool rowTop = (y == ny + 1);
-    const bool carryRow = owned || (rowBottom && t.r == 0) || (rowTop && t.r >= 1);
-    // the item's first column (uniform); a packed group's lanes address their
-    // own segment through a constant per-lane offset
-    const int x0 = 1 + t.xs0 * XS;
-    const int n = tile_columns(t, nx, XS);
-    const size_t colOff = (size_t)(t.xs - t.xs0) * XS * v.pitch;
-    const size_t rowC = (size_t)yc + colOff, rowY = (size_t)y + colOff;
-    auto at = [&](int x, size_t row) { return (size_t)x * v.pitch + row; };
-    const int tB = bnd[BND_BOTTOM], tT = bnd[BND_TOP], tL = bnd[BND_LEFT], tR = bnd[BND_RIGHT];
+    const int tB = d.bnd[BND_BOTTOM], tT = d.bnd[BND_TOP], tL = d.bnd[BND_LEFT], tR = d.bnd[BND_RIGHT];
     auto ow = [](int t) { return t == OUTFLOW || t == WALL; };
-
-    auto load_updated = [&](int x) -> BQ3 {
-        const size_t c = at(x, rowC);
-        BQ3 q{v.h[c], v.hu[c], v.hv[c]};
-        // x is the item's column: a packed item's segments are all inner, so
-        // the test has the same outcome for every lane
-        if (pend && x >= 1 && x <= nx && rowInterior) {
-            const Cell u = update_cell(q.h, q.hu, q.hv, dtdx, dtdy, sIn.sx[c], sIn.sy[c], sIn.su[c], sIn.sv[c]);
-            q = BQ3{u.h, u.hu, u.hv};
-        }
-        return q;
-    };
-    auto fix_rows = [&](BQ3 q) -> BQ3 {
-        const float dh = __shfl_down(q.h, 1, 64), dhu = __shfl_down(q.hu, 1, 64), dhv = __shfl_down(q.hv, 1, 64);
-        const float uh = __shfl_up(q.h, 1, 64), uhu = __shfl_up(q.hu, 1, 64), uhv = __shfl_up(q.hv, 1, 64);
-        if (rowBottom && ow(tB)) q = BQ3{dh, dhu, (tB == WALL) ? -dhv : dhv};
-        if (rowTop && ow(tT)) q = BQ3{uh, uhu, (tT == WALL) ? -uhv : uhv};
-        return q;
-    };
-    auto fix_column = [&](BQ3 raw, BQ3 in, int type) -> BQ3 {
-        const float dh = __shfl_down(in.h, 1, 64), dhu = __shfl_down(in.hu, 1, 64), dhv = __shfl_down(in.hv, 1, 64);
-        const float uh = __shfl_up(in.h, 1, 64), uhu = __shfl_up(in.hu, 1, 64), uhv = __shfl_up(in.hv, 1, 64);
-        BQ3 q = raw;
-        if (rowInterior && ow(type)) q = BQ3{in.h, (type == WALL) ? -in.hu : in.hu, in.hv};
-        if (rowBottom) q = BQ3{dh, dhu, dhv};
-        if (rowTop) q = BQ3{uh, uhu, uhv};
-        return q;
-    };
-    auto store = [&](int x, const BQ3& q) {
-        const size_t c = at(x, rowY);
-        o.h[c] = q.h;
-        o.hu[c] = q.hu;
-        o.hv[c] = q.hv;
-    };
 
     // CONNECT_WITHIN_RANK sides: this iteration's ghost-line step, in place
     // in v before the cells are loaded, each ghost cell by the tile that owns
@@ -513,107 +474,181 @@ __device__ __forceinline__ float fused_tile(const BatchSolver<S>& solver, const 
     // update only as a halo cell, whose edges add neither sums nor speeds
     // (the speeds of x-edges are taken on owned rows; every interior row is
     // owned by one strip, so the maximum is that over all edges).
-    bool ghostRows = false;
-    auto row_step = [&](int side, bool isRow) {
-        const GhostJob j = jb[side];
-        if (j.op == 0) return;
-        const GhostGeom g = gg[side];
-        const unsigned long long rows = __ballot(isRow);  // one lane per group of a packed item
-        const int groups = __popcll(rows), row = (side == BND_BOTTOM) ? 0 : ny + 1;
-        for (int p = (int)(threadIdx.x & 63); p < groups * n; p += 64) {
-            const int x = x0 + (p / n) * XS + p % n;
-            const size_t c = (size_t)x * v.pitch + row;
-            const BQ3 q = ghost_element(A, j, g, x - 1, BQ3{v.h[c], v.hu[c], v.hv[c]}, true);
+    {
+        const TileLanes t = tile_lanes(d, tile, threadIdx.x & 63);
+        const int y = kStripRows * t.yt + t.r;
+        const int x0 = 1 + t.xs0 * XS;
+        const int n = tile_columns(t, nx, XS);
+        bool ghostRows = false;
+        auto row_step = [&](int side, bool isRow) {
+            const GhostJob j = jb[side];
+            if (j.op == 0) return;
+            const GhostGeom g = gg[side];
+            const unsigned long long rows = __ballot(isRow);  // one lane per group of a packed item
+            const int groups = __popcll(rows), row = (side == BND_BOTTOM) ? 0 : ny + 1;
+            for (int p = (int)(threadIdx.x & 63); p < groups * n; p += 64) {
+                const int x = x0 + (p / n) * XS + p % n;
+                const size_t c = (size_t)x * v.pitch + row;
+                const BQ3 q = ghost_element(A, j, g, x - 1, BQ3{v.h[c], v.hu[c], v.hv[c]}, true);
+                v.h[c] = q.h;
+                v.hu[c] = q.hu;
+                v.hv[c] = q.hv;
+            }
+            ghostRows = true;
+        };
+        if (tB == CONNECT_WITHIN_RANK && t.yt == 0) row_step(BND_BOTTOM, y == 0);
+        if (tT == CONNECT_WITHIN_RANK && kStripRows * t.yt + 63 >= ny + 1) row_step(BND_TOP, y == ny + 1);
+        auto column_step = [&](int side, int x) {
+            const GhostJob j = jb[side];
+            if (j.op == 0 || t.r < 1 || t.r > kStripRows || y > ny) return;  // owned rows
+            const size_t c = (size_t)x * v.pitch + y;
+            const BQ3 q = ghost_element(A, j, gg[side], y - 1, BQ3{v.h[c], v.hu[c], v.hv[c]}, true);
             v.h[c] = q.h;
             v.hu[c] = q.hu;
             v.hv[c] = q.hv;
+        };
+        // (the first and last segments are never packed)
+        if (t.first && tL == CONNECT_WITHIN_RANK) column_step(BND_LEFT, 0);
+        if (t.last && tR == CONNECT_WITHIN_RANK) column_step(BND_RIGHT, nx + 1);
+        if (ghostRows) {  // other lanes of the wave load the row cells
+            __builtin_amdgcn_s_waitcnt(0 | (0x7 << 4) | (0xf << 8));  // vmcnt(0)
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         }
-        ghostRows = true;
-    };
-    if (tB == CONNECT_WITHIN_RANK && t.yt == 0) row_step(BND_BOTTOM, rowBottom);
-    if (tT == CONNECT_WITHIN_RANK && kStripRows * t.yt + 63 >= ny + 1) row_step(BND_TOP, rowTop);
-    auto column_step = [&](int side, int x) {
-        const GhostJob j = jb[side];
-        if (j.op == 0 || !owned) return;
-        const size_t c = at(x, rowC);
-        const BQ3 q = ghost_element(A, j, gg[side], y - 1, BQ3{v.h[c], v.hu[c], v.hv[c]}, true);
-        v.h[c] = q.h;
-        v.hu[c] = q.hu;
-        v.hv[c] = q.hv;
-    };
-    if (t.first && tL == CONNECT_WITHIN_RANK) column_step(BND_LEFT, 0);
-    if (t.last && tR == CONNECT_WITHIN_RANK) column_step(BND_RIGHT, nx + 1);
-    if (ghostRows) {  // other lanes of the wave load the row cells
-        __builtin_amdgcn_s_waitcnt(0 | (0x7 << 4) | (0xf << 8));  // vmcnt(0)
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     }
+    auto body = [&](auto form, int lane) -> bool {
+        constexpr bool N = decltype(form)::value;
+        using M = CellMath<N>;
+        const TileLanes t = tile_lanes(d, tile, lane);
+        const int y = kStripRows * t.yt + t.r;
+        const bool rowValid = y <= ny + 1;
+        const int yc = rowValid ? y : ny + 1;
+        const bool owned = (t.r >= 1) && (t.r <= kStripRows) && (y <= ny);
+        const bool rowInterior = (y >= 1) && (y <= ny);
+        const bool hEdgeValid = (t.r <= kStripRows) && (y <= ny);
+        const bool rowBottom = (y == 0);
+        const bool rowTop = (y == ny + 1);
+        const bool carryRow = owned || (rowBottom && t.r == 0) || (rowTop && t.r >= 1);
+        // the item's first column (uniform); a packed group's lanes address their
+        // own segment through a constant per-lane offset
+        const int x0 = 1 + t.xs0 * XS;
+        const int n = tile_columns(t, nx, XS);
+        const int colOff = (t.xs - t.xs0) * XS * v.pitch;
+        const int rowC = yc + colOff, rowY = y + colOff;
+        auto col = [&](int x) { return (size_t)x * v.pitch; };
 
-    BQ3 cur = fix_rows(load_updated(x0));
-    BQ3 prev = load_updated(x0 - 1);
-    if (t.first) prev = fix_column(prev, cur, tL);  // x0 == 1
-    if (t.first && carryRow) store(0, prev);
-    CellQ pq = cell_q(prev.h, prev.hu, prev.hv, v.b[at(x0 - 1, rowC)]);
-    CellQ cq = cell_q(cur.h, cur.hu, cur.hv, v.b[at(x0, rowC)]);
-    // deferred-edge entries: the lane's own column, the block in the high bits
-    const unsigned xLane = (unsigned)(t.xs - t.xs0) * XS, blkBits = (unsigned)blk << kDeferBlockShift;
-    dev::EdgeOut e = solver.solve(pq.xside(), cq.xside());
-    if constexpr (S == SOLVER_AUGRIE_DEFER)  // edge (0|1): only the first segment's items have t.first
-        e = defer_edge(e, owned && t.first, make_uint2(blkBits, (unsigned)y), deferQ, deferCount);
-    float carryH = e.hR, carryHu = e.huR;
-    float smaxv = owned ? e.speed : 0.f;
-    // Column x+1's loads are issued one column ahead (a software pipeline),
-    // as in the single-block fused kernel; past the tile they read column
-    // nx + 1 at most (a packed item's segments are inner ones) and are not
-    // used.  Not for the deferring sweep, which has no registers to spare.
-    struct Raw {
-        float h, hu, hv, sx, sy, su, sv, b;
-    };
-    auto load_raw = [&](int x) -> Raw {
-        const size_t c = at(min(x, nx + 1), rowC);
-        return Raw{v.h[c], v.hu[c], v.hv[c], sIn.sx[c], sIn.sy[c], sIn.su[c], sIn.sv[c], v.b[c]};
-    };
-    constexpr bool kAhead = S != SOLVER_AUGRIE_DEFER;
-    Raw ahead{};
-    if constexpr (kAhead) ahead = load_raw(x0 + 1);
-    for (int k = 0; k < n; ++k) {
-        const int x = x0 + k;
-        const bool rightGhost = t.last && k == n - 1;  // x + 1 == nx + 1
-        const Raw r = kAhead ? ahead : load_raw(x + 1);
-        if constexpr (kAhead) ahead = load_raw(x + 2);
-        BQ3 nxt{r.h, r.hu, r.hv};
-        if (pend && x + 1 <= nx && rowInterior) {
-            const Cell u = update_cell(nxt.h, nxt.hu, nxt.hv, dtdx, dtdy, r.sx, r.sy, r.su, r.sv);
-            nxt = BQ3{u.h, u.hu, u.hv};
+        auto load_updated = [&](int x) -> BQ3 {
+            const size_t c = col(x);
+            const unsigned ro = lane_bytes(rowC);
+            BQ3 q{col_get(v.h, c, ro), col_get(v.hu, c, ro), col_get(v.hv, c, ro)};
+            // x is the item's column: a packed item's segments are all inner, so
+            // the test has the same outcome for every lane
+            if (pend && x >= 1 && x <= nx && rowInterior) {
+                const Cell u = update_cell(q.h, q.hu, q.hv, dtdx, dtdy, col_get(sIn.sx, c, ro), col_get(sIn.sy, c, ro),
+                                           col_get(sIn.su, c, ro), col_get(sIn.sv, c, ro));
+                q = BQ3{u.h, u.hu, u.hv};
+            }
+            return q;
+        };
+        auto fix_rows = [&](BQ3 q) -> BQ3 {
+            const float dh = __shfl_down(q.h, 1, 64), dhu = __shfl_down(q.hu, 1, 64), dhv = __shfl_down(q.hv, 1, 64);
+            const float uh = __shfl_up(q.h, 1, 64), uhu = __shfl_up(q.hu, 1, 64), uhv = __shfl_up(q.hv, 1, 64);
+            if (rowBottom && ow(tB)) q = BQ3{dh, dhu, (tB == WALL) ? -dhv : dhv};
+            if (rowTop && ow(tT)) q = BQ3{uh, uhu, (tT == WALL) ? -uhv : uhv};
+            return q;
+        };
+        auto fix_column = [&](BQ3 raw, BQ3 in, int type) -> BQ3 {
+            const float dh = __shfl_down(in.h, 1, 64), dhu = __shfl_down(in.hu, 1, 64), dhv = __shfl_down(in.hv, 1, 64);
+            const float uh = __shfl_up(in.h, 1, 64), uhu = __shfl_up(in.hu, 1, 64), uhv = __shfl_up(in.hv, 1, 64);
+            BQ3 q = raw;
+            if (rowInterior && ow(type)) q = BQ3{in.h, (type == WALL) ? -in.hu : in.hu, in.hv};
+            if (rowBottom) q = BQ3{dh, dhu, dhv};
+            if (rowTop) q = BQ3{uh, uhu, uhv};
+            return q;
+        };
+        auto store = [&](int x, const BQ3& q) {
+            const size_t c = col(x);
+            const unsigned ro = lane_bytes(rowY);
+            col_set(o.h, c, ro, q.h);
+            col_set(o.hu, c, ro, q.hu);
+            col_set(o.hv, c, ro, q.hv);
+        };
+
+        BQ3 cur = fix_rows(load_updated(x0));
+        BQ3 prev = load_updated(x0 - 1);
+        if (t.first) prev = fix_column(prev, cur, tL);  // x0 == 1
+        if (t.first && carryRow) store(0, prev);
+        const CellQ pq = cell_q<M>(prev.h, prev.hu, prev.hv, col_get(v.b, col(x0 - 1), lane_bytes(rowC)));
+        CellQ cq = cell_q<M>(cur.h, cur.hu, cur.hv, col_get(v.b, col(x0), lane_bytes(rowC)));
+        // deferred-edge entries: the lane's own column, the block in the high bits
+        const unsigned xLane = (unsigned)(t.xs - t.xs0) * XS, blkBits = (unsigned)blk << kDeferBlockShift;
+        bool outside = outside_range<N>(pq) || outside_range<N>(cq);
+        dev::EdgeOut e = solver.template solve<M>(pq.xside(), cq.xside());
+        if constexpr (S == SOLVER_AUGRIE_DEFER)  // edge (0|1): only the first segment's items have t.first
+            e = defer_edge(e, owned && t.first, make_uint2(blkBits, (unsigned)y), deferQ, deferCount);
+        float carryH = e.hR, carryHu = e.huR;
+        float smaxv = owned ? e.speed : 0.f;
+        // Column x+1's loads are issued one column ahead (a software pipeline),
+        // as in the single-block fused kernel; past the tile they read column
+        // nx + 1 at most (a packed item's segments are inner ones) and are not
+        // used.  Not for the deferring sweep, which has no registers to spare.
+        struct Raw {
+            float h, hu, hv, sx, sy, su, sv, b;
+        };
+        auto load_raw = [&](int x) -> Raw {
+            const size_t c = col(min(x, nx + 1));
+            const unsigned ro = lane_bytes(rowC);
+            return Raw{col_get(v.h, c, ro),    col_get(v.hu, c, ro),   col_get(v.hv, c, ro),   col_get(sIn.sx, c, ro),
+                       col_get(sIn.sy, c, ro), col_get(sIn.su, c, ro), col_get(sIn.sv, c, ro), col_get(v.b, c, ro)};
+        };
+        constexpr bool kAhead = S != SOLVER_AUGRIE_DEFER;
+        Raw ahead{};
+        if constexpr (kAhead) ahead = load_raw(x0 + 1);
+        for (int k = 0; k < n; ++k) {
+            const int x = x0 + k;
+            const bool rightGhost = t.last && k == n - 1;  // x + 1 == nx + 1
+            const Raw r = kAhead ? ahead : load_raw(x + 1);
+            if constexpr (kAhead) ahead = load_raw(x + 2);
+            BQ3 nxt{r.h, r.hu, r.hv};
+            if (pend && x + 1 <= nx && rowInterior) {
+                const Cell u = update_cell(nxt.h, nxt.hu, nxt.hv, dtdx, dtdy, r.sx, r.sy, r.su, r.sv);
+                nxt = BQ3{u.h, u.hu, u.hv};
+            }
+            nxt = fix_rows(nxt);
+            if (rightGhost) nxt = fix_column(nxt, cur, tR);
+            const CellQ nq = cell_q<M>(nxt.h, nxt.hu, nxt.hv, r.b);
+            outside = outside || outside_range<N>(nq);
+            if (carryRow) store(x, cur);
+            if (rightGhost && carryRow) store(nx + 1, nxt);
+            dev::EdgeOut ev = solver.template solve<M>(cq.xside(), nq.xside());
+            if constexpr (S == SOLVER_AUGRIE_DEFER)
+                ev = defer_edge(ev, owned, make_uint2(blkBits | ((unsigned)x + xLane), (unsigned)y), deferQ, deferCount);
+            if (owned) smaxv = dev::smax(smaxv, ev.speed);
+            dev::EdgeOut eh = solver.template solve<M>(cq.yside(), cq.yside_from_lane_above());
+            if constexpr (S == SOLVER_AUGRIE_DEFER)
+                eh = defer_edge(eh, owned || y == 0, make_uint2(kDeferY | blkBits | ((unsigned)x + xLane), (unsigned)y),
+                                deferQ, deferCount);
+            if (hEdgeValid) smaxv = dev::smax(smaxv, eh.speed);
+            const float aH = __shfl_up(eh.hR, 1, 64);
+            const float aHv = __shfl_up(eh.huR, 1, 64);
+            if (owned) {
+                const size_t c = col(x);
+                const unsigned ro = lane_bytes(rowY);
+                col_set(sOut.sx, c, ro, carryH + ev.hL);
+                col_set(sOut.su, c, ro, carryHu + ev.huL);
+                col_set(sOut.sy, c, ro, aH + eh.hL);
+                col_set(sOut.sv, c, ro, aHv + eh.huL);
+            }
+            carryH = ev.hR;
+            carryHu = ev.huR;
+            cur = nxt;
+            cq = nq;
         }
-        nxt = fix_rows(nxt);
-        if (rightGhost) nxt = fix_column(nxt, cur, tR);
-        const CellQ nq = cell_q(nxt.h, nxt.hu, nxt.hv, r.b);
-        if (carryRow) store(x, cur);
-        if (rightGhost && carryRow) store(nx + 1, nxt);
-        dev::EdgeOut ev = solver.solve(cq.xside(), nq.xside());
-        if constexpr (S == SOLVER_AUGRIE_DEFER)
-            ev = defer_edge(ev, owned, make_uint2(blkBits | ((unsigned)x + xLane), (unsigned)y), deferQ, deferCount);
-        if (owned) smaxv = dev::smax(smaxv, ev.speed);
-        dev::EdgeOut eh = solver.solve(cq.yside(), cq.yside_from_lane_above());
-        if constexpr (S == SOLVER_AUGRIE_DEFER)
-            eh = defer_edge(eh, owned || y == 0, make_uint2(kDeferY | blkBits | ((unsigned)x + xLane), (unsigned)y),
-                            deferQ, deferCount);
-        if (hEdgeValid) smaxv = dev::smax(smaxv, eh.speed);
-        const float aH = __shfl_up(eh.hR, 1, 64);
-        const float aHv = __shfl_up(eh.huR, 1, 64);
-        if (owned) {
-            const size_t c = at(x, rowY);
-            sOut.sx[c] = carryH + ev.hL;
-            sOut.su[c] = carryHu + ev.huL;
-            sOut.sy[c] = aH + eh.hL;
-            sOut.sv[c] = aHv + eh.huL;
-        }
-        carryH = ev.hR;
-        carryHu = ev.huR;
-        cur = nxt;
-        cq = nq;
-    }
-    return wave_max(smaxv);
+        if (N && __any(outside)) return false;
+        smaxv = wave_max(smaxv);
+        if ((threadIdx.x & 63) == 0) atomicMax(smax, __float_as_uint(smaxv));
+        return true;
+    };
+    run_tile<BatchSolver<S>, 0>(threadIdx.x & 63, body);
 }
 
 // direct = 0: persistent grid, waves pull items until the queue is drained;
@@ -622,9 +657,11 @@ __device__ __forceinline__ float fused_tile(const BatchSolver<S>& solver, const 
 // blockIdx.x * kWavesPerGroup + wave or leaves.  An item is a strip tile of a
 // block that computes this iteration or, for LTS, the ghost-line step of a
 // side of a block that waits (tile kLineTile + side).
-// Six waves per SIMD (at most 80 VGPRs, no spills) with the early column
-// loads; at seven without them the LTS tiling ran 5% and the ensemble 4%
-// slower.  The deferring sweep runs at six without the early loads (77
+// At least six waves per SIMD with the early column loads (AugRie: 69
+// registers, seven waves).  The tile's two forms (run_tile) and the column
+// addresses in scalar registers took the 28-block LTS tiling from 132 to 119 ms
+// for 6 macro steps and the 512-instance ensemble from 149 to 136 ms for 150
+// steps, transfers included.  The deferring sweep runs at six without the early loads (77
 // registers; at seven it spilled), the learned-middle-state solver at its
 // own register budget (its network call needs far more).
 template <int S, int XS>
@@ -650,23 +687,17 @@ batch_fused_kernel(BatchArena A, const BatchBlockDesc* D, BatchBlockState* st, B
         const int sidx = __builtin_amdgcn_readfirstlane(st[blk].sidx);
         const bool pend = __builtin_amdgcn_readfirstlane(st[blk].pend) != 0;
         const float dt = st[blk].maxTimestep;
-        const float m = fused_tile<S, XS>(solver, batch_view(A, d, cur), batch_view(A, d, cur ^ 1),
-                                          batch_sums(A, d, sidx), batch_sums(A, d, sidx ^ 1), pend, dt, d.bnd,
-                                          tile_lanes(d, tile, lane), blk, deferQ, &G->deferCount, A, jobs + 4 * blk,
-                                          geo + 4 * blk);
-        if (lane == 0) atomicMax(&st[blk].smax, __float_as_uint(m));
+        fused_tile<S, XS>(solver, batch_view(A, d, cur), batch_view(A, d, cur ^ 1), batch_sums(A, d, sidx),
+                          batch_sums(A, d, sidx ^ 1), pend, dt, d, tile, blk, deferQ, &G->deferCount, A,
+                          jobs + 4 * blk, geo + 4 * blk, &st[blk].smax);
     };
-    if (direct) {
-        const int item = blockIdx.x * kWavesPerGroup + wave;  // uniform per wave
-        if (item < count) run_item(item);
-        return;
-    }
+    // one loop for both forms, so that the tile exists once in the code
     __shared__ int sBase;
     for (;;) {
-        const int item = next_items(&G->head, &sBase) + wave;
-        if (item - wave >= count) break;  // uniform over the workgroup
-        if (item >= count) continue;
-        run_item(item);
+        const int item = (direct ? blockIdx.x * kWavesPerGroup : next_items(&G->head, &sBase)) + wave;
+        if (item - wave >= count) return;  // uniform over the workgroup
+        if (item < count) run_item(item);
+        if (direct) return;
     }
 }
 

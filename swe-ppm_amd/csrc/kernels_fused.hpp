@@ -153,8 +153,7 @@ template <int S, int XS, int V>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(fused_waves_per_simd(S), 8))) void fused_u_kernel(
     StateView v, FusedIO io, BoundaryInfo bi, DeviceCtl* ctl, int slotIn, int slotOut, int slotClear, float* dtLog,
     int logIdx) {
-    const int lane = threadIdx.x & 63;
-    const int wave = blockIdx.x * kWavesPerGroup + (threadIdx.x >> 6);
+    const int wave = __builtin_amdgcn_readfirstlane(blockIdx.x * kWavesPerGroup + (threadIdx.x >> 6));
     const int nyt = (v.ny + kStripRows - 1) / kStripRows;
     const int nxs = (v.nx + XS - 1) / XS;
     const int nx = v.nx, ny = v.ny;
@@ -173,7 +172,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(fused_waves
     const int items = nyt * nxs;
     int item = wave, first = 0, ncols = XS;
     if (kRecord && io.list) {
-        const int e = listed_item(io, plan_groups(nyt, nxs, XS / kQuietCols), wave);
+        const int e = __builtin_amdgcn_readfirstlane(listed_item(io, plan_groups(nyt, nxs, XS / kQuietCols), wave));
         if (e < 0) return;  // uniform per wave
         item = e >> 6;
         first = (e >> 3) & 7;
@@ -189,176 +188,192 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(fused_waves
 
     const float dtdx = dt / v.dx;
     const float dtdy = dt / v.dy;
-    const int y = kStripRows * yt + lane;
-    const bool rowValid = y <= ny + 1;
-    const int yc = rowValid ? y : ny + 1;
-    const bool owned = (lane >= 1) && (lane <= kStripRows) && (y <= ny);
-    const bool rowInterior = (y >= 1) && (y <= ny);
-    const bool hEdgeValid = (lane <= kStripRows) && (y <= ny);
-    const bool rowBottom = (y == 0);
-    const bool rowTop = (y == ny + 1);
-    const bool carryRow = owned || (rowBottom && lane == 0) || (rowTop && lane >= 1);
     const int x0 = 1 + xs * XS + first * kQuietCols;
     const int x1 = min(x0 + ncols - 1, nx);
     const int tB = bi.type[BND_BOTTOM], tT = bi.type[BND_TOP], tL = bi.type[BND_LEFT], tR = bi.type[BND_RIGHT];
 
-    // Q(k) of the cell (x, yc): interior cells updated, ghosts as stored
-    auto load_updated = [&](int x) -> Q3 {
-        const size_t c = idx(v, x, yc);
-        Q3 q{io.h[c], io.hu[c], io.hv[c]};
-        if (x >= 1 && x <= nx && rowInterior) {
-            const Cell u = update_cell(q.h, q.hu, q.hv, dtdx, dtdy, io.sIn.sx[c], io.sIn.sy[c], io.sIn.su[c],
-                                       io.sIn.sv[c]);
-            q = Q3{u.h, u.hu, u.hv};
-        }
-        return q;
-    };
-    // ghost rows of an interior column: the boundary value of the row next to
-    // it (lane+1 for the bottom row, lane-1 for the top row)
-    auto fix_rows = [&](Q3 q) -> Q3 {
-        const float dh = __shfl_down(q.h, 1, 64), dhu = __shfl_down(q.hu, 1, 64), dhv = __shfl_down(q.hv, 1, 64);
-        const float uh = __shfl_up(q.h, 1, 64), uhu = __shfl_up(q.hu, 1, 64), uhv = __shfl_up(q.hv, 1, 64);
-        if (rowBottom && is_ow(tB)) q = Q3{dh, dhu, (tB == WALL) ? -dhv : dhv};
-        if (rowTop && is_ow(tT)) q = Q3{uh, uhu, (tT == WALL) ? -uhv : uhv};
-        return q;
-    };
-    // a ghost column next to the interior column value `in` (same lane);
-    // corners take the diagonal interior cell (from the neighbouring lane)
-    auto fix_column = [&](Q3 raw, Q3 in, int type) -> Q3 {
-        const float dh = __shfl_down(in.h, 1, 64), dhu = __shfl_down(in.hu, 1, 64), dhv = __shfl_down(in.hv, 1, 64);
-        const float uh = __shfl_up(in.h, 1, 64), uhu = __shfl_up(in.hu, 1, 64), uhv = __shfl_up(in.hv, 1, 64);
-        Q3 q = raw;
-        if (rowInterior && is_ow(type)) q = Q3{in.h, (type == WALL) ? -in.hu : in.hu, in.hv};
-        if (rowBottom) q = Q3{dh, dhu, dhv};
-        if (rowTop) q = Q3{uh, uhu, uhv};
-        return q;
-    };
-    auto store = [&](int x, const Q3& q) {
-        const size_t c = idx(v, x, y);
-        io.hn[c] = q.h;
-        io.hun[c] = q.hu;
-        io.hvn[c] = q.hv;
-    };
+    auto tile = [&](auto form, int lane) -> bool {
+        constexpr bool N = decltype(form)::value;
+        using A = CellMath<N>;
+        const int y = kStripRows * yt + lane;
+        const bool rowValid = y <= ny + 1;
+        const int yc = rowValid ? y : ny + 1;
+        const bool owned = (lane >= 1) && (lane <= kStripRows) && (y <= ny);
+        const bool rowInterior = (y >= 1) && (y <= ny);
+        const bool hEdgeValid = (lane <= kStripRows) && (y <= ny);
+        const bool rowBottom = (y == 0);
+        const bool rowTop = (y == ny + 1);
+        const bool carryRow = owned || (rowBottom && lane == 0) || (rowTop && lane >= 1);
 
-    const float* B = v.b;
-    // columns x0-1 and x0
-    Q3 cur = fix_rows(load_updated(x0));
-    Q3 prev = load_updated(x0 - 1);
-    if (x0 == 1) prev = fix_column(prev, cur, tL);
-    if (x0 == 1 && carryRow) store(0, prev);
-    float cb = B[idx(v, x0 - 1, yc)];
-    float nb = B[idx(v, x0, yc)];
-
-    CellQ pq = cell_q(prev.h, prev.hu, prev.hv, cb);
-    CellQ cq = cell_q(cur.h, cur.hu, cur.hv, nb);
-    dev::EdgeOut e = solver.solve(pq.xside(), cq.xside());
-    // record tile of the columns being solved: a deferred edge touching it
-    // makes it not quiet; the halo edge (x0-1 | x0) counts for the first
-    bool loud = false;
-    if constexpr (S == SOLVER_AUGRIE_DEFER) {
-        loud = e.speed < 0.f;
-        e = defer_edge(e, owned && x0 == 1, make_uint2(0u, (unsigned)y), io.deferQ, &ctl->defer[slotOut]);
-    }
-    float carryH = e.hR, carryHu = e.huR;
-    // x-edges count on owned rows (each interior row is owned by one strip),
-    // so a record tile's maximum depends on its footprint only
-    float smaxTile = owned ? e.speed : 0.f;
-    // the segment's maximum over its record tiles, wave-uniform (float bits:
-    // non-negative floats order like unsigned integers)
-    unsigned smaxRun = 0u;
-    // kQuiet* bits of the record tile's parts whose owned sums were not all +0
-    unsigned loudParts = 0u;
-
-    // Column x+1's loads are issued one column ahead (a software pipeline):
-    // their latency overlaps column x's edges.  The loads past x1 + 1 read
-    // column nx + 1 at most and are not used.  Not for the learned middle
-    // state, whose network call leaves no registers for them.
-    struct Raw {
-        float h, hu, hv, sx, sy, su, sv, b;
-    };
-    auto load_raw = [&](int x) -> Raw {
-        const size_t c = idx(v, min(x, nx + 1), yc);
-        return Raw{io.h[c], io.hu[c], io.hv[c], io.sIn.sx[c], io.sIn.sy[c], io.sIn.su[c], io.sIn.sv[c], B[c]};
-    };
-    constexpr bool kAhead = S != SOLVER_AUGRIE_MLP && S != SOLVER_HYBRID && S != SOLVER_AUGRIE_DEFER;
-    Raw ahead{};
-    if constexpr (kAhead) ahead = load_raw(x0 + 1);
-    for (int x = x0; x <= x1; ++x) {
-        // column x+1 of Q(k)
-        const Raw r = kAhead ? ahead : load_raw(x + 1);
-        if constexpr (kAhead) ahead = load_raw(x + 2);
-        Q3 nxt{r.h, r.hu, r.hv};
-        if (x + 1 <= nx && rowInterior) {
-            const Cell u = update_cell(nxt.h, nxt.hu, nxt.hv, dtdx, dtdy, r.sx, r.sy, r.su, r.sv);
-            nxt = Q3{u.h, u.hu, u.hv};
-        }
-        nxt = fix_rows(nxt);
-        if (x + 1 == nx + 1) nxt = fix_column(nxt, cur, tR);
-        const CellQ nq = cell_q(nxt.h, nxt.hu, nxt.hv, r.b);
-
-        if (carryRow) store(x, cur);
-        if (x + 1 == nx + 1 && carryRow) store(nx + 1, nxt);
-
-        dev::EdgeOut ev = solver.solve(cq.xside(), nq.xside());
-        bool loudEdge = false;
-        if constexpr (S == SOLVER_AUGRIE_DEFER) {
-            loudEdge = ev.speed < 0.f;
-            ev = defer_edge(ev, owned, make_uint2((unsigned)x, (unsigned)y), io.deferQ, &ctl->defer[slotOut]);
-        }
-        if (owned) smaxTile = dev::smax(smaxTile, ev.speed);
-        dev::EdgeOut eh = solver.solve(cq.yside(), cq.yside_from_lane_above());
-        if constexpr (S == SOLVER_AUGRIE_DEFER) {
-            loud = loud || loudEdge || eh.speed < 0.f;
-            eh = defer_edge(eh, owned || y == 0, make_uint2((unsigned)x | kDeferY, (unsigned)y), io.deferQ,
-                            &ctl->defer[slotOut]);
-        }
-        if (hEdgeValid) smaxTile = dev::smax(smaxTile, eh.speed);
-        const float aH = __shfl_up(eh.hR, 1, 64);
-        const float aHv = __shfl_up(eh.huR, 1, 64);
-        if (owned) {
-            const size_t c = idx(v, x, y);
-            const float sx = carryH + ev.hL, su = carryHu + ev.huL, sy = aH + eh.hL, sv = aHv + eh.huL;
-            io.sOut.sx[c] = sx;
-            io.sOut.su[c] = su;
-            io.sOut.sy[c] = sy;
-            io.sOut.sv[c] = sv;
-            if constexpr (kRecord)
-                if ((__float_as_uint(sx) | __float_as_uint(su) | __float_as_uint(sy) | __float_as_uint(sv)) != 0u)
-                    loudParts |= kQuietAll | (lane == 1 ? kQuietBottom : 0u) | (lane == kStripRows ? kQuietTop : 0u) |
-                                 (((x - 1) & (kQuietCols - 1)) == 0 ? kQuietLeft : 0u) |
-                                 ((x & (kQuietCols - 1)) == 0 || x == nx ? kQuietRight : 0u);
-        }
-        carryH = ev.hR;
-        carryHu = ev.huR;
-        cur = nxt;
-        cq = nq;
-        // the end of a record tile: its parts' flags and its maximum.  A tile
-        // reports its right edge (x | x+1) and, first in a run, its left halo
-        // edge; the tile of column 1 always starts a run, so every x-edge is
-        // in some record, and each record's edges lie in its tile's footprint.
-        // A deferred edge at the boundary touches both tiles.
-        if (kRecord && ((x & (kQuietCols - 1)) == 0 || x == x1)) {  // uniform per wave
-            const float tileMax = wave_max(smaxTile);
-            smaxRun = max(smaxRun, __builtin_amdgcn_readfirstlane(__float_as_uint(tileMax)));
-            if (io.quiet) {
-                unsigned quiet = 0u;
-#pragma unroll
-                for (unsigned part = 1u; part <= kQuietRight; part <<= 1)
-                    if (!__any((loudParts & part) != 0u || loud)) quiet |= part;
-                if (lane == 0) {
-                    const int rec = slotNow + yt + nyt * ((x - 1) / kQuietCols);
-                    io.quiet[rec] = quiet;
-                    io.speed[rec] = tileMax;
-                }
+        // Q(k) of the cell (x, yc): interior cells updated, ghosts as stored
+        auto load_updated = [&](int x) -> Q3 {
+            const size_t c = (size_t)x * v.pitch;
+            const unsigned rc = lane_bytes(yc);
+            Q3 q{col_get(io.h, c, rc), col_get(io.hu, c, rc), col_get(io.hv, c, rc)};
+            if (x >= 1 && x <= nx && rowInterior) {
+                const Cell u = update_cell(q.h, q.hu, q.hv, dtdx, dtdy, col_get(io.sIn.sx, c, rc), col_get(io.sIn.sy, c, rc),
+                                           col_get(io.sIn.su, c, rc), col_get(io.sIn.sv, c, rc));
+                q = Q3{u.h, u.hu, u.hv};
             }
-            smaxTile = 0.f;
-            loud = loudEdge;
-            loudParts = 0u;
-        }
-    }
+            return q;
+        };
+        // ghost rows of an interior column: the boundary value of the row next to
+        // it (lane+1 for the bottom row, lane-1 for the top row)
+        auto fix_rows = [&](Q3 q) -> Q3 {
+            const float dh = __shfl_down(q.h, 1, 64), dhu = __shfl_down(q.hu, 1, 64), dhv = __shfl_down(q.hv, 1, 64);
+            const float uh = __shfl_up(q.h, 1, 64), uhu = __shfl_up(q.hu, 1, 64), uhv = __shfl_up(q.hv, 1, 64);
+            if (rowBottom && is_ow(tB)) q = Q3{dh, dhu, (tB == WALL) ? -dhv : dhv};
+            if (rowTop && is_ow(tT)) q = Q3{uh, uhu, (tT == WALL) ? -uhv : uhv};
+            return q;
+        };
+        // a ghost column next to the interior column value `in` (same lane);
+        // corners take the diagonal interior cell (from the neighbouring lane)
+        auto fix_column = [&](Q3 raw, Q3 in, int type) -> Q3 {
+            const float dh = __shfl_down(in.h, 1, 64), dhu = __shfl_down(in.hu, 1, 64), dhv = __shfl_down(in.hv, 1, 64);
+            const float uh = __shfl_up(in.h, 1, 64), uhu = __shfl_up(in.hu, 1, 64), uhv = __shfl_up(in.hv, 1, 64);
+            Q3 q = raw;
+            if (rowInterior && is_ow(type)) q = Q3{in.h, (type == WALL) ? -in.hu : in.hu, in.hv};
+            if (rowBottom) q = Q3{dh, dhu, dhv};
+            if (rowTop) q = Q3{uh, uhu, uhv};
+            return q;
+        };
+        auto store = [&](int x, const Q3& q) {
+            const size_t c = (size_t)x * v.pitch;
+            const unsigned ry = lane_bytes(y);
+            col_set(io.hn, c, ry, q.h);
+            col_set(io.hun, c, ry, q.hu);
+            col_set(io.hvn, c, ry, q.hv);
+        };
 
-    if constexpr (!kRecord) smaxRun = __float_as_uint(wave_max(smaxTile));
-    if (lane == 0) atomicMax(&ctl->smax[slotOut], smaxRun);
+        const float* B = v.b;
+        // columns x0-1 and x0
+        Q3 cur = fix_rows(load_updated(x0));
+        Q3 prev = load_updated(x0 - 1);
+        if (x0 == 1) prev = fix_column(prev, cur, tL);
+        if (x0 == 1 && carryRow) store(0, prev);
+        float cb = col_get(B, (size_t)(x0 - 1) * v.pitch, lane_bytes(yc));
+        float nb = col_get(B, (size_t)x0 * v.pitch, lane_bytes(yc));
+
+        const CellQ pq = cell_q<A>(prev.h, prev.hu, prev.hv, cb);
+        CellQ cq = cell_q<A>(cur.h, cur.hu, cur.hv, nb);
+        bool outside = outside_range<N>(pq) || outside_range<N>(cq);
+        dev::EdgeOut e = solver.template solve<A>(pq.xside(), cq.xside());
+        // record tile of the columns being solved: a deferred edge touching it
+        // makes it not quiet; the halo edge (x0-1 | x0) counts for the first
+        bool loud = false;
+        if constexpr (S == SOLVER_AUGRIE_DEFER) {
+            loud = e.speed < 0.f;
+            e = defer_edge(e, owned && x0 == 1, make_uint2(0u, (unsigned)y), io.deferQ, &ctl->defer[slotOut]);
+        }
+        float carryH = e.hR, carryHu = e.huR;
+        // x-edges count on owned rows (each interior row is owned by one strip),
+        // so a record tile's maximum depends on its footprint only
+        float smaxTile = owned ? e.speed : 0.f;
+        // the segment's maximum over its record tiles, wave-uniform (float bits:
+        // non-negative floats order like unsigned integers)
+        unsigned smaxRun = 0u;
+        // kQuiet* bits of the record tile's parts whose owned sums were not all +0
+        unsigned loudParts = 0u;
+
+        // Column x+1's loads are issued one column ahead (a software pipeline):
+        // their latency overlaps column x's edges.  The loads past x1 + 1 read
+        // column nx + 1 at most and are not used.  Not for the learned middle
+        // state: its network call and the deferring sweep's seven waves leave
+        // no registers for them.
+        struct Raw {
+            float h, hu, hv, sx, sy, su, sv, b;
+        };
+        auto load_raw = [&](int x) -> Raw {
+            const size_t c = (size_t)min(x, nx + 1) * v.pitch;
+            const unsigned rc = lane_bytes(yc);
+            return Raw{col_get(io.h, c, rc),      col_get(io.hu, c, rc),     col_get(io.hv, c, rc),     col_get(io.sIn.sx, c, rc),
+                       col_get(io.sIn.sy, c, rc), col_get(io.sIn.su, c, rc), col_get(io.sIn.sv, c, rc), col_get(B, c, rc)};
+        };
+        constexpr bool kAhead = S != SOLVER_AUGRIE_MLP && S != SOLVER_AUGRIE_DEFER;
+        Raw ahead{};
+        if constexpr (kAhead) ahead = load_raw(x0 + 1);
+        for (int x = x0; x <= x1; ++x) {
+            // column x+1 of Q(k)
+            const Raw r = kAhead ? ahead : load_raw(x + 1);
+            if constexpr (kAhead) ahead = load_raw(x + 2);
+            Q3 nxt{r.h, r.hu, r.hv};
+            if (x + 1 <= nx && rowInterior) {
+                const Cell u = update_cell(nxt.h, nxt.hu, nxt.hv, dtdx, dtdy, r.sx, r.sy, r.su, r.sv);
+                nxt = Q3{u.h, u.hu, u.hv};
+            }
+            nxt = fix_rows(nxt);
+            if (x + 1 == nx + 1) nxt = fix_column(nxt, cur, tR);
+            const CellQ nq = cell_q<A>(nxt.h, nxt.hu, nxt.hv, r.b);
+            outside = outside || outside_range<N>(nq);
+
+            if (carryRow) store(x, cur);
+            if (x + 1 == nx + 1 && carryRow) store(nx + 1, nxt);
+
+            dev::EdgeOut ev = solver.template solve<A>(cq.xside(), nq.xside());
+            bool loudEdge = false;
+            if constexpr (S == SOLVER_AUGRIE_DEFER) {
+                loudEdge = ev.speed < 0.f;
+                ev = defer_edge(ev, owned, make_uint2((unsigned)x, (unsigned)y), io.deferQ, &ctl->defer[slotOut]);
+            }
+            if (owned) smaxTile = dev::smax(smaxTile, ev.speed);
+            dev::EdgeOut eh = solver.template solve<A>(cq.yside(), cq.yside_from_lane_above());
+            if constexpr (S == SOLVER_AUGRIE_DEFER) {
+                loud = loud || loudEdge || eh.speed < 0.f;
+                eh = defer_edge(eh, owned || y == 0, make_uint2((unsigned)x | kDeferY, (unsigned)y), io.deferQ,
+                                &ctl->defer[slotOut]);
+            }
+            if (hEdgeValid) smaxTile = dev::smax(smaxTile, eh.speed);
+            const float aH = __shfl_up(eh.hR, 1, 64);
+            const float aHv = __shfl_up(eh.huR, 1, 64);
+            if (owned) {
+                const size_t c = (size_t)x * v.pitch;
+                const unsigned ry = lane_bytes(y);
+                const float sx = carryH + ev.hL, su = carryHu + ev.huL, sy = aH + eh.hL, sv = aHv + eh.huL;
+                col_set(io.sOut.sx, c, ry, sx);
+                col_set(io.sOut.su, c, ry, su);
+                col_set(io.sOut.sy, c, ry, sy);
+                col_set(io.sOut.sv, c, ry, sv);
+                if constexpr (kRecord)
+                    if ((__float_as_uint(sx) | __float_as_uint(su) | __float_as_uint(sy) | __float_as_uint(sv)) != 0u)
+                        loudParts |= kQuietAll | (lane == 1 ? kQuietBottom : 0u) | (lane == kStripRows ? kQuietTop : 0u) |
+                                     (((x - 1) & (kQuietCols - 1)) == 0 ? kQuietLeft : 0u) |
+                                     ((x & (kQuietCols - 1)) == 0 || x == nx ? kQuietRight : 0u);
+            }
+            carryH = ev.hR;
+            carryHu = ev.huR;
+            cur = nxt;
+            cq = nq;
+            // the end of a record tile: its parts' flags and its maximum.  A tile
+            // reports its right edge (x | x+1) and, first in a run, its left halo
+            // edge; the tile of column 1 always starts a run, so every x-edge is
+            // in some record, and each record's edges lie in its tile's footprint.
+            // A deferred edge at the boundary touches both tiles.
+            if (kRecord && ((x & (kQuietCols - 1)) == 0 || x == x1)) {  // uniform per wave
+                const float tileMax = wave_max(smaxTile);
+                smaxRun = max(smaxRun, __builtin_amdgcn_readfirstlane(__float_as_uint(tileMax)));
+                if (io.quiet) {
+                    unsigned quiet = 0u;
+    #pragma unroll
+                    for (unsigned part = 1u; part <= kQuietRight; part <<= 1)
+                        if (!__any((loudParts & part) != 0u || loud)) quiet |= part;
+                    if (lane == 0) {
+                        const int rec = slotNow + yt + nyt * ((x - 1) / kQuietCols);
+                        io.quiet[rec] = quiet;
+                        io.speed[rec] = tileMax;
+                    }
+                }
+                smaxTile = 0.f;
+                loud = loudEdge;
+                loudParts = 0u;
+            }
+        }
+
+        if (N && __any(outside)) return false;
+        if constexpr (!kRecord) smaxRun = __float_as_uint(wave_max(smaxTile));
+        if (lane == 0) atomicMax(&ctl->smax[slotOut], smaxRun);
+        return true;
+    };
+    run_tile<dev::SolverCtx<S, true>, V>(threadIdx.x & 63, tile);
 }
 
 }  // namespace swe

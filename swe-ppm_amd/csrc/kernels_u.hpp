@@ -29,6 +29,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cfloat>
+#include <type_traits>
 
 #include "mlp.hpp"
 #include "solvers_dev.hpp"
@@ -161,6 +162,32 @@ struct Slots {
 };
 
 __device__ __forceinline__ size_t idx(const StateView& v, int x, int y) { return (size_t)x * v.pitch + y; }
+
+// Access to a column that starts at the wave-uniform offset `col` of a field:
+// the column's address stays in scalar registers and the load or store adds
+// the lane's 32-bit byte offset (lane_bytes).  The empty asm statements keep
+// the compiler from forming field + row, or the offset's 64-bit form, once
+// per lane outside the column loop: that holds two vector registers for each
+// of a sweep's 8 to 15 arrays and costs a vector add per access.  Registers of
+// the fused sweeps with 64-bit indices and in this form: HLLE 77 -> 55, f-wave
+// 78 -> 56, Hybrid 71 -> 63, AugRie 86 -> 81.
+typedef __attribute__((address_space(1))) char GlobalByte;
+typedef __attribute__((address_space(1))) float GlobalFloat;
+// byte offset of element `row` (non-negative) of a column
+__device__ __forceinline__ unsigned lane_bytes(int row) {
+    unsigned o = (unsigned)row * 4u;
+    asm("" : "+v"(o));
+    return o;
+}
+__device__ __forceinline__ GlobalFloat* col_ptr(const float* f, size_t col, unsigned bytes) {
+    GlobalByte* p = (GlobalByte*)const_cast<float*>(f + col);
+    asm("" : "+s"(p));
+    return (GlobalFloat*)(p + bytes);
+}
+__device__ __forceinline__ float col_get(const float* f, size_t col, unsigned bytes) { return *col_ptr(f, col, bytes); }
+__device__ __forceinline__ void col_set(float* f, size_t col, unsigned bytes, float value) {
+    *col_ptr(f, col, bytes) = value;
+}
 
 // dt rule of flavour U (SWE_DimensionalSplittingMpi.cpp:448-456)
 __device__ __forceinline__ float timestep_from_max(float s, float dx, float dy) {
@@ -333,18 +360,48 @@ struct CellQ {
     }
 };
 
+template <class A = dev::Ieee>
 __device__ __forceinline__ CellQ cell_q(float h, float hu, float hv, float b) {
     CellQ q;
     q.h = h;
     q.hu = hu;
     q.hv = hv;
     q.b = b;
-    q.inv = 1.f / h;
+    q.inv = A::rcp(h);
     q.u = hu * q.inv;
     q.v = hv * q.inv;
-    q.sq = sqrtf(h);
+    q.sq = A::sqrt(h);
     q.c = kSqrtGravity * q.sq;
     return q;
+}
+
+// The two forms of a sweep's tile.  A wave first runs its tile with the short
+// divisions and roots of NormalRange and notes any loaded cell outside
+// dev::in_normal_range; if there was one, it runs the tile again with the
+// compiler's forms and overwrites what it wrote (a tile reads one set of
+// buffers and writes another, and reports its maximum only at the end).  The
+// general form is cold code after the loop, so it takes no registers from it;
+// a choice per column inside the loop spilled (17 registers for AugRie).
+// Measured with the short forms and the scalar column addresses (lane_bytes),
+// before and after, us per step: 2048^2 islands with every cell moving 163 ->
+// 142, 2048^2 islands 48.6 -> 46.0, Hybrid 1500 x 901 117 -> 97; f-wave and HLLE
+// are bound by memory and stay.
+// body(std::true_type / std::false_type, lane) runs the tile and returns true
+// if every cell was in the range.
+template <class Ctx, int V, class Body>
+__device__ __forceinline__ void run_tile(int lane, const Body& body) {
+    if constexpr (V == 0 && Ctx::kNormalForm) {
+        if (body(std::true_type(), lane)) return;
+        asm volatile("" : "+v"(lane));  // nothing of the general form is computed before
+    }
+    (void)body(std::false_type(), lane);
+}
+template <bool N>
+using CellMath = std::conditional_t<N, dev::NormalRange, dev::Ieee>;
+
+template <bool N>
+__device__ __forceinline__ bool outside_range(const CellQ& q) {
+    return N && !dev::in_normal_range(q.h, q.b, q.u, q.v);
 }
 
 // Strip sweep.  One wave per (y-tile, x-segment); 4 waves per workgroup.
@@ -358,8 +415,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MODE == MOD
                                                                      8))) void sweep_u_kernel(
     StateView v, SumsView sums, float* hn, float* hun, float* hvn, BoundaryInfo bi, DeviceCtl* ctl, Slots sl,
     float dtFixed, int fuseBc, float* dtLog, int logIdx) {
-    const int lane = threadIdx.x & 63;
-    const int wave = blockIdx.x * kWavesPerGroup + (threadIdx.x >> 6);
+    const int wave = __builtin_amdgcn_readfirstlane(blockIdx.x * kWavesPerGroup + (threadIdx.x >> 6));
     const int nyt = (v.ny + kStripRows - 1) / kStripRows;
     const int nxs = (v.nx + XS - 1) / XS;
     if (wave >= nyt * nxs) return;  // uniform per wave
@@ -367,12 +423,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MODE == MOD
     const dev::SolverCtx<S, true> solver(S == SOLVER_AUGRIE_MLP ? ctl->mlp : nullptr);
     const int yt = wave % nyt;
     const int xs = wave / nyt;
-    const int y = kStripRows * yt + lane;  // rows y0-1 .. y0+62 with y0 = 62*yt + 1
-    const bool rowValid = y <= v.ny + 1;
-    const int yc = rowValid ? y : v.ny + 1;
-    const bool owned = (lane >= 1) && (lane <= kStripRows) && (y <= v.ny);
-    const bool rowInterior = (y >= 1) && (y <= v.ny);
-    const bool hEdgeValid = (lane <= kStripRows) && (y <= v.ny);  // edge (y|y+1), y in [0, ny]
     const int x0 = 1 + xs * XS;
     const int x1 = min(x0 + XS - 1, v.nx);
 
@@ -383,125 +433,148 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MODE == MOD
         dtdy = dt / v.dy;
     }
 
-    const float* H = v.h;
-    const float* HU = v.hu;
-    const float* HV = v.hv;
-    const float* B = v.b;
-    size_t o = idx(v, x0 - 1, yc);
-    float ch = H[o], chu = HU[o], chv = HV[o], cb = B[o];
-    o += v.pitch;
-    float nh = H[o], nhu = HU[o], nhv = HV[o], nb = B[o];
-    // HLLE, f-wave and AugRie load column x+1 one column ahead (a software
-    // pipeline: the loads' latency overlaps column x's edges); past x1 + 1
-    // the loads stay on column nx + 1 and are not used.
-    constexpr bool kAhead = S == SOLVER_HLLE || S == SOLVER_FWAVE || S == SOLVER_AUGRIE;
-    float ah = 0.f, ahu = 0.f, ahv = 0.f, ab = 0.f;
-    if constexpr (kAhead) {
-        o += v.pitch;  // column x0 + 1 <= nx + 1
-        ah = H[o];
-        ahu = HU[o];
-        ahv = HV[o];
-        ab = B[o];
-    }
+    auto tile = [&](auto form, int lane) -> bool {
+        constexpr bool N = decltype(form)::value;
+        using A = CellMath<N>;
+        const int y = kStripRows * yt + lane;  // rows y0-1 .. y0+62 with y0 = 62*yt + 1
+        const bool rowValid = y <= v.ny + 1;
+        const int yc = rowValid ? y : v.ny + 1;
+        const bool owned = (lane >= 1) && (lane <= kStripRows) && (y <= v.ny);
+        const bool rowInterior = (y >= 1) && (y <= v.ny);
+        const bool hEdgeValid = (lane <= kStripRows) && (y <= v.ny);  // edge (y|y+1), y in [0, ny]
 
-    // In MODE_UPDATE the new buffer must end up a complete state: ghost cells
-    // not rewritten by the fused boundary conditions are carried over.  Each
-    // ghost row is carried by exactly one lane: row 0 by lane 0 of tile 0,
-    // row ny+1 by the tile where it is lane >= 1, other rows by their owner.
-    const bool carryRow = owned || (y == 0 && lane == 0) || (y == v.ny + 1 && lane >= 1);
-    if (MODE == MODE_UPDATE && x0 == 1 && carryRow && !(fuseBc && bc_handles(v, bi, 0, y))) {
-        const size_t g = idx(v, 0, y);
-        hn[g] = ch;
-        hun[g] = chu;
-        hvn[g] = chv;
-    }
-
-    // per-cell quantities (velocities, celerity, sqrt h) are computed once
-    // when a cell is loaded and reused by its four edges
-    CellQ cq = cell_q(ch, chu, chv, cb);
-    CellQ nq = cell_q(nh, nhu, nhv, nb);
-
-    // halo vertical edge (x0-1 | x0)
-    dev::EdgeOut e = solver.solve(cq.xside(), nq.xside());
-    float carryH = e.hR, carryHu = e.huR;
-    float smaxv = rowInterior ? e.speed : 0.f;
-
-    for (int x = x0; x <= x1; ++x) {
-        ch = nh;
-        chu = nhu;
-        chv = nhv;
-        cb = nb;
-        cq = nq;
+        const float* H = v.h;
+        const float* HU = v.hu;
+        const float* HV = v.hv;
+        const float* B = v.b;
+        size_t o = (size_t)(x0 - 1) * v.pitch;  // the column's offset, wave-uniform
+        unsigned ro = lane_bytes(yc);
+        float ch = col_get(H, o, ro), chu = col_get(HU, o, ro), chv = col_get(HV, o, ro), cb = col_get(B, o, ro);
+        o += v.pitch;
+        float nh = col_get(H, o, ro), nhu = col_get(HU, o, ro), nhv = col_get(HV, o, ro), nb = col_get(B, o, ro);
+        // HLLE, f-wave and AugRie load column x+1 one column ahead (a software
+        // pipeline: the loads' latency overlaps column x's edges); past x1 + 1
+        // the loads stay on column nx + 1 and are not used.
+        constexpr bool kAhead = S == SOLVER_HLLE || S == SOLVER_FWAVE || S == SOLVER_AUGRIE;
+        float ah = 0.f, ahu = 0.f, ahv = 0.f, ab = 0.f;
         if constexpr (kAhead) {
-            nh = ah;
-            nhu = ahu;
-            nhv = ahv;
-            nb = ab;
-            if (x + 2 <= v.nx + 1) o += v.pitch;  // column x+2, else stay on nx+1
-            ah = H[o];
-            ahu = HU[o];
-            ahv = HV[o];
-            ab = B[o];
-        } else {
-            o += v.pitch;  // column x+1 (<= nx+1)
-            nh = H[o];
-            nhu = HU[o];
-            nhv = HV[o];
-            nb = B[o];
+            o += v.pitch;  // column x0 + 1 <= nx + 1
+            ah = col_get(H, o, ro);
+            ahu = col_get(HU, o, ro);
+            ahv = col_get(HV, o, ro);
+            ab = col_get(B, o, ro);
         }
-        nq = cell_q(nh, nhu, nhv, nb);
 
-        // vertical edge (x | x+1)
-        const dev::EdgeOut ev = solver.solve(cq.xside(), nq.xside());
-        if (rowInterior) smaxv = dev::smax(smaxv, ev.speed);
-
-        // horizontal edge (y | y+1): upper cell from lane+1
-        const dev::EdgeOut eh = solver.solve(cq.yside(), cq.yside_from_lane_above());
-        if (hEdgeValid) smaxv = dev::smax(smaxv, eh.speed);
-        // up-going part of edge (y-1 | y) from lane-1
-        const float aH = __shfl_up(eh.hR, 1, 64);
-        const float aHv = __shfl_up(eh.huR, 1, 64);
-
-        const float sx = carryH + ev.hL;
-        const float su = carryHu + ev.huL;
-        const float sy = aH + eh.hL;
-        const float sv = aHv + eh.huL;
-        carryH = ev.hR;
-        carryHu = ev.huR;
-
-        if (MODE == MODE_STORE && owned) {
-            const size_t c = idx(v, x, y);
-            sums.sx[c] = sx;
-            sums.sy[c] = sy;
-            sums.su[c] = su;
-            sums.sv[c] = sv;
+        // In MODE_UPDATE the new buffer must end up a complete state: ghost cells
+        // not rewritten by the fused boundary conditions are carried over.  Each
+        // ghost row is carried by exactly one lane: row 0 by lane 0 of tile 0,
+        // row ny+1 by the tile where it is lane >= 1, other rows by their owner.
+        const bool carryRow = owned || (y == 0 && lane == 0) || (y == v.ny + 1 && lane >= 1);
+        if (MODE == MODE_UPDATE && x0 == 1 && carryRow && !(fuseBc && bc_handles(v, bi, 0, y))) {
+            const size_t g = idx(v, 0, y);
+            hn[g] = ch;
+            hun[g] = chu;
+            hvn[g] = chv;
         }
-        if (MODE == MODE_UPDATE) {
-            const size_t c = idx(v, x, y);
-            if (owned) {
-                const Cell nc = update_cell(ch, chu, chv, dtdx, dtdy, sx, sy, su, sv);
-                hn[c] = nc.h;
-                hun[c] = nc.hu;
-                hvn[c] = nc.hv;
-                if (fuseBc) write_boundary_ghosts(v, bi, x, y, nc.h, nc.hu, nc.hv, hn, hun, hvn);
-            } else if (carryRow && (y == 0 || y == v.ny + 1) && !(fuseBc && bc_handles(v, bi, x, y))) {
-                hn[c] = ch;  // carry ghost rows into the new buffer
-                hun[c] = chu;
-                hvn[c] = chv;
+
+        // per-cell quantities (velocities, celerity, sqrt h) are computed once
+        // when a cell is loaded and reused by its four edges
+        CellQ cq = cell_q<A>(ch, chu, chv, cb);
+        CellQ nq = cell_q<A>(nh, nhu, nhv, nb);
+
+        bool outside = outside_range<N>(cq) || outside_range<N>(nq);
+
+        // halo vertical edge (x0-1 | x0)
+        const dev::EdgeOut e = solver.template solve<A>(cq.xside(), nq.xside());
+        float carryH = e.hR, carryHu = e.huR;
+        float smaxv = rowInterior ? e.speed : 0.f;
+
+        for (int x = x0; x <= x1; ++x) {
+            ch = nh;
+            chu = nhu;
+            chv = nhv;
+            cb = nb;
+            cq = nq;
+            if constexpr (kAhead) {
+                nh = ah;
+                nhu = ahu;
+                nhv = ahv;
+                nb = ab;
+                if (x + 2 <= v.nx + 1) o += v.pitch;  // column x+2, else stay on nx+1
+                ro = lane_bytes(yc);
+                ah = col_get(H, o, ro);
+                ahu = col_get(HU, o, ro);
+                ahv = col_get(HV, o, ro);
+                ab = col_get(B, o, ro);
+            } else {
+                o += v.pitch;  // column x+1 (<= nx+1)
+                ro = lane_bytes(yc);
+                nh = col_get(H, o, ro);
+                nhu = col_get(HU, o, ro);
+                nhv = col_get(HV, o, ro);
+                nb = col_get(B, o, ro);
+            }
+            nq = cell_q<A>(nh, nhu, nhv, nb);
+            outside = outside || outside_range<N>(nq);
+
+            // vertical edge (x | x+1)
+            const dev::EdgeOut ev = solver.template solve<A>(cq.xside(), nq.xside());
+            if (rowInterior) smaxv = dev::smax(smaxv, ev.speed);
+
+            // horizontal edge (y | y+1): upper cell from lane+1
+            const dev::EdgeOut eh = solver.template solve<A>(cq.yside(), cq.yside_from_lane_above());
+            if (hEdgeValid) smaxv = dev::smax(smaxv, eh.speed);
+            // up-going part of edge (y-1 | y) from lane-1
+            const float aH = __shfl_up(eh.hR, 1, 64);
+            const float aHv = __shfl_up(eh.huR, 1, 64);
+
+            const float sx = carryH + ev.hL;
+            const float su = carryHu + ev.huL;
+            const float sy = aH + eh.hL;
+            const float sv = aHv + eh.huL;
+            carryH = ev.hR;
+            carryHu = ev.huR;
+
+            const size_t c = (size_t)x * v.pitch;
+            if (MODE == MODE_STORE && owned) {
+                const unsigned ry = lane_bytes(y);
+                col_set(sums.sx, c, ry, sx);
+                col_set(sums.sy, c, ry, sy);
+                col_set(sums.su, c, ry, su);
+                col_set(sums.sv, c, ry, sv);
+            }
+            if (MODE == MODE_UPDATE) {
+                const unsigned ry = lane_bytes(y);
+                if (owned) {
+                    const Cell nc = update_cell(ch, chu, chv, dtdx, dtdy, sx, sy, su, sv);
+                    col_set(hn, c, ry, nc.h);
+                    col_set(hun, c, ry, nc.hu);
+                    col_set(hvn, c, ry, nc.hv);
+                    if (fuseBc) write_boundary_ghosts(v, bi, x, y, nc.h, nc.hu, nc.hv, hn, hun, hvn);
+                } else if (carryRow && (y == 0 || y == v.ny + 1) && !(fuseBc && bc_handles(v, bi, x, y))) {
+                    col_set(hn, c, ry, ch);  // carry ghost rows into the new buffer
+                    col_set(hun, c, ry, chu);
+                    col_set(hvn, c, ry, chv);
+                }
             }
         }
-    }
-    if (MODE == MODE_UPDATE && x1 == v.nx && carryRow && !(fuseBc && bc_handles(v, bi, v.nx + 1, y))) {
-        const size_t g = idx(v, v.nx + 1, y);
-        hn[g] = nh;
-        hun[g] = nhu;
-        hvn[g] = nhv;
-    }
+        if (MODE == MODE_UPDATE && x1 == v.nx && carryRow && !(fuseBc && bc_handles(v, bi, v.nx + 1, y))) {
+            const size_t g = idx(v, v.nx + 1, y);
+            hn[g] = nh;
+            hun[g] = nhu;
+            hvn[g] = nhv;
+        }
 
-    if (MODE != MODE_UPDATE) {
-        smaxv = wave_max(smaxv);
-        if (lane == 0) atomicMax(&ctl->smax[sl.use], __float_as_uint(smaxv));
-    } else {
+        if (N && __any(outside)) return false;
+        if (MODE != MODE_UPDATE) {
+            smaxv = wave_max(smaxv);
+            if (lane == 0) atomicMax(&ctl->smax[sl.use], __float_as_uint(smaxv));
+        }
+        return true;
+    };
+    run_tile<dev::SolverCtx<S, true>, V>(threadIdx.x & 63, tile);
+
+    if (MODE == MODE_UPDATE) {
         if (blockIdx.x == 0 && threadIdx.x == 0) {
             ctl->smax[sl.clear] = 0u;  // a later step's maximum starts from zero
             if (dtFixed < 0.f) {

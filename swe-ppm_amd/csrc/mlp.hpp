@@ -315,6 +315,7 @@ __device__ __forceinline__ dev::Middle learned_middle(const unsigned* __restrict
 }
 
 struct LearnedMiddle {
+    using Math = dev::Ieee;
     static constexpr bool kDefers = false;
     const unsigned* F;
     __device__ __forceinline__ dev::Middle operator()(float hL, float hR, float uL, float uR, float cL, float cR,
@@ -331,6 +332,7 @@ struct LearnedMiddle {
 // Dry and two-rarefaction edges take the exact closed forms.  No network call
 // and no Newton loop for wet edges stay in the sweep.
 struct DeferredMiddle {
+    using Math = dev::Ieee;
     static constexpr bool kDefers = true;
     __device__ __forceinline__ dev::Middle operator()(float hL, float hR, float uL, float uR, float cL, float cR,
                                                       float invL, float invR, float bL, float bR) const {
@@ -351,7 +353,9 @@ struct DeferredMiddle {
 namespace dev {
 template <bool ReuseFirst>
 struct SolverCtx<SOLVER_AUGRIE_DEFER, ReuseFirst> {
+    static constexpr bool kNormalForm = false;
     __device__ __forceinline__ explicit SolverCtx(const unsigned*) {}
+    template <class = Ieee>
     __device__ __forceinline__ EdgeOut solve(const Side& L, const Side& R) const {
         return augrie_with(L, R, mlp::DeferredMiddle{});
     }
@@ -359,8 +363,10 @@ struct SolverCtx<SOLVER_AUGRIE_DEFER, ReuseFirst> {
 
 template <bool ReuseFirst>
 struct SolverCtx<SOLVER_AUGRIE_MLP, ReuseFirst> {
+    static constexpr bool kNormalForm = false;
     const unsigned* F;
     __device__ __forceinline__ explicit SolverCtx(const unsigned* frags) : F(frags) {}
+    template <class = Ieee>
     __device__ __forceinline__ EdgeOut solve(const Side& L, const Side& R) const {
         return augrie_with(L, R, mlp::LearnedMiddle{F});
     }

@@ -23,6 +23,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include "exact_math.hpp"
 #include "swe_common.h"
 
 namespace swe {
@@ -48,14 +49,15 @@ struct Side {
     float inv;  // 1 / h (the augmented solver's middle state divides by both depths)
 };
 
+template <class A = Ieee>
 __device__ __forceinline__ Side cell_side(float h, float hu, float b) {
     Side s;
     s.h = h;
     s.hu = hu;
     s.b = b;
-    s.inv = 1.f / h;
+    s.inv = A::rcp(h);
     s.u = hu * s.inv;
-    s.sq = sqrtf(h);
+    s.sq = A::sqrt(h);
     s.c = kSqrtGravity * s.sq;
     return s;
 }
@@ -108,13 +110,14 @@ __device__ __forceinline__ Mirrored mirror_dry(const Side& L, const Side& R) {
 // ---------------------------------------------------------------------------
 // f-wave
 // ---------------------------------------------------------------------------
+template <class A = Ieee>
 __device__ __forceinline__ EdgeOut fwave(const Side& Lin, const Side& Rin) {
     const Mirrored m = mirror_dry(Lin, Rin);
     const Side& L = m.L;
     const Side& R = m.R;
     const float hRoe = 0.5f * (L.h + R.h);
-    const float uRoe = (L.u * L.sq + R.u * R.sq) / (L.sq + R.sq);
-    const float cRoe = sqrtf(kGravity * hRoe);
+    const float uRoe = A::div(L.u * L.sq + R.u * R.sq, L.sq + R.sq);
+    const float cRoe = A::sqrt(kGravity * hRoe);
     const float s1 = smin(L.u - L.c, uRoe - cRoe);
     const float s2 = smax(R.u + R.c, uRoe + cRoe);
 
@@ -122,7 +125,7 @@ __device__ __forceinline__ EdgeOut fwave(const Side& Lin, const Side& Rin) {
     const float fR = R.hu * R.u + 0.5f * kGravity * R.h * R.h;
     const float fL = L.hu * L.u + 0.5f * kGravity * L.h * L.h;
     const float df2 = (fR - fL) + 0.5f * kGravity * (L.h + R.h) * (R.b - L.b);
-    const float invDs = 1.f / (s2 - s1);
+    const float invDs = A::rcp(s2 - s1);
     const float beta1 = (s2 * df1 - df2) * invDs;
     const float beta2 = (df2 - s1 * df1) * invDs;
 
@@ -156,16 +159,15 @@ __device__ __forceinline__ EdgeOut fwave(const Side& Lin, const Side& Rin) {
 // quantities); with ReuseFirst it takes them instead of recomputing them, so
 // it costs no division and one square root (two shocks) or two (shock and
 // rarefaction).  The values are the ones the loop computes, so both forms give
-// identical results.  The compiler peels the first iteration
-// for it, a second copy of the loop body; measured under the 72-register
-// budget of seven waves per SIMD, that pays (the single-block sweeps and the
-// batched kernels use it).
+// identical results (the single-block sweeps and the batched kernels use it).
+// The curves of the next iterate are evaluated at the end of the loop's body,
+// so that it exists once in the code.
 // ---------------------------------------------------------------------------
 struct Middle {
     float hm, s1m, s2m;
 };
 
-template <bool ReuseFirst = false>
+template <bool ReuseFirst = false, class A = Ieee>
 __device__ __forceinline__ Middle middle_state(float hL, float hR, float uL, float uR, float cL, float cR, float invL,
                                                float invR) {
     const float hMin = smin(hL, hR);
@@ -185,12 +187,12 @@ __device__ __forceinline__ Middle middle_state(float hL, float hR, float uL, flo
     const float halfG = 0.5f * kGravity;
     const float quarterG = 0.25f * kGravity;
     const float fMin = du + 2.f * (cMin - cMax);
-    const float gMaxMin = sqrtf(halfG * (invMax + invMin));
+    const float gMaxMin = A::sqrt(halfG * (invMax + invMin));
     const float fMax = du + (hMax - hMin) * gMaxMin;
     if (fMin > 0.f) {
         const float a = smax(0.f, -du + 2.f * (cL + cR));
-        m.hm = a * a / (16.f * kGravity);
-        const float cm = sqrtf(kGravity * m.hm);
+        m.hm = A::div(a * a, 16.f * kGravity);
+        const float cm = A::sqrt0(kGravity * m.hm);
         m.s1m = uL + 2.f * cL - 3.f * cm;
         m.s2m = uR - 2.f * cR + 3.f * cm;
         return m;
@@ -204,17 +206,19 @@ __device__ __forceinline__ Middle middle_state(float hL, float hR, float uL, flo
         // rarefaction root sqrt(g hMin) is taken as the loop takes it (the
         // cell's celerity cMin = sqrt(g) sqrt(hMin) can differ in the last bit)
         invH = shocks ? invMax : invMin;
-        const float r0 = sqrtf(halfG * (invH + invH));
+        const float r0 = A::sqrt(halfG * (invH + invH));
         gMin = shocks ? gMaxMin : r0;
-        s2 = shocks ? r0 : sqrtf(kGravity * hMin);
+        s2 = shocks ? r0 : A::sqrt(kGravity * hMin);
     }
-    for (int it = 0; it < kMaxNewton; ++it) {
-        if (!ReuseFirst || it > 0) {
-            invH = 1.f / h;
-            gMin = sqrtf(halfG * (invH + invMin));
-            // shocks: gMax(h); shock+rarefaction: sqrt(g h)
-            s2 = sqrtf(shocks ? halfG * (invH + invMax) : kGravity * h);
-        }
+    auto curves = [&] {
+        invH = A::rcp(h);
+        gMin = A::sqrt(halfG * (invH + invMin));
+        // shocks: gMax(h); shock+rarefaction: sqrt(g h)
+        s2 = A::sqrt(shocks ? halfG * (invH + invMax) : kGravity * h);
+    };
+    if constexpr (!ReuseFirst) curves();
+#pragma unroll 1
+    for (int it = 1;; ++it) {
         const float t2 = shocks ? (h - hMax) * s2 : 2.f * (s2 - cMax);
         const float phi = (du + (h - hMin) * gMin) + t2;
         const float q = shocks ? s2 : 1.f;
@@ -223,12 +227,13 @@ __device__ __forceinline__ Middle middle_state(float hL, float hR, float uL, flo
         const float first = gMin + (shocks ? s2 : s2 * invH);
         // phi / (first - quarterG invH^2 num / den) with both terms scaled by
         // den: one division instead of two
-        const float step = (phi * den) / (first * den - quarterG * invH * invH * num);
+        const float step = A::div(phi * den, first * den - quarterG * invH * invH * num);
         h = h - step;
-        if (fabsf(step) <= kNewtonTol * h) break;
+        if (fabsf(step) <= kNewtonTol * h || it == kMaxNewton) break;
+        curves();
     }
     m.hm = h;
-    const float cm = sqrtf(kGravity * h);
+    const float cm = A::sqrt(kGravity * h);
     if (shocks) {
         const bool leftIsMin = !(hR < hL);
         const float gL = leftIsMin ? gMin : s2;
@@ -252,12 +257,13 @@ __device__ __forceinline__ Middle middle_state(float hL, float hR, float uL, flo
 // Riemann problem of a wet-wet or inundation edge; the exact Newton
 // middle_state is the default, the learned surrogate plugs in here.
 // ---------------------------------------------------------------------------
-template <bool ReuseFirst>
+template <bool ReuseFirst, class A = Ieee>
 struct ExactMiddle {
+    using Math = A;
     static constexpr bool kDefers = false;
     __device__ __forceinline__ Middle operator()(float hL, float hR, float uL, float uR, float cL, float cR,
                                                  float invL, float invR, float, float) const {
-        return middle_state<ReuseFirst>(hL, hR, uL, uR, cL, cR, invL, invR);
+        return middle_state<ReuseFirst, A>(hL, hR, uL, uR, cL, cR, invL, invR);
     }
 };
 
@@ -270,6 +276,7 @@ struct AugPrep {
     bool wallL, wallR, dryBoth;
 };
 
+template <class A = Ieee>
 __device__ __forceinline__ AugPrep augrie_prepare(const Side& Lin, const Side& Rin) {
     const bool dryLin = Lin.h < kDryTol;
     const bool dryRin = Rin.h < kDryTol;
@@ -291,7 +298,7 @@ __device__ __forceinline__ AugPrep augrie_prepare(const Side& Lin, const Side& R
     p.wallR = false;
     if ((dryLin || dryRin) && !p.dryBoth) {
         if (dryRin) {
-            const Middle t = middle_state(p.hL, p.hL, p.uL, -p.uL, p.cL, p.cL, p.invL, p.invL);
+            const Middle t = middle_state<false, A>(p.hL, p.hL, p.uL, -p.uL, p.cL, p.cL, p.invL, p.invL);
             const float hTest = smax(p.hL, t.hm);
             if (hTest + p.bL < p.bR) {
                 p.wallR = true;
@@ -305,7 +312,7 @@ __device__ __forceinline__ AugPrep augrie_prepare(const Side& Lin, const Side& R
                 p.bR = p.hL + p.bL;
             }
         } else {
-            const Middle t = middle_state(p.hR, p.hR, -p.uR, p.uR, p.cR, p.cR, p.invR, p.invR);
+            const Middle t = middle_state<false, A>(p.hR, p.hR, -p.uR, p.uR, p.cR, p.cR, p.invR, p.invR);
             const float hTest = smax(p.hR, t.hm);
             if (hTest + p.bR < p.bL) {
                 p.wallL = true;
@@ -341,8 +348,9 @@ __device__ __forceinline__ bool still_edge(const Side& L, const Side& R) {
            L.h <= kStillRatio * R.h && R.h <= kStillRatio * L.h;
 }
 
+template <class A = Ieee>
 __device__ __forceinline__ float still_speed(const Side& L, const Side& R) {
-    const float cHat = sqrtf(kGravity * 0.5f * (R.h + L.h));
+    const float cHat = A::sqrt(kGravity * 0.5f * (R.h + L.h));
     const float sE1 = smin(-L.c, -cHat);
     const float sE2 = smax(R.c, cHat);
     return smax(fabsf(sE1), fabsf(sE2));
@@ -350,16 +358,17 @@ __device__ __forceinline__ float still_speed(const Side& L, const Side& R) {
 
 template <typename MiddleFn>
 __device__ __forceinline__ EdgeOut augrie_with(const Side& Lin, const Side& Rin, const MiddleFn& middle) {
+    using A = typename MiddleFn::Math;
     const bool still = still_edge(Lin, Rin);
-    if (__all(still)) return EdgeOut{0.f, 0.f, 0.f, 0.f, still_speed(Lin, Rin)};
-    const AugPrep p = augrie_prepare(Lin, Rin);
+    if (__all(still)) return EdgeOut{0.f, 0.f, 0.f, 0.f, still_speed<A>(Lin, Rin)};
+    const AugPrep p = augrie_prepare<A>(Lin, Rin);
     const bool dryBoth = p.dryBoth;
     const bool wallL = p.wallL, wallR = p.wallR;
     const float hL = p.hL, huL = p.huL, uL = p.uL, cL = p.cL, bL = p.bL;
     const float hR = p.hR, huR = p.huR, uR = p.uR, cR = p.cR, bR = p.bR;
 
-    const float uHat = (cL * uL + cR * uR) / (cL + cR);
-    const float cHat = sqrtf(kGravity * 0.5f * (hR + hL));
+    const float uHat = A::div(cL * uL + cR * uR, cL + cR);
+    const float cHat = A::sqrt(kGravity * 0.5f * (hR + hL));
     const float sE1 = smin(uL - cL, uHat - cHat);
     const float sE2 = smax(uR + cR, uHat + cHat);
 
@@ -369,7 +378,7 @@ __device__ __forceinline__ EdgeOut augrie_with(const Side& Lin, const Side& Rin,
     const float l3 = smax(sE2, mid.s1m);
     const float l2 = 0.5f * (l1 + l3);
     const float dl = l3 - l1;
-    const float invDl = 1.f / dl;
+    const float invDl = A::rcp(dl);
     const float hStarHLL = smax((huL - huR + l3 * hR - l1 * hL) * invDl, 0.f);
 
     const float dh = hR - hL;
@@ -390,14 +399,14 @@ __device__ __forceinline__ EdgeOut augrie_with(const Side& Lin, const Side& Rin,
                        ((l3 > 0.f) && (mid.s2m < 0.f)) || ((uL + cL) * (uR + cR) < 0.f) ||
                        ((uL - cL) * (uR - cR) < 0.f);
 
-    const float invBar = 1.f / s1s2bar;
+    const float invBar = A::rcp(s1s2bar);
     float ddh = sonic ? -db : db * kGravity * hBar * invBar;
     const bool caseA = (l1 < -ct) && (l3 > ct);
     const bool caseB = !caseA && (l1 >= ct);
     const bool caseC = !caseA && !caseB && (l3 <= -ct);
     if (caseA || caseB || caseC) {
         const float hsd = hStarHLL * dl;
-        const float inv13 = 1.f / (l1 * l3);
+        const float inv13 = A::rcp(l1 * l3);
         const float dA = hsd * l1 * inv13;  // hStarHLL dl / l3
         const float dB = hsd * l3 * inv13;  // hStarHLL dl / l1
         const float hiBound = caseA ? dA : (caseB ? dB : hR);
@@ -444,24 +453,25 @@ __device__ __forceinline__ EdgeOut augrie_with(const Side& Lin, const Side& Rin,
     // edge is marked by a negative speed and solved again elsewhere
     if constexpr (MiddleFn::kDefers)
         if (mid.hm < 0.f) o.speed = -1.f;
-    if (still) o = EdgeOut{0.f, 0.f, 0.f, 0.f, still_speed(Lin, Rin)};
+    if (still) o = EdgeOut{0.f, 0.f, 0.f, 0.f, still_speed<A>(Lin, Rin)};
     return o;
 }
 
-template <bool ReuseFirst = false>
+template <bool ReuseFirst = false, class A = Ieee>
 __device__ __forceinline__ EdgeOut augrie(const Side& L, const Side& R) {
-    return augrie_with(L, R, ExactMiddle<ReuseFirst>());
+    return augrie_with(L, R, ExactMiddle<ReuseFirst, A>());
 }
 
 // ---------------------------------------------------------------------------
 // HLLE in fluctuation form, surface-gradient diffusion (well-balanced)
 // ---------------------------------------------------------------------------
+template <class A = Ieee>
 __device__ __forceinline__ EdgeOut hlle(const Side& Lin, const Side& Rin) {
     const Mirrored m = mirror_dry(Lin, Rin);
     const Side& L = m.L;
     const Side& R = m.R;
-    const float uRoe = (L.u * L.sq + R.u * R.sq) / (L.sq + R.sq);
-    const float cRoe = sqrtf(kGravity * 0.5f * (L.h + R.h));
+    const float uRoe = A::div(L.u * L.sq + R.u * R.sq, L.sq + R.sq);
+    const float cRoe = A::sqrt(kGravity * 0.5f * (L.h + R.h));
     const float sL = smin(smin(L.u - L.c, uRoe - cRoe), 0.f);
     const float sR = smax(smax(R.u + R.c, uRoe + cRoe), 0.f);
     const float df1 = R.hu - L.hu;
@@ -470,7 +480,7 @@ __device__ __forceinline__ EdgeOut hlle(const Side& Lin, const Side& Rin) {
     const float df2 = (fR - fL) + 0.5f * kGravity * (L.h + R.h) * (R.b - L.b);
     const float dq1 = (R.h + R.b) - (L.h + L.b);  // surface-gradient form: lake at rest stays at rest
     const float dq2 = R.hu - L.hu;
-    const float invDs = 1.f / (sR - sL);
+    const float invDs = A::rcp(sR - sL);
     const float q1 = (sR * dq1 - df1) * invDs;
     const float q2 = (sR * dq2 - df2) * invDs;
     EdgeOut o;
@@ -487,56 +497,56 @@ __device__ __forceinline__ EdgeOut hlle(const Side& Lin, const Side& Rin) {
     return o;
 }
 
-template <int S>
-struct EdgeSolver;
-
-// ReuseFirst selects the form of the Newton loop (middle_state); the results
-// are the same.
-template <>
-struct EdgeSolver<SOLVER_FWAVE> {
-    template <bool ReuseFirst = false>
-    __device__ __forceinline__ static EdgeOut solve(const Side& L, const Side& R) {
-        return fwave(L, R);
-    }
-};
-template <>
-struct EdgeSolver<SOLVER_AUGRIE> {
-    template <bool ReuseFirst = false>
-    __device__ __forceinline__ static EdgeOut solve(const Side& L, const Side& R) {
-        return augrie<ReuseFirst>(L, R);
-    }
-};
-template <>
-struct EdgeSolver<SOLVER_HLLE> {
-    template <bool ReuseFirst = false>
-    __device__ __forceinline__ static EdgeOut solve(const Side& L, const Side& R) {
-        return hlle(L, R);
-    }
-};
-template <>
-struct EdgeSolver<SOLVER_HYBRID> {
-    template <bool ReuseFirst = false>
-    __device__ __forceinline__ static EdgeOut solve(const Side& L, const Side& R) {
-        if (L.h >= kHybridTol && R.h >= kHybridTol) return fwave(L, R);
-        return augrie<ReuseFirst>(L, R);
-    }
-};
+// One edge with solver S.  ReuseFirst selects the form of the Newton loop
+// (middle_state), A that of divisions and square roots; the results are the
+// same.
+template <int S, bool ReuseFirst = false, class A = Ieee>
+__device__ __forceinline__ EdgeOut solve_edge(const Side& L, const Side& R) {
+    if constexpr (S == SOLVER_FWAVE) return fwave<A>(L, R);
+    if constexpr (S == SOLVER_HLLE) return hlle<A>(L, R);
+    if constexpr (S == SOLVER_HYBRID)
+        if (L.h >= kHybridTol && R.h >= kHybridTol) return fwave<A>(L, R);
+    if constexpr (S == SOLVER_AUGRIE || S == SOLVER_HYBRID) return augrie<ReuseFirst, A>(L, R);
+}
 
 // Solver with per-kernel state, built once at kernel start from an optional
 // parameter block (the learned middle state keeps its network weights in
-// registers; the exact solvers have no state).
+// registers; the exact solvers have no state).  kNormalForm: the sweeps solve
+// the edges of ordinary cells with NormalRange (column_edges in kernels_u.hpp).
 template <int S, bool ReuseFirst = false>
 struct SolverCtx {
+    static constexpr bool kNormalForm = true;
     __device__ __forceinline__ explicit SolverCtx(const unsigned*) {}
+    template <class A = Ieee>
     __device__ __forceinline__ EdgeOut solve(const Side& L, const Side& R) const {
-        return EdgeSolver<S>::template solve<ReuseFirst>(L, R);
+        return solve_edge<S, ReuseFirst, A>(L, R);
     }
 };
 
+// Cells whose edges may be solved with NormalRange: depth and bed below 2^40 and,
+// on a wet cell, velocities below 2^20 in sum.  A dry cell's momentum, velocity,
+// celerity and 1/h reach no result (the augmented solver sets them to zero, the
+// others mirror the wet side, and an edge between two dry cells returns zeros),
+// so every operand of a wet edge is normal:
+//   * h >= 0.01, so celerities lie in [0.3, 2^22] and every sum of two, every
+//     depth sum and its root is bounded away from zero;
+//   * speeds are below 2^23, and the fastest two of an edge differ by at least
+//     2 cHat less their rounding, > 0.3: the divisions by l3 - l1 and s2 - s1;
+//   * 1 / (l1 l3) and 1 / s1s2bar are used only where the operands exceed 1e-12;
+//   * Newton's depths stay between hMin and about 2^60, its two curve roots
+//     above 2^-30, so its denominator lies above 2^-90;
+//   * 2 (cL + cR) - du is zero or at least 2^-24, and its square a normal number.
+// Numerators below 2^-102 occur in two places, the Roe velocity and the Newton
+// step; the first is added to a celerity above 0.2, the second to a depth above
+// 0.01, and neither changes the sum in any rounding.  A NaN fails the test.
+__device__ __forceinline__ bool in_normal_range(float h, float b, float u, float v) {
+    return (fabsf(h) + fabsf(b) <= 0x1p40f) && (h < kDryTol || fabsf(u) + fabsf(v) <= 0x1p20f);
+}
+
 // Convenience for raw edge states (one-off evaluations).
-template <int S>
+template <int S, bool ReuseFirst = false, class A = Ieee>
 __device__ __forceinline__ EdgeOut solve_raw(float hL, float hR, float huL, float huR, float bL, float bR) {
-    return EdgeSolver<S>::solve(cell_side(hL, huL, bL), cell_side(hR, huR, bR));
+    return solve_edge<S, ReuseFirst, A>(cell_side<A>(hL, huL, bL), cell_side<A>(hR, huR, bR));
 }
 
 }  // namespace dev

@@ -21,19 +21,14 @@ constexpr int SOLVER_AUGRIE_DEFER = 5;
 // Waves per SIMD the flavour-U sweeps of each solver are compiled for
 // (its amdgpu_waves_per_eu floor; the build fails where the compiler cannot
 // meet it).  A SIMD lane has 512 registers: 7 waves need at most 72 per lane,
-// 6 at most 80.  Hybrid and the deferring learned sweep fit 7 (71-72
-// registers, no spills).  AugRie's fused kernel keeps a quiet-tile record
-// and loads each column one column ahead (8 registers): 86 registers at 5
-// waves.  Measured on the 2048^2 islands against 6 waves without the early
-// loads (79 registers; the loads spill at 6): 2.5% faster with quiet tiles
-// skipped, 12% faster with every tile computed, 2.6% slower on the disturbed
-// islands, where every edge runs the full solver.  HLLE (77) and f-wave (78)
-// keep 6 with the early loads; the in-sweep network call holds 136 vector
+// 6 at most 80.  Every exact solver loads each column one column ahead (8
+// registers).  AugRie's fused kernel also keeps a quiet-tile record: 75
+// registers, 6 waves; Hybrid (70) and the deferring learned sweep fit 7; HLLE
+// and f-wave (57) exceed their 6.  The in-sweep network call holds 136 vector
 // and 32 accumulation registers (3 waves).
 constexpr int fused_waves_per_simd(int solver) {
     return (solver == SOLVER_HYBRID || solver == SOLVER_AUGRIE_DEFER) ? 7
            : solver == SOLVER_AUGRIE_MLP                             ? 3
-           : solver == SOLVER_AUGRIE                                 ? 5
                                                                      : 6;
 }
 
