@@ -27,7 +27,7 @@
 // Zero: a zero numerator gives +0 (an IEEE division keeps the sign); sqrt0 also
 // takes x = 0.  A numerator below 2^-102 may be rounded wrongly, by less than
 // 2^-100 of 1 / b; the callers add such quotients to numbers far larger
-// (solvers_dev.hpp, in_normal_range).
+// (in_normal_range).
 #pragma once
 
 #include <hip/hip_runtime.h>

@@ -306,11 +306,8 @@ __device__ __forceinline__ int next_items(int* head, int* sBase) {
     return base;
 }
 
-// The batched kernels take the Newton loop's first iteration from the bracket
-// (middle_state<true>), as the fused single-block kernel does: measured faster
-// under their 72-register budget, same results.
 template <int S>
-using BatchSolver = dev::SolverCtx<S, true>;
+using BatchSolver = dev::SolverCtx<S>;
 
 // ---- tiles of a block (strip_tiling / tile_lanes) ---------------------------
 __device__ __forceinline__ TileLanes tile_lanes(const BatchBlockDesc& d, int tile, int lane) {

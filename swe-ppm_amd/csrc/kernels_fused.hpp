@@ -182,9 +182,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(fused_waves
     const int yt = item % nyt;
     const int xs = item / nyt;
     const int slotNow = (io.step & 1) * nyt * ((nx + kQuietCols - 1) / kQuietCols);
-    // the Newton loop's first iteration from the bracket (middle_state<true>):
-    // measured 3% faster at seven waves per SIMD, same results
-    const dev::SolverCtx<S, true> solver(S == SOLVER_AUGRIE_MLP ? ctl->mlp : nullptr);
+    const dev::SolverCtx<S> solver(S == SOLVER_AUGRIE_MLP ? ctl->mlp : nullptr);
 
     const float dtdx = dt / v.dx;
     const float dtdy = dt / v.dy;
@@ -373,7 +371,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(fused_waves
         if (lane == 0) atomicMax(&ctl->smax[slotOut], smaxRun);
         return true;
     };
-    run_tile<dev::SolverCtx<S, true>, V>(threadIdx.x & 63, tile);
+    run_tile<dev::SolverCtx<S>, V>(threadIdx.x & 63, tile);
 }
 
 }  // namespace swe

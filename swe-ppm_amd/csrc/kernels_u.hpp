@@ -32,7 +32,7 @@
 #include <type_traits>
 
 #include "mlp.hpp"
-#include "solvers_dev.hpp"
+#include "edge_solver.hpp"
 #include "swe_common.h"
 
 namespace swe {
@@ -419,8 +419,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MODE == MOD
     const int nyt = (v.ny + kStripRows - 1) / kStripRows;
     const int nxs = (v.nx + XS - 1) / XS;
     if (wave >= nyt * nxs) return;  // uniform per wave
-    // the Newton loop's first iteration from the bracket, as in the fused kernel
-    const dev::SolverCtx<S, true> solver(S == SOLVER_AUGRIE_MLP ? ctl->mlp : nullptr);
+    const dev::SolverCtx<S> solver(S == SOLVER_AUGRIE_MLP ? ctl->mlp : nullptr);
     const int yt = wave % nyt;
     const int xs = wave / nyt;
     const int x0 = 1 + xs * XS;
@@ -572,7 +571,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MODE == MOD
         }
         return true;
     };
-    run_tile<dev::SolverCtx<S, true>, V>(threadIdx.x & 63, tile);
+    run_tile<dev::SolverCtx<S>, V>(threadIdx.x & 63, tile);
 
     if (MODE == MODE_UPDATE) {
         if (blockIdx.x == 0 && threadIdx.x == 0) {

@@ -27,7 +27,7 @@
 
 #include <hip/hip_runtime.h>
 
-#include "solvers_dev.hpp"
+#include "edge_solver.hpp"
 
 namespace swe {
 namespace mlp {
@@ -315,7 +315,6 @@ __device__ __forceinline__ dev::Middle learned_middle(const unsigned* __restrict
 }
 
 struct LearnedMiddle {
-    using Math = dev::Ieee;
     static constexpr bool kDefers = false;
     const unsigned* F;
     __device__ __forceinline__ dev::Middle operator()(float hL, float hR, float uL, float uR, float cL, float cR,
@@ -332,7 +331,6 @@ struct LearnedMiddle {
 // Dry and two-rarefaction edges take the exact closed forms.  No network call
 // and no Newton loop for wet edges stay in the sweep.
 struct DeferredMiddle {
-    using Math = dev::Ieee;
     static constexpr bool kDefers = true;
     __device__ __forceinline__ dev::Middle operator()(float hL, float hR, float uL, float uR, float cL, float cR,
                                                       float invL, float invR, float bL, float bR) const {
@@ -351,8 +349,8 @@ struct DeferredMiddle {
 }  // namespace mlp
 
 namespace dev {
-template <bool ReuseFirst>
-struct SolverCtx<SOLVER_AUGRIE_DEFER, ReuseFirst> {
+template <>
+struct SolverCtx<SOLVER_AUGRIE_DEFER> {
     static constexpr bool kNormalForm = false;
     __device__ __forceinline__ explicit SolverCtx(const unsigned*) {}
     template <class = Ieee>
@@ -361,8 +359,8 @@ struct SolverCtx<SOLVER_AUGRIE_DEFER, ReuseFirst> {
     }
 };
 
-template <bool ReuseFirst>
-struct SolverCtx<SOLVER_AUGRIE_MLP, ReuseFirst> {
+template <>
+struct SolverCtx<SOLVER_AUGRIE_MLP> {
     static constexpr bool kNormalForm = false;
     const unsigned* F;
     __device__ __forceinline__ explicit SolverCtx(const unsigned* frags) : F(frags) {}

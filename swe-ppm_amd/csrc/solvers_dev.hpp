@@ -13,7 +13,9 @@
 //   HLLE     -- Einfeldt 1988 in fluctuation form;
 //   Hybrid   -- f-wave when both depths >= kHybridTol, AugRie otherwise.
 //
-// Written for wave64 execution: the wet/dry and wave-direction decisions are
+// This is the general form, for every operand; the sweeps solve the edges of
+// ordinary cells with augrie_normal.hpp and the short divisions of
+// exact_math.hpp, to the same bits.  Written for wave64 execution: the wet/dry and wave-direction decisions are
 // predicates folded into selects; only the expensive, spatially clustered
 // paths (wet/dry wall test, Newton loops) are real branches, which stay
 // uniform inside most waves.  Every floating-point expression keeps one fixed
@@ -154,20 +156,11 @@ __device__ __forceinline__ EdgeOut fwave(const Side& Lin, const Side& Rin) {
 // concave on the search interval, so the iterates increase monotonically.
 // cL, cR are the cells' celerities sqrt(g) sqrt(h); invL, invR are 1 / hL,
 // 1 / hR, computed once per cell.
-// ReuseFirst: the first iteration starts at hMax or hMin, where 1/h is known
-// and, for two shocks, one of the two curve square roots (the bracket's own
-// quantities); with ReuseFirst it takes them instead of recomputing them, so
-// it costs no division and one square root (two shocks) or two (shock and
-// rarefaction).  The values are the ones the loop computes, so both forms give
-// identical results (the single-block sweeps and the batched kernels use it).
-// The curves of the next iterate are evaluated at the end of the loop's body,
-// so that it exists once in the code.
 // ---------------------------------------------------------------------------
 struct Middle {
     float hm, s1m, s2m;
 };
 
-template <bool ReuseFirst = false, class A = Ieee>
 __device__ __forceinline__ Middle middle_state(float hL, float hR, float uL, float uR, float cL, float cR, float invL,
                                                float invR) {
     const float hMin = smin(hL, hR);
@@ -187,38 +180,24 @@ __device__ __forceinline__ Middle middle_state(float hL, float hR, float uL, flo
     const float halfG = 0.5f * kGravity;
     const float quarterG = 0.25f * kGravity;
     const float fMin = du + 2.f * (cMin - cMax);
-    const float gMaxMin = A::sqrt(halfG * (invMax + invMin));
+    const float gMaxMin = sqrtf(halfG * (invMax + invMin));
     const float fMax = du + (hMax - hMin) * gMaxMin;
     if (fMin > 0.f) {
         const float a = smax(0.f, -du + 2.f * (cL + cR));
-        m.hm = A::div(a * a, 16.f * kGravity);
-        const float cm = A::sqrt0(kGravity * m.hm);
+        m.hm = a * a / (16.f * kGravity);
+        const float cm = sqrtf(kGravity * m.hm);
         m.s1m = uL + 2.f * cL - 3.f * cm;
         m.s2m = uR - 2.f * cR + 3.f * cm;
         return m;
     }
     const bool shocks = fMax <= 0.f;
     float h = shocks ? hMax : hMin;
-    float invH = 0.f, gMin = 0.f, s2 = 0.f;
-    if constexpr (ReuseFirst) {
-        // at h = hMax the shock curve of hMin is gMaxMin and the new root is
-        // gMax(hMax); at h = hMin the new root is gMin(hMin) and the
-        // rarefaction root sqrt(g hMin) is taken as the loop takes it (the
-        // cell's celerity cMin = sqrt(g) sqrt(hMin) can differ in the last bit)
-        invH = shocks ? invMax : invMin;
-        const float r0 = A::sqrt(halfG * (invH + invH));
-        gMin = shocks ? gMaxMin : r0;
-        s2 = shocks ? r0 : A::sqrt(kGravity * hMin);
-    }
-    auto curves = [&] {
-        invH = A::rcp(h);
-        gMin = A::sqrt(halfG * (invH + invMin));
+    float gMin = 0.f, s2 = 0.f;
+    for (int it = 0; it < kMaxNewton; ++it) {
+        const float invH = 1.f / h;
+        gMin = sqrtf(halfG * (invH + invMin));
         // shocks: gMax(h); shock+rarefaction: sqrt(g h)
-        s2 = A::sqrt(shocks ? halfG * (invH + invMax) : kGravity * h);
-    };
-    if constexpr (!ReuseFirst) curves();
-#pragma unroll 1
-    for (int it = 1;; ++it) {
+        s2 = sqrtf(shocks ? halfG * (invH + invMax) : kGravity * h);
         const float t2 = shocks ? (h - hMax) * s2 : 2.f * (s2 - cMax);
         const float phi = (du + (h - hMin) * gMin) + t2;
         const float q = shocks ? s2 : 1.f;
@@ -227,13 +206,12 @@ __device__ __forceinline__ Middle middle_state(float hL, float hR, float uL, flo
         const float first = gMin + (shocks ? s2 : s2 * invH);
         // phi / (first - quarterG invH^2 num / den) with both terms scaled by
         // den: one division instead of two
-        const float step = A::div(phi * den, first * den - quarterG * invH * invH * num);
+        const float step = (phi * den) / (first * den - quarterG * invH * invH * num);
         h = h - step;
-        if (fabsf(step) <= kNewtonTol * h || it == kMaxNewton) break;
-        curves();
+        if (fabsf(step) <= kNewtonTol * h) break;
     }
     m.hm = h;
-    const float cm = A::sqrt(kGravity * h);
+    const float cm = sqrtf(kGravity * h);
     if (shocks) {
         const bool leftIsMin = !(hR < hL);
         const float gL = leftIsMin ? gMin : s2;
@@ -257,13 +235,11 @@ __device__ __forceinline__ Middle middle_state(float hL, float hR, float uL, flo
 // Riemann problem of a wet-wet or inundation edge; the exact Newton
 // middle_state is the default, the learned surrogate plugs in here.
 // ---------------------------------------------------------------------------
-template <bool ReuseFirst, class A = Ieee>
 struct ExactMiddle {
-    using Math = A;
     static constexpr bool kDefers = false;
     __device__ __forceinline__ Middle operator()(float hL, float hR, float uL, float uR, float cL, float cR,
                                                  float invL, float invR, float, float) const {
-        return middle_state<ReuseFirst, A>(hL, hR, uL, uR, cL, cR, invL, invR);
+        return middle_state(hL, hR, uL, uR, cL, cR, invL, invR);
     }
 };
 
@@ -276,7 +252,6 @@ struct AugPrep {
     bool wallL, wallR, dryBoth;
 };
 
-template <class A = Ieee>
 __device__ __forceinline__ AugPrep augrie_prepare(const Side& Lin, const Side& Rin) {
     const bool dryLin = Lin.h < kDryTol;
     const bool dryRin = Rin.h < kDryTol;
@@ -298,7 +273,7 @@ __device__ __forceinline__ AugPrep augrie_prepare(const Side& Lin, const Side& R
     p.wallR = false;
     if ((dryLin || dryRin) && !p.dryBoth) {
         if (dryRin) {
-            const Middle t = middle_state<false, A>(p.hL, p.hL, p.uL, -p.uL, p.cL, p.cL, p.invL, p.invL);
+            const Middle t = middle_state(p.hL, p.hL, p.uL, -p.uL, p.cL, p.cL, p.invL, p.invL);
             const float hTest = smax(p.hL, t.hm);
             if (hTest + p.bL < p.bR) {
                 p.wallR = true;
@@ -312,7 +287,7 @@ __device__ __forceinline__ AugPrep augrie_prepare(const Side& Lin, const Side& R
                 p.bR = p.hL + p.bL;
             }
         } else {
-            const Middle t = middle_state<false, A>(p.hR, p.hR, -p.uR, p.uR, p.cR, p.cR, p.invR, p.invR);
+            const Middle t = middle_state(p.hR, p.hR, -p.uR, p.uR, p.cR, p.cR, p.invR, p.invR);
             const float hTest = smax(p.hR, t.hm);
             if (hTest + p.bR < p.bL) {
                 p.wallL = true;
@@ -348,9 +323,8 @@ __device__ __forceinline__ bool still_edge(const Side& L, const Side& R) {
            L.h <= kStillRatio * R.h && R.h <= kStillRatio * L.h;
 }
 
-template <class A = Ieee>
 __device__ __forceinline__ float still_speed(const Side& L, const Side& R) {
-    const float cHat = A::sqrt(kGravity * 0.5f * (R.h + L.h));
+    const float cHat = sqrtf(kGravity * 0.5f * (R.h + L.h));
     const float sE1 = smin(-L.c, -cHat);
     const float sE2 = smax(R.c, cHat);
     return smax(fabsf(sE1), fabsf(sE2));
@@ -358,17 +332,16 @@ __device__ __forceinline__ float still_speed(const Side& L, const Side& R) {
 
 template <typename MiddleFn>
 __device__ __forceinline__ EdgeOut augrie_with(const Side& Lin, const Side& Rin, const MiddleFn& middle) {
-    using A = typename MiddleFn::Math;
     const bool still = still_edge(Lin, Rin);
-    if (__all(still)) return EdgeOut{0.f, 0.f, 0.f, 0.f, still_speed<A>(Lin, Rin)};
-    const AugPrep p = augrie_prepare<A>(Lin, Rin);
+    if (__all(still)) return EdgeOut{0.f, 0.f, 0.f, 0.f, still_speed(Lin, Rin)};
+    const AugPrep p = augrie_prepare(Lin, Rin);
     const bool dryBoth = p.dryBoth;
     const bool wallL = p.wallL, wallR = p.wallR;
     const float hL = p.hL, huL = p.huL, uL = p.uL, cL = p.cL, bL = p.bL;
     const float hR = p.hR, huR = p.huR, uR = p.uR, cR = p.cR, bR = p.bR;
 
-    const float uHat = A::div(cL * uL + cR * uR, cL + cR);
-    const float cHat = A::sqrt(kGravity * 0.5f * (hR + hL));
+    const float uHat = (cL * uL + cR * uR) / (cL + cR);
+    const float cHat = sqrtf(kGravity * 0.5f * (hR + hL));
     const float sE1 = smin(uL - cL, uHat - cHat);
     const float sE2 = smax(uR + cR, uHat + cHat);
 
@@ -378,7 +351,7 @@ __device__ __forceinline__ EdgeOut augrie_with(const Side& Lin, const Side& Rin,
     const float l3 = smax(sE2, mid.s1m);
     const float l2 = 0.5f * (l1 + l3);
     const float dl = l3 - l1;
-    const float invDl = A::rcp(dl);
+    const float invDl = 1.f / dl;
     const float hStarHLL = smax((huL - huR + l3 * hR - l1 * hL) * invDl, 0.f);
 
     const float dh = hR - hL;
@@ -399,14 +372,14 @@ __device__ __forceinline__ EdgeOut augrie_with(const Side& Lin, const Side& Rin,
                        ((l3 > 0.f) && (mid.s2m < 0.f)) || ((uL + cL) * (uR + cR) < 0.f) ||
                        ((uL - cL) * (uR - cR) < 0.f);
 
-    const float invBar = A::rcp(s1s2bar);
+    const float invBar = 1.f / s1s2bar;
     float ddh = sonic ? -db : db * kGravity * hBar * invBar;
     const bool caseA = (l1 < -ct) && (l3 > ct);
     const bool caseB = !caseA && (l1 >= ct);
     const bool caseC = !caseA && !caseB && (l3 <= -ct);
     if (caseA || caseB || caseC) {
         const float hsd = hStarHLL * dl;
-        const float inv13 = A::rcp(l1 * l3);
+        const float inv13 = 1.f / (l1 * l3);
         const float dA = hsd * l1 * inv13;  // hStarHLL dl / l3
         const float dB = hsd * l3 * inv13;  // hStarHLL dl / l1
         const float hiBound = caseA ? dA : (caseB ? dB : hR);
@@ -453,14 +426,11 @@ __device__ __forceinline__ EdgeOut augrie_with(const Side& Lin, const Side& Rin,
     // edge is marked by a negative speed and solved again elsewhere
     if constexpr (MiddleFn::kDefers)
         if (mid.hm < 0.f) o.speed = -1.f;
-    if (still) o = EdgeOut{0.f, 0.f, 0.f, 0.f, still_speed<A>(Lin, Rin)};
+    if (still) o = EdgeOut{0.f, 0.f, 0.f, 0.f, still_speed(Lin, Rin)};
     return o;
 }
 
-template <bool ReuseFirst = false, class A = Ieee>
-__device__ __forceinline__ EdgeOut augrie(const Side& L, const Side& R) {
-    return augrie_with(L, R, ExactMiddle<ReuseFirst, A>());
-}
+__device__ __forceinline__ EdgeOut augrie(const Side& L, const Side& R) { return augrie_with(L, R, ExactMiddle()); }
 
 // ---------------------------------------------------------------------------
 // HLLE in fluctuation form, surface-gradient diffusion (well-balanced)
@@ -495,58 +465,6 @@ __device__ __forceinline__ EdgeOut hlle(const Side& Lin, const Side& Rin) {
     o.speed = smax(fabsf(sL), fabsf(sR));
     if (m.dryL && m.dryR) o = EdgeOut{0.f, 0.f, 0.f, 0.f, 0.f};
     return o;
-}
-
-// One edge with solver S.  ReuseFirst selects the form of the Newton loop
-// (middle_state), A that of divisions and square roots; the results are the
-// same.
-template <int S, bool ReuseFirst = false, class A = Ieee>
-__device__ __forceinline__ EdgeOut solve_edge(const Side& L, const Side& R) {
-    if constexpr (S == SOLVER_FWAVE) return fwave<A>(L, R);
-    if constexpr (S == SOLVER_HLLE) return hlle<A>(L, R);
-    if constexpr (S == SOLVER_HYBRID)
-        if (L.h >= kHybridTol && R.h >= kHybridTol) return fwave<A>(L, R);
-    if constexpr (S == SOLVER_AUGRIE || S == SOLVER_HYBRID) return augrie<ReuseFirst, A>(L, R);
-}
-
-// Solver with per-kernel state, built once at kernel start from an optional
-// parameter block (the learned middle state keeps its network weights in
-// registers; the exact solvers have no state).  kNormalForm: the sweeps solve
-// the edges of ordinary cells with NormalRange (column_edges in kernels_u.hpp).
-template <int S, bool ReuseFirst = false>
-struct SolverCtx {
-    static constexpr bool kNormalForm = true;
-    __device__ __forceinline__ explicit SolverCtx(const unsigned*) {}
-    template <class A = Ieee>
-    __device__ __forceinline__ EdgeOut solve(const Side& L, const Side& R) const {
-        return solve_edge<S, ReuseFirst, A>(L, R);
-    }
-};
-
-// Cells whose edges may be solved with NormalRange: depth and bed below 2^40 and,
-// on a wet cell, velocities below 2^20 in sum.  A dry cell's momentum, velocity,
-// celerity and 1/h reach no result (the augmented solver sets them to zero, the
-// others mirror the wet side, and an edge between two dry cells returns zeros),
-// so every operand of a wet edge is normal:
-//   * h >= 0.01, so celerities lie in [0.3, 2^22] and every sum of two, every
-//     depth sum and its root is bounded away from zero;
-//   * speeds are below 2^23, and the fastest two of an edge differ by at least
-//     2 cHat less their rounding, > 0.3: the divisions by l3 - l1 and s2 - s1;
-//   * 1 / (l1 l3) and 1 / s1s2bar are used only where the operands exceed 1e-12;
-//   * Newton's depths stay between hMin and about 2^60, its two curve roots
-//     above 2^-30, so its denominator lies above 2^-90;
-//   * 2 (cL + cR) - du is zero or at least 2^-24, and its square a normal number.
-// Numerators below 2^-102 occur in two places, the Roe velocity and the Newton
-// step; the first is added to a celerity above 0.2, the second to a depth above
-// 0.01, and neither changes the sum in any rounding.  A NaN fails the test.
-__device__ __forceinline__ bool in_normal_range(float h, float b, float u, float v) {
-    return (fabsf(h) + fabsf(b) <= 0x1p40f) && (h < kDryTol || fabsf(u) + fabsf(v) <= 0x1p20f);
-}
-
-// Convenience for raw edge states (one-off evaluations).
-template <int S, bool ReuseFirst = false, class A = Ieee>
-__device__ __forceinline__ EdgeOut solve_raw(float hL, float hR, float huL, float huR, float bL, float bR) {
-    return solve_edge<S, ReuseFirst, A>(cell_side<A>(hL, huL, bL), cell_side<A>(hR, huR, bR));
 }
 
 }  // namespace dev
