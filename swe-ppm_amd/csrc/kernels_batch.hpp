@@ -366,7 +366,7 @@ __device__ __forceinline__ bool strip_sums(const BatchSolver<S>& solver, const S
     }
     if (N && __any(outside)) return false;
     smaxv = wave_max(smaxv);
-    if ((threadIdx.x & 63) == 0) atomicMax(smax, __float_as_uint(smaxv));
+    if ((threadIdx.x & 63) == 0) raise_max(smax, __float_as_uint(smaxv));
     return true;
 }
 
@@ -642,7 +642,7 @@ __device__ __forceinline__ void fused_tile(const BatchSolver<S>& solver, const S
         }
         if (N && __any(outside)) return false;
         smaxv = wave_max(smaxv);
-        if ((threadIdx.x & 63) == 0) atomicMax(smax, __float_as_uint(smaxv));
+        if ((threadIdx.x & 63) == 0) raise_max(smax, __float_as_uint(smaxv));
         return true;
     };
     run_tile<BatchSolver<S>, 0>(threadIdx.x & 63, body);

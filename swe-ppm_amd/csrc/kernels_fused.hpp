@@ -368,7 +368,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(fused_waves
 
         if (N && __any(outside)) return false;
         if constexpr (!kRecord) smaxRun = __float_as_uint(wave_max(smaxTile));
-        if (lane == 0) atomicMax(&ctl->smax[slotOut], smaxRun);
+        if (lane == 0) raise_max(&ctl->smax[slotOut], smaxRun);
         return true;
     };
     run_tile<dev::SolverCtx<S>, V>(threadIdx.x & 63, tile);

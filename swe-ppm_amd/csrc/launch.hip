@@ -167,7 +167,7 @@ __global__ __launch_bounds__(kPlanGroup) void quiet_plan_kernel(const unsigned* 
     if (threadIdx.x == 0) {
         count[blockIdx.x] = total;
         if (nbusy) atomicAdd(&ctl->busy[slotOut], nbusy);
-        if (mx > 0u) atomicMax(&ctl->smax[slotOut], mx);
+        if (mx > 0u) raise_max(&ctl->smax[slotOut], mx);
     }
 }
 

@@ -110,7 +110,7 @@ __global__ __launch_bounds__(256) void batch_defer_solve_kernel(BatchArena A, co
                 atomicAdd(&sh[cr], o.hR);
                 atomicAdd(&sm[cr], o.huR);
             }
-            if (o.speed > 0.f) atomicMax(&st[blk].smax, __float_as_uint(o.speed));
+            if (o.speed > 0.f) raise_max(&st[blk].smax, __float_as_uint(o.speed));
         }
     }
 }
