@@ -289,7 +289,9 @@ int swe_hip_solve_edges(int solver, int math, int64_t n, const float* hL, const 
 /* Tuning of the device loop (swe_hip_run): strategy 0 = recompute (max pass
  * + update pass), 1 = store (flux pass writing 4 net-update sums + apply
  * pass), 2 = fused (one launch per step that applies the previous update on
- * load; the default); xseg = x columns per wavefront strip (4, 8, 10, 12,
+ * load, or, for HLLE and f-wave with the IEEE arithmetic on blocks of 2^19
+ * cells and more, one that updates and takes the new state's CFL maximum; the
+ * default); xseg = x columns per wavefront strip (4, 8, 10, 12,
  * 16 or 32; the sweeps of strategies 0 and 1 run 4 as 16); -1 keeps the
  * current value.  All strategies and widths give
  * identical results.  Until the caller sets xseg, a block uses the widest of

@@ -40,7 +40,9 @@ struct Ieee {
     __device__ __forceinline__ static float rcp(float b) { return 1.f / b; }
     __device__ __forceinline__ static float div(float a, float b) { return a / b; }
     __device__ __forceinline__ static float sqrt(float x) { return sqrtf(x); }
-    __device__ __forceinline__ static float sqrt0(float x) { return sqrtf(x); }
+    // std::min / std::max semantics (first operand wins ties), not fminf / fmaxf
+    __device__ __forceinline__ static float min(float a, float b) { return (b < a) ? b : a; }
+    __device__ __forceinline__ static float max(float a, float b) { return (a < b) ? b : a; }
 };
 
 struct NormalRange {
@@ -59,6 +61,10 @@ struct NormalRange {
         return __builtin_fmaf(__builtin_fmaf(-g, g, x), 0.5f * y, g);
     }
     __device__ __forceinline__ static float sqrt(float x) { return root(x, __builtin_amdgcn_rsqf(x)); }
+    // one instruction, for results of arithmetic that are no NaN (the sign of a
+    // zero may differ from Ieee's)
+    __device__ __forceinline__ static float min(float a, float b) { return __builtin_fminf(a, b); }
+    __device__ __forceinline__ static float max(float a, float b) { return __builtin_fmaxf(a, b); }
     // x = 0 too: the reciprocal root of a positive number keeps 0 * y at 0
     __device__ __forceinline__ static float sqrt0(float x) {
         return root(x, __builtin_amdgcn_rsqf(__builtin_fmaxf(x, 0x1p-100f)));

@@ -189,6 +189,19 @@ __device__ __forceinline__ void col_set(float* f, size_t col, unsigned bytes, fl
     *col_ptr(f, col, bytes) = value;
 }
 
+// A store that every lane of the wave executes: lanes that hold nothing to
+// store pass kNoStore as their offset, past the column's bound of `pitch`
+// elements, and the hardware's range check drops them.  Without a branch
+// around it the compiler knows how many stores are in flight and waits for a
+// prefetched column's loads only; around a conditional store it has to count
+// on the path without it, and so waits for the last column's stores to be
+// acknowledged as well, in every column.
+constexpr unsigned kNoStore = 0xfffffffcu;
+__device__ __forceinline__ void col_put(float* f, size_t col, int pitch, unsigned bytes, float value) {
+    __builtin_amdgcn_raw_buffer_store_b32(
+        __float_as_uint(value), __builtin_amdgcn_make_buffer_rsrc(f + col, 0, pitch * 4, 0x00020000), bytes, 0, 0);
+}
+
 // dt rule of flavour U (SWE_DimensionalSplittingMpi.cpp:448-456)
 __device__ __forceinline__ float timestep_from_max(float s, float dx, float dy) {
     if (s > kMinSpeed) {
@@ -343,22 +356,19 @@ __device__ __forceinline__ Cell update_cell(float h, float hu, float hv, float d
     c.h = h - (dtdx * sx + dtdy * sy);
     c.hu = hu - dtdx * su;
     c.hv = hv - dtdy * sv;
-    if (c.h < 0.f) {
-        c.h = 0.f;
-        c.hu = 0.f;
-        c.hv = 0.f;
-    } else if (c.h < kClampTol) {
-        c.hu = 0.f;
-        c.hv = 0.f;
-    }
+    // a depth below 0 becomes 0, and a cell below the clamp loses its momentum
+    const bool thin = c.h < kClampTol;
+    c.hu = thin ? 0.f : c.hu;
+    c.hv = thin ? 0.f : c.hv;
+    c.h = c.h < 0.f ? 0.f : c.h;
     return c;
 }
 
 // One loaded cell: state plus the quantities its edges share.
 struct CellQ {
-    float h, hu, hv, b, u, v, c, sq, inv;
-    __device__ __forceinline__ dev::Side xside() const { return dev::Side{h, hu, b, u, c, sq, inv}; }
-    __device__ __forceinline__ dev::Side yside() const { return dev::Side{h, hv, b, v, c, sq, inv}; }
+    float h, hu, hv, b, u, v, c, sq, inv, fx, fy;
+    __device__ __forceinline__ dev::Side xside() const { return dev::Side{h, hu, b, u, c, sq, inv, fx}; }
+    __device__ __forceinline__ dev::Side yside() const { return dev::Side{h, hv, b, v, c, sq, inv, fy}; }
     // the y-side of the cell held by lane + 1 (the cell above), by shuffle
     __device__ __forceinline__ dev::Side yside_from_lane_above() const {
         dev::Side s;
@@ -369,6 +379,7 @@ struct CellQ {
         s.c = __shfl_down(c, 1, 64);
         s.sq = __shfl_down(sq, 1, 64);
         s.inv = __shfl_down(inv, 1, 64);
+        s.f = __shfl_down(fy, 1, 64);
         return s;
     }
 };
@@ -385,6 +396,8 @@ __device__ __forceinline__ CellQ cell_q(float h, float hu, float hv, float b) {
     q.v = hv * q.inv;
     q.sq = A::sqrt(h);
     q.c = kSqrtGravity * q.sq;
+    q.fx = dev::momentum_flux(h, hu, q.u);
+    q.fy = dev::momentum_flux(h, hv, q.v);
     return q;
 }
 

@@ -294,6 +294,16 @@ int launch_fused_u(int solver, int variant, int xseg, StateView v, FusedIO io, B
     return fused_u_v<0>(solver, xseg, v, io, bi, ctl, slotIn, slotOut, slotClear, dtLog, logIdx, stream);
 }
 
+int launch_advance_u(int solver, int xseg, StateView v, float* hn, float* hun, float* hvn, BoundaryInfo bi,
+                     DeviceCtl* ctl, int slotIn, int slotOut, int slotClear, int last, float* dtLog, int logIdx,
+                     hipStream_t stream) {
+    if (solver == SOLVER_HLLE)
+        return launch_advance_u_solver<SOLVER_HLLE>(xseg, v, hn, hun, hvn, bi, ctl, slotIn, slotOut, slotClear, last,
+                                                    dtLog, logIdx, stream);
+    return launch_advance_u_solver<SOLVER_FWAVE>(xseg, v, hn, hun, hvn, bi, ctl, slotIn, slotOut, slotClear, last,
+                                                 dtLog, logIdx, stream);
+}
+
 int launch_solve_edges(int solver, int variant, int64_t n, const float* in, float* out, hipStream_t stream) {
     return variant == 1 ? solve_edges_v<1>(solver, n, in, out, stream) : solve_edges_v<0>(solver, n, in, out, stream);
 }

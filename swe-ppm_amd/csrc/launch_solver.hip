@@ -11,6 +11,7 @@
 #include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
 
+#include "kernels_advance.hpp"
 #include "kernels_fused.hpp"
 #include "kernels_s.hpp"
 #include "kernels_u.hpp"
@@ -144,6 +145,33 @@ template int launch_solve_edges_solver<SWE_SOLVER_ID, SWE_VARIANT>(int64_t, cons
 #endif
 template int launch_fused_u_solver<SWE_SOLVER_ID, SWE_VARIANT>(int, StateView, FusedIO, BoundaryInfo, DeviceCtl*, int,
                                                                int, int, float*, int, hipStream_t);
+
+#if SWE_VARIANT == 0 && (SWE_SOLVER_ID == 0 || SWE_SOLVER_ID == 1)
+template <int S>
+int launch_advance_u_solver(int xseg, StateView v, float* hn, float* hun, float* hvn, BoundaryInfo bi, DeviceCtl* ctl,
+                            int slotIn, int slotOut, int slotClear, int last, float* dtLog, int logIdx,
+                            hipStream_t stream) {
+    const int nyt = (v.ny + kAdvanceRows - 1) / kAdvanceRows;
+    auto go = [&](auto xsTag) {
+        constexpr int XS = decltype(xsTag)::value;
+        const int waves = nyt * ((v.nx + XS - 1) / XS);
+        hipLaunchKernelGGL((advance_u_kernel<S, XS>), dim3((waves + kWavesPerGroup - 1) / kWavesPerGroup),
+                           dim3(64 * kWavesPerGroup), 0, stream, v, hn, hun, hvn, bi, ctl, slotIn, slotOut, slotClear,
+                           last, dtLog, logIdx);
+    };
+    if (xseg >= 32)
+        go(std::integral_constant<int, 32>());
+    else if (xseg >= 16)
+        go(std::integral_constant<int, 16>());
+    else
+        go(std::integral_constant<int, 8>());
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return hip_fail(e, "advance_u_kernel launch");
+    return 0;
+}
+template int launch_advance_u_solver<SWE_SOLVER_ID>(int, StateView, float*, float*, float*, BoundaryInfo, DeviceCtl*,
+                                                    int, int, int, int, float*, int, hipStream_t);
+#endif
 
 #if SWE_VARIANT == 0 && SWE_SOLVER_ID != 4
 template <int S>

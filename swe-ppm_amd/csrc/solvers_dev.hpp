@@ -49,7 +49,12 @@ struct Side {
     float c;    // sqrt(g h)
     float sq;   // sqrt(h)
     float inv;  // 1 / h (the augmented solver's middle state divides by both depths)
+    float f;    // hu u + g h^2 / 2 (momentum flux)
 };
+
+__device__ __forceinline__ float momentum_flux(float h, float hu, float u) {
+    return hu * u + 0.5f * kGravity * h * h;
+}
 
 template <class A = Ieee>
 __device__ __forceinline__ Side cell_side(float h, float hu, float b) {
@@ -61,6 +66,7 @@ __device__ __forceinline__ Side cell_side(float h, float hu, float b) {
     s.u = hu * s.inv;
     s.sq = A::sqrt(h);
     s.c = kSqrtGravity * s.sq;
+    s.f = momentum_flux(h, hu, s.u);
     return s;
 }
 
@@ -82,31 +88,68 @@ __device__ __forceinline__ void acc_wave(float s, float zh, float zhu, EdgeOut& 
 }
 
 // A dry neighbour of an f-wave / HLLE edge is a reflecting wall: the wet
-// state mirrored (h, -hu, b; the velocity negates exactly).
+// state mirrored (h, -hu, b; the velocity negates exactly).  A wave without
+// dry cells keeps its states.
 struct Mirrored {
     Side L, R;
-    bool dryL, dryR, mirrorR;
+    bool dryL, dryR, mirrorR, any;
 };
 __device__ __forceinline__ Mirrored mirror_dry(const Side& L, const Side& R) {
     Mirrored m;
     m.dryL = L.h < kDryTol;
     m.dryR = R.h < kDryTol;
     m.mirrorR = !m.dryL && m.dryR;
-    m.L.h = m.dryL ? R.h : L.h;
-    m.L.hu = m.dryL ? -R.hu : L.hu;
-    m.L.b = m.dryL ? R.b : L.b;
-    m.L.u = m.dryL ? -R.u : L.u;
-    m.L.c = m.dryL ? R.c : L.c;
-    m.L.sq = m.dryL ? R.sq : L.sq;
-    m.L.inv = m.dryL ? R.inv : L.inv;
-    m.R.h = m.mirrorR ? L.h : R.h;
-    m.R.hu = m.mirrorR ? -L.hu : R.hu;
-    m.R.b = m.mirrorR ? L.b : R.b;
-    m.R.u = m.mirrorR ? -L.u : R.u;
-    m.R.c = m.mirrorR ? L.c : R.c;
-    m.R.sq = m.mirrorR ? L.sq : R.sq;
-    m.R.inv = m.mirrorR ? L.inv : R.inv;
+    m.any = __any(m.dryL || m.dryR);
+    m.L = L;
+    m.R = R;
+    if (m.any) {
+        m.L.h = m.dryL ? R.h : L.h;
+        m.L.hu = m.dryL ? -R.hu : L.hu;
+        m.L.b = m.dryL ? R.b : L.b;
+        m.L.u = m.dryL ? -R.u : L.u;
+        m.L.c = m.dryL ? R.c : L.c;
+        m.L.sq = m.dryL ? R.sq : L.sq;
+        m.L.f = m.dryL ? R.f : L.f;  // (-hu)(-u)
+        m.R.h = m.mirrorR ? L.h : R.h;
+        m.R.hu = m.mirrorR ? -L.hu : R.hu;
+        m.R.b = m.mirrorR ? L.b : R.b;
+        m.R.u = m.mirrorR ? -L.u : R.u;
+        m.R.c = m.mirrorR ? L.c : R.c;
+        m.R.sq = m.mirrorR ? L.sq : R.sq;
+        m.R.f = m.mirrorR ? L.f : R.f;
+    }
     return m;
+}
+// the net updates of a mirrored side, and of an edge between two dry cells
+__device__ __forceinline__ void drop_dry(const Mirrored& m, EdgeOut& o) {
+    if (m.any) {
+        o.hL = m.dryL ? 0.f : o.hL;
+        o.huL = m.dryL ? 0.f : o.huL;
+        o.hR = m.mirrorR ? 0.f : o.hR;
+        o.huR = m.mirrorR ? 0.f : o.huR;
+        if (m.dryL && m.dryR) o = EdgeOut{0.f, 0.f, 0.f, 0.f, 0.f};
+    }
+}
+
+// Einfeldt's speeds of an edge between two wet states
+struct Speeds {
+    float s1, s2;
+};
+template <class A>
+__device__ __forceinline__ Speeds einfeldt(const Side& L, const Side& R) {
+    const float uRoe = A::div(L.u * L.sq + R.u * R.sq, L.sq + R.sq);
+    const float cRoe = A::sqrt(kGravity * 0.5f * (L.h + R.h));
+    return Speeds{A::min(L.u - L.c, uRoe - cRoe), A::max(R.u + R.c, uRoe + cRoe)};
+}
+
+// The speed that fwave / hlle report for an edge, alone: HLLE's are cut at 0.
+template <int S, class A>
+__device__ __forceinline__ float edge_speed(const Side& Lin, const Side& Rin) {
+    const Mirrored m = mirror_dry(Lin, Rin);
+    Speeds s = einfeldt<A>(m.L, m.R);
+    if constexpr (S == SOLVER_HLLE) s = Speeds{A::min(s.s1, 0.f), A::max(s.s2, 0.f)};
+    const float speed = A::max(fabsf(s.s1), fabsf(s.s2));
+    return m.any && m.dryL && m.dryR ? 0.f : speed;
 }
 
 // ---------------------------------------------------------------------------
@@ -117,29 +160,28 @@ __device__ __forceinline__ EdgeOut fwave(const Side& Lin, const Side& Rin) {
     const Mirrored m = mirror_dry(Lin, Rin);
     const Side& L = m.L;
     const Side& R = m.R;
-    const float hRoe = 0.5f * (L.h + R.h);
-    const float uRoe = A::div(L.u * L.sq + R.u * R.sq, L.sq + R.sq);
-    const float cRoe = A::sqrt(kGravity * hRoe);
-    const float s1 = smin(L.u - L.c, uRoe - cRoe);
-    const float s2 = smax(R.u + R.c, uRoe + cRoe);
+    const Speeds s = einfeldt<A>(L, R);
+    const float s1 = s.s1, s2 = s.s2;
 
     const float df1 = R.hu - L.hu;
-    const float fR = R.hu * R.u + 0.5f * kGravity * R.h * R.h;
-    const float fL = L.hu * L.u + 0.5f * kGravity * L.h * L.h;
-    const float df2 = (fR - fL) + 0.5f * kGravity * (L.h + R.h) * (R.b - L.b);
+    const float df2 = (R.f - L.f) + 0.5f * kGravity * (L.h + R.h) * (R.b - L.b);
     const float invDs = A::rcp(s2 - s1);
     const float beta1 = (s2 * df1 - df2) * invDs;
     const float beta2 = (df2 - s1 * df1) * invDs;
 
     EdgeOut o{0.f, 0.f, 0.f, 0.f, 0.f};
-    acc_wave(s1, beta1, beta1 * s1, o);
-    acc_wave(s2, beta2, beta2 * s2, o);
-    o.hL = m.dryL ? 0.f : o.hL;
-    o.huL = m.dryL ? 0.f : o.huL;
-    o.hR = m.mirrorR ? 0.f : o.hR;
-    o.huR = m.mirrorR ? 0.f : o.huR;
-    o.speed = smax(fabsf(s1), fabsf(s2));
-    if (m.dryL && m.dryR) o = EdgeOut{0.f, 0.f, 0.f, 0.f, 0.f};
+    if (__all(s1 < -kZeroTol && s2 > kZeroTol)) {
+        // the waves part in every lane: one to each side (added to +0 as below)
+        o.hL = 0.f + beta1;
+        o.huL = 0.f + beta1 * s1;
+        o.hR = 0.f + beta2;
+        o.huR = 0.f + beta2 * s2;
+    } else {
+        acc_wave(s1, beta1, beta1 * s1, o);
+        acc_wave(s2, beta2, beta2 * s2, o);
+    }
+    o.speed = A::max(fabsf(s1), fabsf(s2));
+    drop_dry(m, o);
     return o;
 }
 
@@ -440,14 +482,11 @@ __device__ __forceinline__ EdgeOut hlle(const Side& Lin, const Side& Rin) {
     const Mirrored m = mirror_dry(Lin, Rin);
     const Side& L = m.L;
     const Side& R = m.R;
-    const float uRoe = A::div(L.u * L.sq + R.u * R.sq, L.sq + R.sq);
-    const float cRoe = A::sqrt(kGravity * 0.5f * (L.h + R.h));
-    const float sL = smin(smin(L.u - L.c, uRoe - cRoe), 0.f);
-    const float sR = smax(smax(R.u + R.c, uRoe + cRoe), 0.f);
+    const Speeds s = einfeldt<A>(L, R);
+    const float sL = A::min(s.s1, 0.f);
+    const float sR = A::max(s.s2, 0.f);
     const float df1 = R.hu - L.hu;
-    const float fR = R.hu * R.u + 0.5f * kGravity * R.h * R.h;
-    const float fL = L.hu * L.u + 0.5f * kGravity * L.h * L.h;
-    const float df2 = (fR - fL) + 0.5f * kGravity * (L.h + R.h) * (R.b - L.b);
+    const float df2 = (R.f - L.f) + 0.5f * kGravity * (L.h + R.h) * (R.b - L.b);
     const float dq1 = (R.h + R.b) - (L.h + L.b);  // surface-gradient form: lake at rest stays at rest
     const float dq2 = R.hu - L.hu;
     const float invDs = A::rcp(sR - sL);
@@ -458,12 +497,8 @@ __device__ __forceinline__ EdgeOut hlle(const Side& Lin, const Side& Rin) {
     o.huL = sL * q2;
     o.hR = df1 - o.hL;
     o.huR = df2 - o.huL;
-    o.hL = m.dryL ? 0.f : o.hL;
-    o.huL = m.dryL ? 0.f : o.huL;
-    o.hR = m.mirrorR ? 0.f : o.hR;
-    o.huR = m.mirrorR ? 0.f : o.huR;
-    o.speed = smax(fabsf(sL), fabsf(sR));
-    if (m.dryL && m.dryR) o = EdgeOut{0.f, 0.f, 0.f, 0.f, 0.f};
+    o.speed = A::max(fabsf(sL), fabsf(sR));
+    drop_dry(m, o);
     return o;
 }
 

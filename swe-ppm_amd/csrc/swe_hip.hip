@@ -14,6 +14,7 @@
 
 #include "../../include/swe_hip.h"
 #include "../../include/swe_hip_mlp.h"
+#include "kernels_advance.hpp"
 #include "kernels_s.hpp"
 #include "kernels_u.hpp"
 #include "swe_internal.h"
@@ -131,6 +132,22 @@ namespace {
 
 size_t field_elems(const swe_hip_block* k) { return (size_t)(k->nx + 2) * k->pitch; }
 
+// Compute units of the current device (0: unknown).
+int device_cus() {
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
+        return 0;
+    return cus;
+}
+
+// Cells from which the light solvers' device loop takes the one-pass form.
+// Measured (islands, us per step, f-wave / HLLE, fused at its default width
+// against one pass): 512^2 21 / 17 against 20 / 17, 768^2 25 / 21 against 21 /
+// 19, 1024^2 28 / 22 against 23 / 22, 2048^2 59 / 54 against 46 / 44, 3000^2 154 /
+// 152 against 77 / 77, 4096^2 276 / 275 against 141 / 140.
+constexpr long kAdvanceCells = 1l << 19;
+
 // Default strip width of a flavour-U block.  A wider segment loads and solves
 // fewer halo columns per owned column and pays a wave's fixed start fewer
 // times, but gives fewer waves; narrow segments spread the work more evenly
@@ -155,10 +172,8 @@ size_t field_elems(const swe_hip_block* k) { return (size_t)(k->nx + 2) * k->pit
 //   learned 2048^2  181 /  174 /  166 /  172 / 220   (12); 3000^2: 285 at 12, 280 at 16 (16)
 //   HLLE 2048^2     129 /  116 /  105 /   95 /  90   (16); f-wave 134 / 122 / 104 / 96 / 100 (16)
 int default_xseg(int nx, int ny, int solver) {
-    int dev = 0, cus = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
-        return 8;
+    const int cus = device_cus();
+    if (cus <= 0) return 8;
     const double strips = (double)((ny + kStripRows - 1) / kStripRows);
     const double simds = 4.0 * cus;
     static const double heavy[3] = {12.0, 4.0, 0.0}, learned[3] = {5.0, 3.0, 0.0}, light[3] = {2.0, 1.0, 0.0};
@@ -169,6 +184,25 @@ int default_xseg(int nx, int ny, int solver) {
     const int widths[3] = {16, 12, 8};
     for (int i = 0; i < 3; i++)
         if (strips * ((nx + widths[i] - 1) / widths[i]) / simds >= t[i]) return widths[i];
+    return 8;
+}
+
+// Whether the fused strategy's device loop takes the one-pass form
+// (kernels_advance.hpp): the light solvers on blocks whose state and sums pass
+// through memory every step.
+bool advance_pays(const swe_hip_block* k) {
+    return k->strategy == 2 && k->math == 0 && (k->solver == SOLVER_HLLE || k->solver == SOLVER_FWAVE) &&
+           (long)k->nx * k->ny >= kAdvanceCells;
+}
+// Its strip width until the caller sets one: the widest that still gives every
+// SIMD eight waves.  Measured at 8 / 16 / 32 columns (f-wave, us per step):
+// 1024^2 23 / 33 / 59, 2048^2 46 / 46 / 63, 3000^2 80 / 77 / 84, 4096^2 152 / 143 /
+// 144.
+int advance_width(const swe_hip_block* k) {
+    if (k->xsegSet) return k->xseg;
+    const double strips = (double)((k->ny + kAdvanceRows - 1) / kAdvanceRows), simds = 4.0 * device_cus();
+    for (int w : {32, 16})
+        if (strips * ((k->nx + w - 1) / w) / simds >= 8.0) return w;
     return 8;
 }
 
@@ -454,7 +488,8 @@ int run_u_device_loop(swe_hip_block* k, int nsteps, float* t_inout, float* dt_lo
     if (int r = ensure_dtlog(k, nsteps)) return r;
     if (k->strategy == 0 || k->strategy == 2)
         if (int r = ensure_second_buffer(k)) return r;
-    if (k->strategy == 2) {
+    const bool onePass = advance_pays(k);
+    if (k->strategy == 2 && !onePass) {
         if (int r = ensure_second_sums(k)) return r;
         if (int r = ensure_quiet_record(k)) return r;
     }
@@ -468,7 +503,24 @@ int run_u_device_loop(swe_hip_block* k, int nsteps, float* t_inout, float* dt_lo
     if (int r = launch_ctl_reset(k->ctl, 0, k->stream)) return r;
     if (tm) HIP_TRY(tm->mark(k->stream, 0));
     if (int r = launch_apply_bc(view(k, k->cur), k->bi, k->stream)) return r;
-    if (k->strategy == 2) {
+    if (onePass) {
+        // light solvers: max sweep on Q(0), then one launch per step
+        for (int slot = 1; slot < 3; ++slot)
+            if (int r = launch_ctl_reset(k->ctl, slot, k->stream)) return r;
+        if (tm && tm->perKernel) HIP_TRY(tm->mark(k->stream, 1));
+        if (int r = launch_sweep_u(k->solver, k->math, MODE_MAX, k->xseg, view(k, k->cur), sums_view(k), nullptr,
+                                   nullptr, nullptr, k->bi, k->ctl, Slots{0, 1}, -1.f, 0, nullptr, 0, k->stream))
+            return r;
+        for (int s = 0; s < nsteps; ++s) {
+            const int o = k->cur ^ 1;
+            if (tm && tm->perKernel) HIP_TRY(tm->mark(k->stream, 1));
+            if (int r = launch_advance_u(k->solver, advance_width(k), view(k, k->cur), k->h[o], k->hu[o], k->hv[o],
+                                         k->bi, k->ctl, s % 3, (s + 1) % 3, (s + 2) % 3, s + 1 == nsteps, k->dtlog, s,
+                                         k->stream))
+                return r;
+            k->cur = o;
+        }
+    } else if (k->strategy == 2) {
         // fused: sweep(STORE) on Q(0), then one launch per step that applies
         // the previous update on load, then the last update
         for (int slot = 1; slot < 3; ++slot)

@@ -102,6 +102,14 @@ int launch_fused_u_solver(int xseg, StateView v, FusedIO io, BoundaryInfo bi, De
                           int slotClear, float* dtLog, int logIdx, hipStream_t stream);
 int launch_fused_u(int solver, int variant, int xseg, StateView v, FusedIO io, BoundaryInfo bi, DeviceCtl* ctl,
                    int slotIn, int slotOut, int slotClear, float* dtLog, int logIdx, hipStream_t stream);
+// One-pass step of the light solvers (kernels_advance.hpp; HLLE or f-wave).
+template <int S>
+int launch_advance_u_solver(int xseg, StateView v, float* hn, float* hun, float* hvn, BoundaryInfo bi, DeviceCtl* ctl,
+                            int slotIn, int slotOut, int slotClear, int last, float* dtLog, int logIdx,
+                            hipStream_t stream);
+int launch_advance_u(int solver, int xseg, StateView v, float* hn, float* hun, float* hvn, BoundaryInfo bi,
+                     DeviceCtl* ctl, int slotIn, int slotOut, int slotClear, int last, float* dtLog, int logIdx,
+                     hipStream_t stream);
 // Learned middle state with deferred hard edges (launch_defer.hip): the
 // deferring fused sweep (io.deferQ set), then the launch that solves the
 // edges it queued in ctl->defer[slotOut] and completes the sums of vNew.
