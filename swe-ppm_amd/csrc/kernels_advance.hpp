@@ -43,9 +43,9 @@ advance_u_kernel(StateView v, float* hn, float* hun, float* hvn, BoundaryInfo bi
     const int nx = v.nx, ny = v.ny;
     const int nyt = (ny + kAdvanceRows - 1) / kAdvanceRows;
     const int nxs = (nx + XS - 1) / XS;
-    const float dt = timestep_from_max(__uint_as_float(ctl->smax[slotIn]), v.dx, v.dy);
+    const float dt = timestep_from_max(ctl->smax[slotIn].value(), v.dx, v.dy);
+    if (blockIdx.x == 0) ctl->smax[slotClear].clear();
     if (blockIdx.x == 0 && threadIdx.x == 0) {
-        ctl->smax[slotClear] = 0u;
         ctl->dt = dt;
         ctl->t += dt;
         ctl->steps += 1;
@@ -175,8 +175,8 @@ advance_u_kernel(StateView v, float* hn, float* hun, float* hvn, BoundaryInfo bi
         }
         if (N && __any(outside)) return false;
         if (!last) {
-            const float smaxv = wave_max(dev::smax(owned ? smaxX : 0.f, hEdge ? smaxY : 0.f));
-            if (lane == 0) raise_max(&ctl->smax[slotOut], __float_as_uint(smaxv));
+            const float smaxv = wave_max<N>(dev::smax(owned ? smaxX : 0.f, hEdge ? smaxY : 0.f));
+            if (lane == 0) raise_max(ctl->smax[slotOut], __float_as_uint(smaxv));
         }
         return true;
     };

@@ -365,7 +365,7 @@ __device__ __forceinline__ bool strip_sums(const BatchSolver<S>& solver, const S
         carryHu = ev.huR;
     }
     if (N && __any(outside)) return false;
-    smaxv = wave_max(smaxv);
+    smaxv = wave_max<N>(smaxv);
     if ((threadIdx.x & 63) == 0) raise_max(smax, __float_as_uint(smaxv));
     return true;
 }
@@ -641,7 +641,7 @@ __device__ __forceinline__ void fused_tile(const BatchSolver<S>& solver, const S
             cq = nq;
         }
         if (N && __any(outside)) return false;
-        smaxv = wave_max(smaxv);
+        smaxv = wave_max<N>(smaxv);
         if ((threadIdx.x & 63) == 0) raise_max(smax, __float_as_uint(smaxv));
         return true;
     };

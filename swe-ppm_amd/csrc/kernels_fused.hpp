@@ -158,9 +158,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(fused_waves
     const int nxs = (v.nx + XS - 1) / XS;
     const int nx = v.nx, ny = v.ny;
 
-    const float dt = io.dtFixed >= 0.f ? io.dtFixed : timestep_from_max(__uint_as_float(ctl->smax[slotIn]), v.dx, v.dy);
+    const float dt = io.dtFixed >= 0.f ? io.dtFixed : timestep_from_max(ctl->smax[slotIn].value(), v.dx, v.dy);
+    if (blockIdx.x == 0) ctl->smax[slotClear].clear();
     if (blockIdx.x == 0 && threadIdx.x == 0) {
-        ctl->smax[slotClear] = 0u;
         ctl->defer[slotClear] = 0u;
         ctl->busy[slotClear] = 0u;
         ctl->dt = dt;
@@ -347,7 +347,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(fused_waves
             // in some record, and each record's edges lie in its tile's footprint.
             // A deferred edge at the boundary touches both tiles.
             if (kRecord && ((x & (kQuietCols - 1)) == 0 || x == x1)) {  // uniform per wave
-                const float tileMax = wave_max(smaxTile);
+                const float tileMax = wave_max<N>(smaxTile);
                 smaxRun = max(smaxRun, __builtin_amdgcn_readfirstlane(__float_as_uint(tileMax)));
                 if (io.quiet) {
                     unsigned quiet = 0u;
@@ -367,8 +367,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(fused_waves
         }
 
         if (N && __any(outside)) return false;
-        if constexpr (!kRecord) smaxRun = __float_as_uint(wave_max(smaxTile));
-        if (lane == 0) raise_max(&ctl->smax[slotOut], smaxRun);
+        if constexpr (!kRecord) smaxRun = __float_as_uint(wave_max<N>(smaxTile));
+        if (lane == 0) raise_max(ctl->smax[slotOut], smaxRun);
         return true;
     };
     run_tile<dev::SolverCtx<S>, V>(threadIdx.x & 63, tile);

@@ -72,8 +72,8 @@ __global__ __launch_bounds__(256) void sweep_s_x_kernel(StateView v, SumsView su
             cb = nb;
         }
         if (N && __any(outside)) return false;
-        smaxv = wave_max(smaxv);
-        if (lane == 0) raise_max(&ctl->smax[par], __float_as_uint(smaxv));
+        smaxv = wave_max<N>(smaxv);
+        if (lane == 0) raise_max(ctl->smax[par], __float_as_uint(smaxv));
         return true;
     };
     run_tile<dev::SolverCtx<S>, 0>(threadIdx.x & 63, tile);

@@ -137,11 +137,34 @@ struct BoundaryInfo {
     int type[4];  // BoundaryType per side
 };
 
-// Device control block of one SWE block: the CFL maxima (two, used
-// alternately so that a step can clear the next one without a memset),
+// A CFL maximum (float bits of non-negative speeds: unsigned order == float
+// order), kept in kCflWords words, one to a cache line: workgroup g raises word
+// g % kCflWords, and the maximum is that over the words.  Consecutive
+// workgroups go to the chip's dies in turn, so a word is raised from one die;
+// see raise_max for what one word costs.  With the maximum over a wave's lanes
+// taken by data-parallel primitives, us per step with one word and with eight:
+// AugRie 2048^2 with every cell moving 114 -> 107, split step 1024^2 137 -> 125.
+constexpr int kCflWords = 8, kCflStride = 32;
+struct CflMax {
+    unsigned int word[kCflWords * kCflStride];
+    __device__ __forceinline__ unsigned bits() const {
+        unsigned m = 0u;
+#pragma unroll
+        for (int i = 0; i < kCflWords; ++i) m = max(m, word[i * kCflStride]);
+        return m;
+    }
+    __device__ __forceinline__ float value() const { return __uint_as_float(bits()); }
+    // by the first threads of one workgroup
+    __device__ __forceinline__ void clear() {
+        if (threadIdx.x < kCflWords) word[threadIdx.x * kCflStride] = 0u;
+    }
+};
+
+// Device control block of one SWE block: the CFL maxima (three, used in
+// turn so that a step can clear the next one without a memset),
 // the current dt and simulated time and a per-step dt log.
 struct DeviceCtl {
-    unsigned int smax[3];  // float bits of non-negative speeds: unsigned order == float order
+    CflMax smax[3];
     float dt;
     float t;
     int steps;
@@ -212,10 +235,30 @@ __device__ __forceinline__ float timestep_from_max(float s, float dx, float dy) 
     return FLT_MAX;
 }
 
+// The maximum over the wave's lanes.  Dpp: by data-parallel-primitive moves
+// (within rows of 16 lanes, then across rows), valid in lane 63 and returned as a
+// uniform value; for non-negative numbers without NaN.  It takes about a tenth
+// of the time of the exchange through LDS.
+template <int Ctrl>
+__device__ __forceinline__ float dpp_max_step(float v) {
+    const int o = __builtin_amdgcn_update_dpp(0, __float_as_int(v), Ctrl, 0xf, 0xf, false);
+    return __builtin_fmaxf(v, __int_as_float(o));
+}
+template <bool Dpp = false>
 __device__ __forceinline__ float wave_max(float v) {
+    if constexpr (Dpp) {
+        v = dpp_max_step<0x111>(v);  // row_shr:1, 2, 4, 8; lanes shifted in read +0
+        v = dpp_max_step<0x112>(v);
+        v = dpp_max_step<0x114>(v);
+        v = dpp_max_step<0x118>(v);
+        v = dpp_max_step<0x142>(v);  // row_bcast:15
+        v = dpp_max_step<0x143>(v);  // row_bcast:31
+        return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
+    } else {
 #pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) v = dev::smax(v, __shfl_xor(v, off, 64));
-    return v;
+        for (int off = 32; off >= 1; off >>= 1) v = dev::smax(v, __shfl_xor(v, off, 64));
+        return v;
+    }
 }
 
 // Raise a maximum of the running launch (float bits of a non-negative number)
@@ -226,9 +269,13 @@ __device__ __forceinline__ float wave_max(float v) {
 // wave set a launch's time wherever waves are short.  us per step with an
 // atomic per wave and in this form: f-wave 2048^2 in 16-column strips (4352
 // waves) 93 -> 62, Hybrid 1500 x 901 90 -> 76, AugRie 2048^2 with every cell
-// moving 132 -> 120, 2048^2 islands 43 -> 40, 4096^2 trench 65 -> 49.
+// moving 132 -> 120, 2048^2 islands 43 -> 40, 4096^2 trench 65 -> 49.  (Waves that
+// end together all find the old value, hence the several words of a CflMax.)
 __device__ __forceinline__ void raise_max(unsigned* m, unsigned bits) {
     if (bits > __hip_atomic_load(m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(m, bits);
+}
+__device__ __forceinline__ void raise_max(CflMax& m, unsigned bits) {
+    raise_max(&m.word[(blockIdx.x % kCflWords) * kCflStride], bits);
 }
 
 // Deferred edges (SOLVER_AUGRIE_DEFER).  An entry is (x, y) of the edge's left
@@ -453,7 +500,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MODE == MOD
 
     float dtdx = 0.f, dtdy = 0.f, dt = 0.f;
     if (MODE == MODE_UPDATE) {
-        dt = dtFixed >= 0.f ? dtFixed : timestep_from_max(__uint_as_float(ctl->smax[sl.use]), v.dx, v.dy);
+        dt = dtFixed >= 0.f ? dtFixed : timestep_from_max(ctl->smax[sl.use].value(), v.dx, v.dy);
         dtdx = dt / v.dx;
         dtdy = dt / v.dy;
     }
@@ -592,16 +639,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MODE == MOD
 
         if (N && __any(outside)) return false;
         if (MODE != MODE_UPDATE) {
-            smaxv = wave_max(smaxv);
-            if (lane == 0) raise_max(&ctl->smax[sl.use], __float_as_uint(smaxv));
+            smaxv = wave_max<N>(smaxv);
+            if (lane == 0) raise_max(ctl->smax[sl.use], __float_as_uint(smaxv));
         }
         return true;
     };
     run_tile<dev::SolverCtx<S>, V>(threadIdx.x & 63, tile);
 
     if (MODE == MODE_UPDATE) {
+        if (blockIdx.x == 0) ctl->smax[sl.clear].clear();  // a later step's maximum starts from zero
         if (blockIdx.x == 0 && threadIdx.x == 0) {
-            ctl->smax[sl.clear] = 0u;  // a later step's maximum starts from zero
             if (dtFixed < 0.f) {
                 ctl->dt = dt;
                 ctl->t += dt;
@@ -620,7 +667,7 @@ __global__ __launch_bounds__(256) void apply_u_kernel(StateView v, SumsView sums
     const int y = blockIdx.x * 64 + (threadIdx.x & 63) + 1;
     const int xseg = blockIdx.y * 4 + (threadIdx.x >> 6);
     const int x0 = 1 + xseg * XS;
-    const float dt = dtFixed >= 0.f ? dtFixed : timestep_from_max(__uint_as_float(ctl->smax[sl.use]), v.dx, v.dy);
+    const float dt = dtFixed >= 0.f ? dtFixed : timestep_from_max(ctl->smax[sl.use].value(), v.dx, v.dy);
     const float dtdx = dt / v.dx;
     const float dtdy = dt / v.dy;
     if (y <= v.ny && x0 <= v.nx) {
@@ -635,8 +682,8 @@ __global__ __launch_bounds__(256) void apply_u_kernel(StateView v, SumsView sums
             if (fuseBc) write_boundary_ghosts(v, bi, x, y, nc.h, nc.hu, nc.hv, v.h, v.hu, v.hv);
         }
     }
+    if (blockIdx.x == 0 && blockIdx.y == 0) ctl->smax[sl.clear].clear();
     if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) {
-        ctl->smax[sl.clear] = 0u;
         if (dtFixed < 0.f) {
             ctl->dt = dt;
             ctl->t += dt;

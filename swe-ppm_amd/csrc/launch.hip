@@ -103,7 +103,7 @@ __global__ __launch_bounds__(kPlanGroup) void quiet_plan_kernel(const unsigned* 
     const int slotNow = (step & 1) * tiles, slotPrev = ((step - 1) & 1) * tiles;
     const unsigned prevBusy = ctl->busy[slotPrev3];
     if (rbSeq != 0u && blockIdx.x == 0 && threadIdx.x == 0)  // the previous launch's maximum to the host
-        __hip_atomic_store(&ctl->ring[rbSeq % kReadbackRing], ((unsigned long long)rbSeq << 32) | ctl->smax[slotPrev3],
+        __hip_atomic_store(&ctl->ring[rbSeq % kReadbackRing], ((unsigned long long)rbSeq << 32) | ctl->smax[slotPrev3].bits(),
                            __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     const int piece = prevBusy == 0u ? fine : (int)min((unsigned)fine, max(1u, (prevBusy + kPlanWaves - 1) / kPlanWaves));
     const int yt = seg % nyt, xs = seg / nyt;
@@ -167,7 +167,7 @@ __global__ __launch_bounds__(kPlanGroup) void quiet_plan_kernel(const unsigned* 
     if (threadIdx.x == 0) {
         count[blockIdx.x] = total;
         if (nbusy) atomicAdd(&ctl->busy[slotOut], nbusy);
-        if (mx > 0u) raise_max(&ctl->smax[slotOut], mx);
+        if (mx > 0u) raise_max(ctl->smax[slotOut], mx);
     }
 }
 
@@ -179,14 +179,14 @@ __global__ __launch_bounds__(kPlanGroup) void quiet_plan_kernel(const unsigned* 
 // the host learns the maximum while the stream runs on.
 __global__ void readback_kernel(const DeviceCtl* ctl, int slot, unsigned seq) {
     if (threadIdx.x == 0) {
-        const unsigned long long w = ((unsigned long long)seq << 32) | ctl->smax[slot];
+        const unsigned long long w = ((unsigned long long)seq << 32) | ctl->smax[slot].bits();
         __hip_atomic_store(&ctl->ring[seq % kReadbackRing], w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
 }
 
 __global__ void ctl_reset_kernel(DeviceCtl* ctl, int par) {
+    if (blockIdx.x == 0) ctl->smax[par].clear();
     if (threadIdx.x == 0 && blockIdx.x == 0) {
-        ctl->smax[par] = 0u;
         ctl->defer[par] = 0u;
         ctl->busy[par] = 0u;
     }

@@ -56,7 +56,7 @@ __global__ __launch_bounds__(256) void defer_solve_kernel(StateView v, SumsView 
         }
     }
     smaxv = wave_max(smaxv);
-    if (lane == 0 && smaxv > 0.f) raise_max(&ctl->smax[slot], __float_as_uint(smaxv));
+    if (lane == 0 && smaxv > 0.f) raise_max(ctl->smax[slot], __float_as_uint(smaxv));
 }
 
 }  // namespace

@@ -1099,8 +1099,9 @@ int swe_hip_fluxes(swe_hip_block* k, float* max_timestep) {
     } else {
         if (int r = launch_ctl_reset(k->ctl, 0, k->stream)) return r;
         if (int r = launch_sweep_s_x(k->solver, view(k, k->cur), sums_view(k), k->ctl, 0, k->stream)) return r;
-        HIP_TRY(hipMemcpyAsync(&bits, &k->ctl->smax[0], sizeof(bits), hipMemcpyDeviceToHost, k->stream));
-        HIP_TRY(hipStreamSynchronize(k->stream));
+        if (++k->rbSeq == 0u) k->rbSeq = 1u;  // 0 means "no report"
+        if (int r = launch_readback(k->ctl, 0, k->rbSeq, k->stream)) return r;
+        if (int r = wait_readback(k, k->rbSeq, &bits)) return r;
         float s;
         std::memcpy(&s, &bits, sizeof(s));
         const float dt = (float).4 * (k->dx / s);  // SWE_DimensionalSplitting.cpp:221, no zero guard
