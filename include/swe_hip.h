@@ -298,7 +298,9 @@ int swe_hip_solve_edges(int solver, int math, int64_t n, const float* hL, const 
  * 16 and 12 for which nyt * ceil(nx/xseg) / (CUs * 4) reaches the solver's
  * threshold (nyt = ceil(ny/62); AugRie 12, 4; with a learned middle state
  * attached 5, 3; HLLE, f-wave, Hybrid 2, 1), else 8 (swe_hip_set_surrogate
- * re-picks it).  The fused loop skips quiet tiles (swe_hip_set_quiet_skip)
+ * re-picks it); with strategy 2 a block too small to fill the GPU at that
+ * width runs strips of 1, 2 or 4 columns instead (HLLE and f-wave on larger
+ * blocks: their one-pass launch picks 8, 16 or 32).  The fused loop skips quiet tiles (swe_hip_set_quiet_skip)
  * at widths that are multiples of 4. */
 int swe_hip_set_tuning(swe_hip_block* blk, int strategy, int xseg);
 int swe_hip_get_tuning(swe_hip_block* blk, int* strategy, int* xseg);

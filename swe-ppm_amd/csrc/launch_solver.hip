@@ -45,6 +45,9 @@ int go_u(StateView v, SumsView sums, float* hn, float* hun, float* hvn, Boundary
 template <int S, int MODE, int V>
 int go_u_xs(int xseg, StateView v, SumsView sums, float* hn, float* hun, float* hvn, BoundaryInfo bi,
             DeviceCtl* ctl, Slots sl, float dtFixed, int fuseBc, float* dtLog, int logIdx, hipStream_t stream) {
+    if constexpr (V == 0 && MODE == MODE_STORE)
+        if (xseg <= 2)  // the first pass of a small block (narrow_width)
+            return go_u<S, MODE, 2, V>(v, sums, hn, hun, hvn, bi, ctl, sl, dtFixed, fuseBc, dtLog, logIdx, stream);
     switch (xseg) {
         case 8:
         case 10:  // width 10 runs the sweeps at 8
@@ -111,7 +114,11 @@ int launch_fused_u_solver(int xseg, StateView v, FusedIO io, BoundaryInfo bi, De
                                bi, ctl, slotIn, slotOut, slotClear, dtLog, logIdx);
         }
     };
-    if (xseg == 4)
+    if (V == 0 && xseg == 1)  // narrow widths of small blocks (narrow_width)
+        go(std::integral_constant<int, V == 0 ? 1 : 8>());
+    else if (V == 0 && xseg == 2)
+        go(std::integral_constant<int, V == 0 ? 2 : 8>());
+    else if (xseg == 4)
         go(std::integral_constant<int, 4>());
     else if (xseg == 10)
         go(std::integral_constant<int, 10>());

@@ -54,6 +54,8 @@ struct swe_hip_block {
     int math = 0;      // 0 IEEE (bit-compatible), 1 fast
     int xseg = 8;      // columns per wavefront strip (default_xseg)
     bool xsegSet = false;  // set by the caller: kept when a network is attached or detached
+    bool narrowOk = true;  // the fused strategy may take narrow_width instead
+    int cus = 256;         // compute units of the block's device
     int cur = 0;       // index of the current state buffer
     BoundaryInfo bi{{PASSIVE, PASSIVE, PASSIVE, PASSIVE}};
     float* h[2] = {nullptr, nullptr};
@@ -171,8 +173,7 @@ constexpr long kAdvanceCells = 1l << 19;
 //          8192^2  1879 / 1417 / 1387 / 1346 / 1360  (16)
 //   learned 2048^2  181 /  174 /  166 /  172 / 220   (12); 3000^2: 285 at 12, 280 at 16 (16)
 //   HLLE 2048^2     129 /  116 /  105 /   95 /  90   (16); f-wave 134 / 122 / 104 / 96 / 100 (16)
-int default_xseg(int nx, int ny, int solver) {
-    const int cus = device_cus();
+int default_xseg(int nx, int ny, int solver, int cus) {
     if (cus <= 0) return 8;
     const double strips = (double)((ny + kStripRows - 1) / kStripRows);
     const double simds = 4.0 * cus;
@@ -200,10 +201,52 @@ bool advance_pays(const swe_hip_block* k) {
 // 144.
 int advance_width(const swe_hip_block* k) {
     if (k->xsegSet) return k->xseg;
-    const double strips = (double)((k->ny + kAdvanceRows - 1) / kAdvanceRows), simds = 4.0 * device_cus();
+    const double strips = (double)((k->ny + kAdvanceRows - 1) / kAdvanceRows), simds = 4.0 * k->cus;
     for (int w : {32, 16})
         if (strips * ((k->nx + w - 1) / w) / simds >= 8.0) return w;
     return 8;
+}
+
+// Strip width of the fused strategy on a block that does not fill the GPU at
+// default_xseg's widths, or 0.  One wave's columns are a chain of dependent
+// operations, about 1 us per column for the light solvers and 3 for the
+// augmented one, so a launch of few waves lasts as long as its widest strip;
+// once a SIMD has a few waves the halo column per strip costs more than
+// that saves.  The narrowest width is taken whose waves per SIMD stay below
+// the solver's limit.  Measured, us per step at 1 / 2 / 4 / 8 columns:
+//   f-wave 64x50     7.1 /  8.7 / 10.7 / 14.3     256^2   13.2 / 11.1 / 12.7 / 18.0
+//          512^2    22.1 / 16.9 / 15.7 / 19.2     1000x500 34.1 / 25.6 / 19.2 / 21.1
+//   Hybrid 64x50    13.9 / 16.9 / 21.6 / 25.1     256^2   18.3 / 20.4 / 31.6 / 47.6
+//          512^2    27.0 / 24.5 / 34.4 / 53.7     1500x901 47.3 / 48.9 / 45.2 / 54.6
+//          2048^2   90.8 / 80.3 / 77.9 / 79.7     4096^2   341 / 306 / 274 / 280
+//   AugRie 64x50    11.9 / 16.2 / 27.6 / 28.3     256^2   15.5 / 17.6 / 31.1 / 32.2
+//          512^2    26.7 / 21.2 / 32.8 / 33.7     1000x500 36.0 / 29.8 / 33.2 / 34.0
+//          1024^2   42.3 / 42.2 / 33.8 / 34.4
+// (AugRie's 4 and 8 columns record and skip quiet tiles, which the narrower
+// ones do not: there a lake at rest is solved edge by edge, and on larger
+// blocks that costs more.)
+int narrow_width(int nx, int ny, int solver, int cus) {
+    struct Limit {
+        int width;
+        double waves;  // per SIMD
+    };
+    static const Limit light[] = {{1, 0.625}, {2, 1.0}, {4, 2.25}}, hybrid[] = {{1, 2.0}, {2, 4.5}, {4, 1e30}},
+                       augrie[] = {{1, 2.0}, {2, 4.5}, {0, 1e30}};
+    const Limit* t = solver == SOLVER_AUGRIE ? augrie : solver == SOLVER_HYBRID ? hybrid : light;
+    const double strips = (double)((ny + kStripRows - 1) / kStripRows);
+    for (int i = 0; i < 3; ++i)
+        if (strips * ((nx + std::max(t[i].width, 1) - 1) / std::max(t[i].width, 1)) <= t[i].waves * 4.0 * cus)
+            return t[i].width;
+    return 0;
+}
+
+// Strip width of the fused strategy's launches: the caller's or the autotuner's
+// choice, else the narrow width of a small block, else default_xseg's.  (The
+// fast arithmetic and the learned middle state keep the wider strips.)
+int launch_width(const swe_hip_block* k) {
+    if (!k->narrowOk || k->math != 0 || k->mlp || k->strategy != 2 || k->cus <= 0) return k->xseg;
+    const int w = narrow_width(k->nx, k->ny, k->solver, k->cus);
+    return w > 0 ? w : k->xseg;
 }
 
 // AugRie with a network attached runs the learned-middle-state instantiation
@@ -366,13 +409,13 @@ int pc_fused(swe_hip_block* k, int slotIn, int out, float dtFixed, unsigned rbSe
     io.dtFixed = dtFixed;
     const int step = k->pcStep + 1;
     const int es = eff_solver(k);
-    if (k->skipQuiet && es == SOLVER_AUGRIE && k->xseg % kQuietCols == 0) {
+    if (k->skipQuiet && es == SOLVER_AUGRIE && launch_width(k) % kQuietCols == 0) {
         if (int r = ensure_quiet_record(k)) return r;
         io.quiet = k->quiet;
         io.speed = k->tspeed;
         io.step = step;
         if (step >= 3) {
-            if (int r = launch_quiet_plan(k->quiet, k->tspeed, k->nx, k->ny, k->xseg, step, k->ctl, slotIn, out,
+            if (int r = launch_quiet_plan(k->quiet, k->tspeed, k->nx, k->ny, launch_width(k), step, k->ctl, slotIn, out,
                                           k->tlist, k->tcount, rbSeq, k->stream))
                 return r;
             rbSeq = 0u;
@@ -382,7 +425,7 @@ int pc_fused(swe_hip_block* k, int slotIn, int out, float dtFixed, unsigned rbSe
     }
     if (rbSeq != 0u)
         if (int r = launch_readback(k->ctl, slotIn, rbSeq, k->stream)) return r;
-    if (int r = launch_fused_u(es, k->math, k->xseg, view(k, k->cur), io, k->bi, k->ctl, slotIn, out, (out + 1) % 3,
+    if (int r = launch_fused_u(es, k->math, launch_width(k), view(k, k->cur), io, k->bi, k->ctl, slotIn, out, (out + 1) % 3,
                                nullptr, 0, k->stream))
         return r;
     k->pcStep = step;
@@ -493,6 +536,7 @@ int run_u_device_loop(swe_hip_block* k, int nsteps, float* t_inout, float* dt_lo
         if (int r = ensure_second_sums(k)) return r;
         if (int r = ensure_quiet_record(k)) return r;
     }
+    const int xseg = launch_width(k);
     // the learned middle state's fused loop defers its hard edges to a second launch per step
     const bool defer = k->strategy == 2 && nsteps > 1 && eff_solver(k) == SOLVER_AUGRIE_MLP;
     if (defer)
@@ -508,7 +552,7 @@ int run_u_device_loop(swe_hip_block* k, int nsteps, float* t_inout, float* dt_lo
         for (int slot = 1; slot < 3; ++slot)
             if (int r = launch_ctl_reset(k->ctl, slot, k->stream)) return r;
         if (tm && tm->perKernel) HIP_TRY(tm->mark(k->stream, 1));
-        if (int r = launch_sweep_u(k->solver, k->math, MODE_MAX, k->xseg, view(k, k->cur), sums_view(k), nullptr,
+        if (int r = launch_sweep_u(k->solver, k->math, MODE_MAX, xseg, view(k, k->cur), sums_view(k), nullptr,
                                    nullptr, nullptr, k->bi, k->ctl, Slots{0, 1}, -1.f, 0, nullptr, 0, k->stream))
             return r;
         for (int s = 0; s < nsteps; ++s) {
@@ -527,7 +571,7 @@ int run_u_device_loop(swe_hip_block* k, int nsteps, float* t_inout, float* dt_lo
             if (int r = launch_ctl_reset(k->ctl, slot, k->stream)) return r;
         SumsView set[2] = {sums_view(k), sums2_view(k)};
         if (tm && tm->perKernel) HIP_TRY(tm->mark(k->stream, 1));
-        if (int r = launch_sweep_u(eff_solver(k), k->math, MODE_STORE, k->xseg, view(k, k->cur), set[0], nullptr, nullptr,
+        if (int r = launch_sweep_u(eff_solver(k), k->math, MODE_STORE, xseg, view(k, k->cur), set[0], nullptr, nullptr,
                                    nullptr, k->bi, k->ctl, Slots{0, 1}, -1.f, 0, nullptr, 0, k->stream))
             return r;
         const bool extTimed = tm && tm->perKernel && !defer;
@@ -542,11 +586,11 @@ int run_u_device_loop(swe_hip_block* k, int nsteps, float* t_inout, float* dt_lo
             io.step = s;
             // (only the augmented solver keeps a record, at widths of whole record tiles)
             const int es = defer ? SOLVER_AUGRIE_DEFER : eff_solver(k);
-            const bool record = (es == SOLVER_AUGRIE || es == SOLVER_AUGRIE_DEFER) && k->xseg % kQuietCols == 0;
+            const bool record = (es == SOLVER_AUGRIE || es == SOLVER_AUGRIE_DEFER) && xseg % kQuietCols == 0;
             if (k->skipQuiet && s >= 3 && record) {
                 if (tm && tm->perKernel && !extTimed) HIP_TRY(tm->mark(k->stream, 0));
                 if (tm) ++tm->plans;
-                if (int r = launch_quiet_plan(k->quiet, k->tspeed, k->nx, k->ny, k->xseg, s, k->ctl, (s + 2) % 3, s % 3,
+                if (int r = launch_quiet_plan(k->quiet, k->tspeed, k->nx, k->ny, xseg, s, k->ctl, (s + 2) % 3, s % 3,
                                               k->tlist, k->tcount, 0u, k->stream))
                     return r;
                 io.list = k->tlist;
@@ -559,14 +603,14 @@ int run_u_device_loop(swe_hip_block* k, int nsteps, float* t_inout, float* dt_lo
             }
             if (defer) {
                 io.deferQ = k->deferQ;
-                if (int r = launch_fused_defer(k->xseg, view(k, k->cur), io, k->bi, k->ctl, (s - 1) % 3, s % 3,
+                if (int r = launch_fused_defer(xseg, view(k, k->cur), io, k->bi, k->ctl, (s - 1) % 3, s % 3,
                                                (s + 1) % 3, k->dtlog, s - 1, k->stream))
                     return r;
                 if (int r = launch_defer_solve(view(k, o), set[s & 1], k->ctl, s % 3, k->deferQ, k->deferCap,
                                                deferGroups, k->stream))
                     return r;
             } else {
-                const int r = launch_fused_u(eff_solver(k), k->math, k->xseg, view(k, k->cur), io, k->bi, k->ctl,
+                const int r = launch_fused_u(eff_solver(k), k->math, xseg, view(k, k->cur), io, k->bi, k->ctl,
                                              (s - 1) % 3, s % 3, (s + 1) % 3, k->dtlog, s - 1, k->stream);
                 g_fusedTimer = LaunchTimer{};
                 if (r) return r;
@@ -817,7 +861,8 @@ int swe_hip_create(int nx, int ny, float dx, float dy, float ox, float oy, int s
     k->oy = oy;
     k->solver = solver;
     k->flavour = flavour;
-    k->xseg = default_xseg(nx, ny, solver);
+    k->cus = device_cus();
+    k->xseg = default_xseg(nx, ny, solver, k->cus);
     const size_t bytes = field_elems(k) * sizeof(float);
     hipError_t e = hipSuccess;
     if (e == hipSuccess) e = hipStreamCreateWithFlags(&k->stream, hipStreamNonBlocking);
@@ -1066,7 +1111,7 @@ int swe_hip_fluxes(swe_hip_block* k, float* max_timestep) {
                 k->cur ^= 1;
                 k->pcSums ^= 1;
             } else {
-                if (int r = launch_sweep_u(eff_solver(k), k->math, MODE_STORE, k->xseg, view(k, k->cur), pc_sums(k),
+                if (int r = launch_sweep_u(eff_solver(k), k->math, MODE_STORE, launch_width(k), view(k, k->cur), pc_sums(k),
                                            nullptr, nullptr, nullptr, k->bi, k->ctl, Slots{out, (out + 1) % 3}, -1.f,
                                            0, nullptr, 0, k->stream))
                     return r;
@@ -1573,6 +1618,7 @@ int swe_hip_set_tuning(swe_hip_block* k, int strategy, int xseg) {
     if (xseg != -1) {
         k->xseg = xseg;
         k->xsegSet = true;
+        k->narrowOk = false;
     }
     return SWE_HIP_OK;
 }
@@ -1657,11 +1703,22 @@ int swe_hip_autotune(swe_hip_block* k, int steps, float* ms_per_step) {
     }
     const int widths[SWE_HIP_TUNE_WIDTHS] = {4, 8, 10, 12, 16, 32};
     const int oldXseg = k->xseg;
+    const bool oldNarrowOk = k->narrowOk;
     int best = oldXseg, rc = 0;
     float bestMs = 0.f;
     // one untimed run first (first launches of the process, allocations)
     if (e == hipSuccess) rc = swe_hip_run_timed(k, 2, nullptr, nullptr, nullptr, nullptr);
     if (e == hipSuccess && rc == 0) copy_state(false);
+    // the narrow width of a small block, where the caller has not chosen one
+    bool narrowBest = false;
+    float narrowMs = 0.f;
+    if (e == hipSuccess && rc == 0 && k->narrowOk && launch_width(k) != k->xseg) {
+        rc = swe_hip_run_timed(k, steps, nullptr, &narrowMs, nullptr, nullptr);
+        narrowMs /= steps;
+        narrowBest = rc == 0;
+        if (rc == 0) copy_state(false);
+    }
+    k->narrowOk = false;
     for (int i = 0; i < SWE_HIP_TUNE_WIDTHS && e == hipSuccess && rc == 0; ++i) {
         k->xseg = widths[i];
         float total = 0.f;
@@ -1710,12 +1767,14 @@ int swe_hip_autotune(swe_hip_block* k, int steps, float* ms_per_step) {
     k->cur = cur0;
     if (rc || e != hipSuccess) {
         k->xseg = oldXseg;
+        k->narrowOk = oldNarrowOk;
         k->strategy = oldStrategy;
         return rc ? rc : hip_fail(e, "swe_hip_autotune");
     }
     k->xseg = best;
     k->strategy = bestStrategy;
     k->xsegSet = true;
+    k->narrowOk = narrowBest && narrowMs < bestMs;
     return SWE_HIP_OK;
 }
 
@@ -1748,7 +1807,7 @@ int swe_hip_set_surrogate(swe_hip_block* k, swe_hip_mlp* m) {
         k->net = m;
     }
     k->mlp = frags;
-    if (!k->xsegSet) k->xseg = default_xseg(k->nx, k->ny, frags ? SOLVER_AUGRIE_DEFER : k->solver);
+    if (!k->xsegSet) k->xseg = default_xseg(k->nx, k->ny, frags ? SOLVER_AUGRIE_DEFER : k->solver, k->cus);
     return SWE_HIP_OK;
 }
 
@@ -1866,7 +1925,8 @@ int swe_hip_run_noalloc(int nx, int ny, float dx, float dy, int solver, const in
                   nx, ny, need, (size_t)SWE_HIP_NOALLOC_SCRATCH_BYTES);
         return SWE_HIP_EINVAL;
     }
-    k.xseg = default_xseg(nx, ny, solver);
+    k.cus = device_cus();
+    k.xseg = default_xseg(nx, ny, solver, k.cus);
     unsigned char* base = nullptr;
     if (int r = noalloc_scratch(&base)) return r;
     const size_t field = align256(field_elems(&k) * sizeof(float));
