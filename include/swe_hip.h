@@ -298,8 +298,8 @@ int swe_hip_solve_edges(int solver, int math, int64_t n, const float* hL, const 
  * 16 and 12 for which nyt * ceil(nx/xseg) / (CUs * 4) reaches the solver's
  * threshold (nyt = ceil(ny/62); AugRie 12, 4; with a learned middle state
  * attached 5, 3; HLLE, f-wave, Hybrid 2, 1), else 8 (swe_hip_set_surrogate
- * re-picks it); with strategy 2 a block too small to fill the GPU at that
- * width runs strips of 1, 2 or 4 columns instead (HLLE and f-wave on larger
+ * re-picks it); with strategy 2 a block that does not fill the GPU at that
+ * width runs strips of 1 to 8 columns instead (HLLE and f-wave on larger
  * blocks: their one-pass launch picks 8, 16 or 32).  The fused loop skips quiet tiles (swe_hip_set_quiet_skip)
  * at widths that are multiples of 4. */
 int swe_hip_set_tuning(swe_hip_block* blk, int strategy, int xseg);
@@ -322,7 +322,7 @@ int swe_hip_autotune(swe_hip_block* blk, int steps, float* ms_per_step);
 
 /* Quiet-tile skipping of the fused device loop (strategy 2), on by default,
  * for the augmented solver (AugRie, with or without a learned middle state)
- * at strip widths that are multiples of 4.  A tile of 62 rows x 4 columns
+ * at strip widths that are multiples of 4.  A tile of 62 rows x 2 columns
  * whose net-update sums were all +0 on the last two steps, with the adjacent
  * rows and columns of its four neighbours quiet on the last step, would
  * compute the same zero sums and the same CFL maximum again from an

@@ -63,24 +63,48 @@ namespace swe {
 // the halo a neighbouring tile reads.
 constexpr unsigned kQuietAll = 1u, kQuietBottom = 2u, kQuietTop = 4u, kQuietLeft = 8u, kQuietRight = 16u;
 // Record tiles are kQuietCols columns wide; a wave's segment of XS columns
-// spans XS / kQuietCols of them.
-constexpr int kQuietCols = 4;
+// spans XS / kQuietCols of them.  A launch with few busy tiles lasts as long as
+// one of them, whose columns are a chain of dependent operations.  us per step
+// with tiles of 4 / 2 / 1 columns: 1024^2 islands 33.8 / 26.8 / 24.4, 2048^2 islands
+// from the start 37.0 / 31.1 / 31.7 and from step 400 67 / 55 / 60, 4096^2 trench
+// from the start 35.8 / 32.0 / 35.6 and from step 600 48.7 / 49.3 / 53.9, every cell
+// moving 2048^2 104 / 104 / 108, 4096^2 332 / 341 / 351: one column solves an edge
+// column twice per column and doubles the plan's work.
+constexpr int kQuietCols = 2;
+constexpr int kRecordWidth = 4;  // strip widths with a record are multiples of this
+constexpr int kEntryBits = 4;    // list entry: segment << 2 bits | first tile << bits | tiles - 1
+// Most wave segments of a block whose quiet tiles are skipped (list entries
+// hold the segment in 24 bits).
+constexpr long kMaxSegments = 1l << (32 - 2 * kEntryBits);
 // Waves the quiet-tile plan aims to fill with busy record tiles before it
-// lengthens the pieces it lists: four per SIMD of the chip.  Measured on the
-// 2048^2 islands, the 4096^2 trench and the 4096^2 islands (us per step):
-// 1024: 92.9 / - / -; 2048: 85.6 / 92.4 / 169.4; 3072: 81.3 / 89.2 / 166.9;
-// 4096: 79.7 / 89.0 / 165.6; 5120: 81.0 / 90.3 / 165.0; 6144: 82.5 / 93.3 /
-// 166.1; 8192: 88.3 / - / -.  Shorter pieces give more waves to hide the
-// busy tiles' latency but solve more halo edges.
-constexpr unsigned kPlanWaves = 4096;
+// lengthens the pieces it lists: eight per SIMD of the chip.  Measured with 4096 /
+// 6144 / 8192 (us per step, strips of 8 columns at 2048^2, of 16 at 4096^2): 2048^2
+// islands from step 400 66 / 61 / 54, every cell moving 108 / 104 / 105; 4096^2
+// islands from step 300 105 / 90 / 90, trench from step 600 51 / 49 / 50.  Shorter
+// pieces give more waves to hide the busy tiles' latency but solve more halo
+// edges.
+constexpr unsigned kPlanWaves = 8192;
 
-// Lanes the quiet-tile plan gives a wave segment of `fine` record tiles: the
-// smallest power of two >= fine, so that a segment's lanes share one wave.
-__host__ __device__ constexpr int plan_lanes(int fine) { return fine <= 1 ? 1 : fine <= 2 ? 2 : fine <= 4 ? 4 : 8; }
+// Lanes the quiet-tile plan gives a wave segment of `fine` record tiles (1 to
+// 16): the smallest power of two >= fine, so that a segment's lanes share one
+// wave.
+__host__ __device__ constexpr int plan_lanes(int fine) {
+    int l = 1;
+    while (l < fine) l *= 2;
+    return l;
+}
 // Workgroups of the plan (and entries of its count array) for nyt x nxs
 // segments of `fine` record tiles.
 __host__ __device__ constexpr int plan_groups(int nyt, int nxs, int fine) {
     return (nyt * nxs * plan_lanes(fine) + kPlanGroup - 1) / kPlanGroup;
+}
+
+// Waves of a launch in list mode: one per segment, or twice kPlanWaves where
+// that is more (short pieces of few busy tiles), but no more than record tiles.
+__host__ constexpr int list_waves(int nyt, int nxs, int nx) {
+    const int tiles = nyt * ((nx + kQuietCols - 1) / kQuietCols), some = 2 * (int)kPlanWaves;
+    const int want = nyt * nxs > some ? nyt * nxs : some;
+    return want < tiles ? want : tiles;
 }
 
 // Which fused kernels keep the quiet record: the augmented solver's, exact
@@ -90,7 +114,7 @@ __host__ __device__ constexpr int plan_groups(int nyt, int nxs, int fine) {
 // runs the deferring variant instead), at widths that are whole record tiles.
 template <int S>
 constexpr bool quiet_record(int xs) {
-    return (S == SOLVER_AUGRIE || S == SOLVER_AUGRIE_DEFER) && xs % kQuietCols == 0;
+    return (S == SOLVER_AUGRIE || S == SOLVER_AUGRIE_DEFER) && xs % kRecordWidth == 0;
 }
 
 struct FusedIO {
@@ -110,7 +134,7 @@ struct FusedIO {
     float* speed = nullptr;
     int step = 0;  // launch index within the run (1, 2, ...)
     // list mode: workgroup g of the plan lists count[g] runs of record tiles
-    // to compute at list[g * kPlanGroup * kPlanPieces ...]
+    // to compute at list[g * kPlanGroup ...]
     const unsigned* list = nullptr;
     const unsigned* count = nullptr;
     // >= 0: the previous update's dt, given by the caller (the per-call
@@ -118,29 +142,38 @@ struct FusedIO {
     float dtFixed = -1.f;
 };
 
-// The list entry of wave w in list mode, or -1 past the last listed entry: a
-// wave scan over the group counts finds the group holding the w-th entry.
-__device__ __forceinline__ int listed_item(const FusedIO& io, int groups, int w) {
+// The w-th list entry, or kNoEntry past the last one.  Each lane takes four
+// group counts (a block of 4096 x 4096 has 134 groups), a scan over the wave
+// finds the lane whose groups hold the entry, and the rest is scalar.
+constexpr unsigned kNoEntry = 0xffffffffu;  // no entry: first tile + tiles - 1 < tiles per segment
+__device__ __forceinline__ unsigned listed_item(const FusedIO& io, int groups, int w) {
     const int lane = threadIdx.x & 63;
-    for (int base = 0; base < groups; base += 64) {  // uniform per wave
-        const unsigned c = (base + lane < groups) ? io.count[base + lane] : 0u;
-        unsigned incl = c;
+    for (int base = 0; base < groups; base += 256) {  // uniform per wave
+        unsigned c[4], sum = 0u;
 #pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-            const unsigned o = __shfl_up(incl, off, 64);
-            incl += (lane >= off) ? o : 0u;
+        for (int i = 0; i < 4; ++i) {
+            const int g = base + 4 * lane + i;
+            c[i] = g < groups ? io.count[g] : 0u;
+            sum += c[i];
         }
-        const unsigned total = __shfl(incl, 63, 64);
+        const unsigned incl = wave_scan(sum);
+        const unsigned total = (unsigned)__builtin_amdgcn_readlane((int)incl, 63);
         if ((unsigned)w < total) {
-            const unsigned long long m = __ballot(incl > (unsigned)w);
-            const int g = __builtin_ctzll(m);
-            const unsigned excl = __shfl(incl - c, g, 64);
-            return (int)__builtin_amdgcn_readfirstlane(
-                io.list[(size_t)(base + g) * kPlanGroup * kPlanPieces + (w - excl)]);
+            const int l = __builtin_ctzll(__ballot(incl > (unsigned)w));
+            int g = base + 4 * l;
+            unsigned at = (unsigned)w - (unsigned)__builtin_amdgcn_readlane((int)(incl - sum), l);
+#pragma unroll
+            for (int i = 0; i < 3; ++i) {
+                const unsigned ci = (unsigned)__builtin_amdgcn_readlane((int)c[i], l);
+                if (at < ci) break;
+                at -= ci;
+                ++g;
+            }
+            return io.list[(size_t)g * kPlanGroup + at];
         }
         w -= (int)total;
     }
-    return -1;
+    return kNoEntry;
 }
 
 struct Q3 {
@@ -159,219 +192,228 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(fused_waves
     const int nx = v.nx, ny = v.ny;
 
     const float dt = io.dtFixed >= 0.f ? io.dtFixed : timestep_from_max(ctl->smax[slotIn].value(), v.dx, v.dy);
-    if (blockIdx.x == 0) ctl->smax[slotClear].clear();
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        ctl->defer[slotClear] = 0u;
-        ctl->busy[slotClear] = 0u;
-        ctl->dt = dt;
-        ctl->t += dt;
-        ctl->steps += 1;
-        if (dtLog) dtLog[logIdx] = dt;
+    if (blockIdx.x == 0) {
+        ctl->smax[slotClear].clear();
+        if (threadIdx.x == 0) {
+            ctl->defer[slotClear] = 0u;
+            ctl->busy[slotClear] = 0u;
+            ctl->dt = dt;
+            ctl->t += dt;
+            ctl->steps += 1;
+            if (dtLog) dtLog[logIdx] = dt;
+        }
     }
     constexpr bool kRecord = quiet_record<S>(XS);
     const int items = nyt * nxs;
-    int item = wave, first = 0, ncols = XS;
-    if (kRecord && io.list) {
-        const int e = __builtin_amdgcn_readfirstlane(listed_item(io, plan_groups(nyt, nxs, XS / kQuietCols), wave));
-        if (e < 0) return;  // uniform per wave
-        item = e >> 6;
-        first = (e >> 3) & 7;
-        ncols = ((e & 7) + 1) * kQuietCols;
-    }
-    if (item >= items) return;  // uniform per wave
-    const int yt = item % nyt;
-    const int xs = item / nyt;
-    const int slotNow = (io.step & 1) * nyt * ((nx + kQuietCols - 1) / kQuietCols);
-    const dev::SolverCtx<S> solver(S == SOLVER_AUGRIE_MLP ? ctl->mlp : nullptr);
-
-    const float dtdx = dt / v.dx;
-    const float dtdy = dt / v.dy;
-    const int x0 = 1 + xs * XS + first * kQuietCols;
-    const int x1 = min(x0 + ncols - 1, nx);
-    const int tB = bi.type[BND_BOTTOM], tT = bi.type[BND_TOP], tL = bi.type[BND_LEFT], tR = bi.type[BND_RIGHT];
-
-    auto tile = [&](auto form, int lane) -> bool {
-        constexpr bool N = decltype(form)::value;
-        using A = CellMath<N>;
-        const int y = kStripRows * yt + lane;
-        const bool rowValid = y <= ny + 1;
-        const int yc = rowValid ? y : ny + 1;
-        const bool owned = (lane >= 1) && (lane <= kStripRows) && (y <= ny);
-        const bool rowInterior = (y >= 1) && (y <= ny);
-        const bool hEdgeValid = (lane <= kStripRows) && (y <= ny);
-        const bool rowBottom = (y == 0);
-        const bool rowTop = (y == ny + 1);
-        const bool carryRow = owned || (rowBottom && lane == 0) || (rowTop && lane >= 1);
-
-        // Q(k) of the cell (x, yc): interior cells updated, ghosts as stored
-        auto load_updated = [&](int x) -> Q3 {
-            const size_t c = (size_t)x * v.pitch;
-            const unsigned rc = lane_bytes(yc);
-            Q3 q{col_get(io.h, c, rc), col_get(io.hu, c, rc), col_get(io.hv, c, rc)};
-            if (x >= 1 && x <= nx && rowInterior) {
-                const Cell u = update_cell(q.h, q.hu, q.hv, dtdx, dtdy, col_get(io.sIn.sx, c, rc), col_get(io.sIn.sy, c, rc),
-                                           col_get(io.sIn.su, c, rc), col_get(io.sIn.sv, c, rc));
-                q = Q3{u.h, u.hu, u.hv};
-            }
-            return q;
-        };
-        // ghost rows of an interior column: the boundary value of the row next to
-        // it (lane+1 for the bottom row, lane-1 for the top row)
-        auto fix_rows = [&](Q3 q) -> Q3 {
-            const float dh = __shfl_down(q.h, 1, 64), dhu = __shfl_down(q.hu, 1, 64), dhv = __shfl_down(q.hv, 1, 64);
-            const float uh = __shfl_up(q.h, 1, 64), uhu = __shfl_up(q.hu, 1, 64), uhv = __shfl_up(q.hv, 1, 64);
-            if (rowBottom && is_ow(tB)) q = Q3{dh, dhu, (tB == WALL) ? -dhv : dhv};
-            if (rowTop && is_ow(tT)) q = Q3{uh, uhu, (tT == WALL) ? -uhv : uhv};
-            return q;
-        };
-        // a ghost column next to the interior column value `in` (same lane);
-        // corners take the diagonal interior cell (from the neighbouring lane)
-        auto fix_column = [&](Q3 raw, Q3 in, int type) -> Q3 {
-            const float dh = __shfl_down(in.h, 1, 64), dhu = __shfl_down(in.hu, 1, 64), dhv = __shfl_down(in.hv, 1, 64);
-            const float uh = __shfl_up(in.h, 1, 64), uhu = __shfl_up(in.hu, 1, 64), uhv = __shfl_up(in.hv, 1, 64);
-            Q3 q = raw;
-            if (rowInterior && is_ow(type)) q = Q3{in.h, (type == WALL) ? -in.hu : in.hu, in.hv};
-            if (rowBottom) q = Q3{dh, dhu, dhv};
-            if (rowTop) q = Q3{uh, uhu, uhv};
-            return q;
-        };
-        auto store = [&](int x, const Q3& q) {
-            const size_t c = (size_t)x * v.pitch;
-            const unsigned ry = lane_bytes(y);
-            col_set(io.hn, c, ry, q.h);
-            col_set(io.hun, c, ry, q.hu);
-            col_set(io.hvn, c, ry, q.hv);
-        };
-
-        const float* B = v.b;
-        // columns x0-1 and x0
-        Q3 cur = fix_rows(load_updated(x0));
-        Q3 prev = load_updated(x0 - 1);
-        if (x0 == 1) prev = fix_column(prev, cur, tL);
-        if (x0 == 1 && carryRow) store(0, prev);
-        float cb = col_get(B, (size_t)(x0 - 1) * v.pitch, lane_bytes(yc));
-        float nb = col_get(B, (size_t)x0 * v.pitch, lane_bytes(yc));
-
-        const CellQ pq = cell_q<A>(prev.h, prev.hu, prev.hv, cb);
-        CellQ cq = cell_q<A>(cur.h, cur.hu, cur.hv, nb);
-        bool outside = outside_range<N>(pq) || outside_range<N>(cq);
-        dev::EdgeOut e = solver.template solve<A>(pq.xside(), cq.xside());
-        // record tile of the columns being solved: a deferred edge touching it
-        // makes it not quiet; the halo edge (x0-1 | x0) counts for the first
-        bool loud = false;
-        if constexpr (S == SOLVER_AUGRIE_DEFER) {
-            loud = e.speed < 0.f;
-            e = defer_edge(e, owned && x0 == 1, make_uint2(0u, (unsigned)y), io.deferQ, &ctl->defer[slotOut]);
+    // list mode: entry after entry until the list ends (the grid covers the
+    // usual lists once)
+    for (int w = wave;; w += gridDim.x * kWavesPerGroup) {
+        int item = w, first = 0, ncols = XS;
+        if (kRecord && io.list) {
+            const unsigned e =
+                __builtin_amdgcn_readfirstlane(listed_item(io, plan_groups(nyt, nxs, XS / kQuietCols), w));
+            if (e == kNoEntry) return;  // uniform per wave
+            constexpr unsigned mask = (1u << kEntryBits) - 1u;
+            item = (int)(e >> (2 * kEntryBits));
+            first = (int)((e >> kEntryBits) & mask);
+            ncols = (int)((e & mask) + 1u) * kQuietCols;
         }
-        float carryH = e.hR, carryHu = e.huR;
-        // x-edges count on owned rows (each interior row is owned by one strip),
-        // so a record tile's maximum depends on its footprint only
-        float smaxTile = owned ? e.speed : 0.f;
-        // the segment's maximum over its record tiles, wave-uniform (float bits:
-        // non-negative floats order like unsigned integers)
-        unsigned smaxRun = 0u;
-        // kQuiet* bits of the record tile's parts whose owned sums were not all +0
-        unsigned loudParts = 0u;
+        if (item >= items) return;  // uniform per wave
+        const int yt = item % nyt;
+        const int xs = item / nyt;
+        const int slotNow = (io.step & 1) * nyt * ((nx + kQuietCols - 1) / kQuietCols);
+        const dev::SolverCtx<S> solver(S == SOLVER_AUGRIE_MLP ? ctl->mlp : nullptr);
 
-        // Column x+1's loads are issued one column ahead (a software pipeline):
-        // their latency overlaps column x's edges.  The loads past x1 + 1 read
-        // column nx + 1 at most and are not used.  Not for the learned middle
-        // state: its network call and the deferring sweep's seven waves leave
-        // no registers for them.
-        struct Raw {
-            float h, hu, hv, sx, sy, su, sv, b;
-        };
-        auto load_raw = [&](int x) -> Raw {
-            const size_t c = (size_t)min(x, nx + 1) * v.pitch;
-            const unsigned rc = lane_bytes(yc);
-            return Raw{col_get(io.h, c, rc),      col_get(io.hu, c, rc),     col_get(io.hv, c, rc),     col_get(io.sIn.sx, c, rc),
-                       col_get(io.sIn.sy, c, rc), col_get(io.sIn.su, c, rc), col_get(io.sIn.sv, c, rc), col_get(B, c, rc)};
-        };
-        constexpr bool kAhead = S != SOLVER_AUGRIE_MLP && S != SOLVER_AUGRIE_DEFER;
-        Raw ahead{};
-        if constexpr (kAhead) ahead = load_raw(x0 + 1);
-        for (int x = x0; x <= x1; ++x) {
-            // column x+1 of Q(k)
-            const Raw r = kAhead ? ahead : load_raw(x + 1);
-            if constexpr (kAhead) ahead = load_raw(x + 2);
-            Q3 nxt{r.h, r.hu, r.hv};
-            if (x + 1 <= nx && rowInterior) {
-                const Cell u = update_cell(nxt.h, nxt.hu, nxt.hv, dtdx, dtdy, r.sx, r.sy, r.su, r.sv);
-                nxt = Q3{u.h, u.hu, u.hv};
-            }
-            nxt = fix_rows(nxt);
-            if (x + 1 == nx + 1) nxt = fix_column(nxt, cur, tR);
-            const CellQ nq = cell_q<A>(nxt.h, nxt.hu, nxt.hv, r.b);
-            outside = outside || outside_range<N>(nq);
+        const float dtdx = dt / v.dx;
+        const float dtdy = dt / v.dy;
+        const int x0 = 1 + xs * XS + first * kQuietCols;
+        const int x1 = min(x0 + ncols - 1, nx);
+        const bool ghostRows = yt == 0 || kStripRows * yt + 63 >= ny + 1;  // the strip holds a ghost row
+        const int tB = bi.type[BND_BOTTOM], tT = bi.type[BND_TOP], tL = bi.type[BND_LEFT], tR = bi.type[BND_RIGHT];
 
-            if (carryRow) store(x, cur);
-            if (x + 1 == nx + 1 && carryRow) store(nx + 1, nxt);
+        auto tile = [&](auto form, int lane) -> bool {
+            constexpr bool N = decltype(form)::value;
+            using A = CellMath<N>;
+            const int y = kStripRows * yt + lane;
+            const bool rowValid = y <= ny + 1;
+            const int yc = rowValid ? y : ny + 1;
+            const bool owned = (lane >= 1) && (lane <= kStripRows) && (y <= ny);
+            const bool rowInterior = (y >= 1) && (y <= ny);
+            const bool hEdgeValid = (lane <= kStripRows) && (y <= ny);
+            const bool rowBottom = (y == 0);
+            const bool rowTop = (y == ny + 1);
+            const bool carryRow = owned || (rowBottom && lane == 0) || (rowTop && lane >= 1);
 
-            dev::EdgeOut ev = solver.template solve<A>(cq.xside(), nq.xside());
-            bool loudEdge = false;
-            if constexpr (S == SOLVER_AUGRIE_DEFER) {
-                loudEdge = ev.speed < 0.f;
-                ev = defer_edge(ev, owned, make_uint2((unsigned)x, (unsigned)y), io.deferQ, &ctl->defer[slotOut]);
-            }
-            if (owned) smaxTile = dev::smax(smaxTile, ev.speed);
-            dev::EdgeOut eh = solver.template solve<A>(cq.yside(), cq.yside_from_lane_above());
-            if constexpr (S == SOLVER_AUGRIE_DEFER) {
-                loud = loud || loudEdge || eh.speed < 0.f;
-                eh = defer_edge(eh, owned || y == 0, make_uint2((unsigned)x | kDeferY, (unsigned)y), io.deferQ,
-                                &ctl->defer[slotOut]);
-            }
-            if (hEdgeValid) smaxTile = dev::smax(smaxTile, eh.speed);
-            const float aH = __shfl_up(eh.hR, 1, 64);
-            const float aHv = __shfl_up(eh.huR, 1, 64);
-            if (owned) {
+            // a column as stored: Q(k-1), S(k-1) and the bed (column nx + 1 at most)
+            struct Raw {
+                float h, hu, hv, sx, sy, su, sv, b;
+            };
+            auto load_raw = [&](int x) -> Raw {
+                const size_t c = (size_t)min(x, nx + 1) * v.pitch;
+                const unsigned rc = lane_bytes(yc);
+                return Raw{col_get(io.h, c, rc),      col_get(io.hu, c, rc),     col_get(io.hv, c, rc),
+                           col_get(io.sIn.sx, c, rc), col_get(io.sIn.sy, c, rc), col_get(io.sIn.su, c, rc),
+                           col_get(io.sIn.sv, c, rc), col_get(v.b, c, rc)};
+            };
+            // Q(k) of its cells: interior cells updated, ghosts as stored
+            auto updated = [&](const Raw& r, int x) -> Q3 {
+                Q3 q{r.h, r.hu, r.hv};
+                if (x >= 1 && x <= nx && rowInterior) {
+                    const Cell u = update_cell(q.h, q.hu, q.hv, dtdx, dtdy, r.sx, r.sy, r.su, r.sv);
+                    q = Q3{u.h, u.hu, u.hv};
+                }
+                return q;
+            };
+            // ghost rows of an interior column: the boundary value of the row next to
+            // it (lane+1 for the bottom row, lane-1 for the top row)
+            auto fix_rows = [&](Q3 q) -> Q3 {
+                if (!ghostRows) return q;
+                const float dh = __shfl_down(q.h, 1, 64), dhu = __shfl_down(q.hu, 1, 64), dhv = __shfl_down(q.hv, 1, 64);
+                const float uh = __shfl_up(q.h, 1, 64), uhu = __shfl_up(q.hu, 1, 64), uhv = __shfl_up(q.hv, 1, 64);
+                if (rowBottom && is_ow(tB)) q = Q3{dh, dhu, (tB == WALL) ? -dhv : dhv};
+                if (rowTop && is_ow(tT)) q = Q3{uh, uhu, (tT == WALL) ? -uhv : uhv};
+                return q;
+            };
+            // a ghost column next to the interior column value `in` (same lane);
+            // corners take the diagonal interior cell (from the neighbouring lane)
+            auto fix_column = [&](Q3 raw, Q3 in, int type) -> Q3 {
+                const float dh = __shfl_down(in.h, 1, 64), dhu = __shfl_down(in.hu, 1, 64), dhv = __shfl_down(in.hv, 1, 64);
+                const float uh = __shfl_up(in.h, 1, 64), uhu = __shfl_up(in.hu, 1, 64), uhv = __shfl_up(in.hv, 1, 64);
+                Q3 q = raw;
+                if (rowInterior && is_ow(type)) q = Q3{in.h, (type == WALL) ? -in.hu : in.hu, in.hv};
+                if (rowBottom) q = Q3{dh, dhu, dhv};
+                if (rowTop) q = Q3{uh, uhu, uhv};
+                return q;
+            };
+            auto store = [&](int x, const Q3& q) {
                 const size_t c = (size_t)x * v.pitch;
                 const unsigned ry = lane_bytes(y);
-                const float sx = carryH + ev.hL, su = carryHu + ev.huL, sy = aH + eh.hL, sv = aHv + eh.huL;
-                col_set(io.sOut.sx, c, ry, sx);
-                col_set(io.sOut.su, c, ry, su);
-                col_set(io.sOut.sy, c, ry, sy);
-                col_set(io.sOut.sv, c, ry, sv);
-                if constexpr (kRecord)
-                    if ((__float_as_uint(sx) | __float_as_uint(su) | __float_as_uint(sy) | __float_as_uint(sv)) != 0u)
-                        loudParts |= kQuietAll | (lane == 1 ? kQuietBottom : 0u) | (lane == kStripRows ? kQuietTop : 0u) |
-                                     (((x - 1) & (kQuietCols - 1)) == 0 ? kQuietLeft : 0u) |
-                                     ((x & (kQuietCols - 1)) == 0 || x == nx ? kQuietRight : 0u);
-            }
-            carryH = ev.hR;
-            carryHu = ev.huR;
-            cur = nxt;
-            cq = nq;
-            // the end of a record tile: its parts' flags and its maximum.  A tile
-            // reports its right edge (x | x+1) and, first in a run, its left halo
-            // edge; the tile of column 1 always starts a run, so every x-edge is
-            // in some record, and each record's edges lie in its tile's footprint.
-            // A deferred edge at the boundary touches both tiles.
-            if (kRecord && ((x & (kQuietCols - 1)) == 0 || x == x1)) {  // uniform per wave
-                const float tileMax = wave_max<N>(smaxTile);
-                smaxRun = max(smaxRun, __builtin_amdgcn_readfirstlane(__float_as_uint(tileMax)));
-                if (io.quiet) {
-                    unsigned quiet = 0u;
-    #pragma unroll
-                    for (unsigned part = 1u; part <= kQuietRight; part <<= 1)
-                        if (!__any((loudParts & part) != 0u || loud)) quiet |= part;
-                    if (lane == 0) {
-                        const int rec = slotNow + yt + nyt * ((x - 1) / kQuietCols);
-                        io.quiet[rec] = quiet;
-                        io.speed[rec] = tileMax;
-                    }
-                }
-                smaxTile = 0.f;
-                loud = loudEdge;
-                loudParts = 0u;
-            }
-        }
+                col_set(io.hn, c, ry, q.h);
+                col_set(io.hun, c, ry, q.hu);
+                col_set(io.hvn, c, ry, q.hv);
+            };
 
-        if (N && __any(outside)) return false;
-        if constexpr (!kRecord) smaxRun = __float_as_uint(wave_max<N>(smaxTile));
-        if (lane == 0) raise_max(ctl->smax[slotOut], smaxRun);
-        return true;
-    };
-    run_tile<dev::SolverCtx<S>, V>(threadIdx.x & 63, tile);
+            // columns x0-1, x0 and (a software pipeline) x0+1: every load at once.
+            // The learned middle state loads column by column: its network call and
+            // the deferring sweep's seven waves leave no registers to load ahead.
+            constexpr bool kAhead = S != SOLVER_AUGRIE_MLP && S != SOLVER_AUGRIE_DEFER;
+            const Raw r0 = load_raw(x0 - 1), r1 = load_raw(x0);
+            Raw ahead{};
+            if constexpr (kAhead) ahead = load_raw(x0 + 1);
+            Q3 cur = fix_rows(updated(r1, x0));
+            Q3 prev = updated(r0, x0 - 1);
+            if (x0 == 1) prev = fix_column(prev, cur, tL);
+            if (x0 == 1 && carryRow) store(0, prev);
+
+            const CellQ pq = cell_q<A>(prev.h, prev.hu, prev.hv, r0.b);
+            CellQ cq = cell_q<A>(cur.h, cur.hu, cur.hv, r1.b);
+            bool outside = outside_range<N>(pq) || outside_range<N>(cq);
+            dev::EdgeOut e = solver.template solve<A>(pq.xside(), cq.xside());
+            // record tile of the columns being solved: a deferred edge touching it
+            // makes it not quiet; the halo edge (x0-1 | x0) counts for the first
+            bool loud = false;
+            if constexpr (S == SOLVER_AUGRIE_DEFER) {
+                loud = e.speed < 0.f;
+                e = defer_edge(e, owned && x0 == 1, make_uint2(0u, (unsigned)y), io.deferQ, &ctl->defer[slotOut]);
+            }
+            float carryH = e.hR, carryHu = e.huR;
+            // The x- and the y-edges' maxima of this lane's row in the record tile.
+            // x-edges count on owned rows (each interior row is owned by one strip),
+            // so a record tile's maximum depends on its footprint only; which lanes
+            // count is the same in every column, so they are masked at the tile's end.
+            float smaxX = e.speed, smaxY = 0.f;
+            auto tile_max = [&] {
+                return wave_max<N>(dev::smax(owned ? smaxX : 0.f, hEdgeValid ? smaxY : 0.f));
+            };
+            // the segment's maximum over its record tiles, wave-uniform (float bits:
+            // non-negative floats order like unsigned integers)
+            unsigned smaxRun = 0u;
+            // lanes whose owned sums were not all +0 in some column of the record
+            // tile, and in its first and last column
+            unsigned long long loudAll = 0u, loudFirst = 0u, loudLast = 0u;
+
+            for (int x = x0; x <= x1; ++x) {
+                // column x+1 of Q(k); the loads of the next one overlap this one's edges
+                const Raw r = kAhead ? ahead : load_raw(x + 1);
+                if constexpr (kAhead) ahead = load_raw(x + 2);
+                Q3 nxt = fix_rows(updated(r, x + 1));
+                if (x + 1 == nx + 1) nxt = fix_column(nxt, cur, tR);
+                const CellQ nq = cell_q<A>(nxt.h, nxt.hu, nxt.hv, r.b);
+                outside = outside || outside_range<N>(nq);
+
+                if (carryRow) store(x, cur);
+                if (x + 1 == nx + 1 && carryRow) store(nx + 1, nxt);
+
+                dev::EdgeOut ev = solver.template solve<A>(cq.xside(), nq.xside());
+                bool loudEdge = false;
+                if constexpr (S == SOLVER_AUGRIE_DEFER) {
+                    loudEdge = ev.speed < 0.f;
+                    ev = defer_edge(ev, owned, make_uint2((unsigned)x, (unsigned)y), io.deferQ, &ctl->defer[slotOut]);
+                }
+                smaxX = A::max(smaxX, ev.speed);
+                dev::EdgeOut eh = solver.template solve<A>(cq.yside(), cq.yside_from_lane_above());
+                if constexpr (S == SOLVER_AUGRIE_DEFER) {
+                    loud = loud || loudEdge || eh.speed < 0.f;
+                    eh = defer_edge(eh, owned || y == 0, make_uint2((unsigned)x | kDeferY, (unsigned)y), io.deferQ,
+                                    &ctl->defer[slotOut]);
+                }
+                smaxY = A::max(smaxY, eh.speed);
+                const float aH = __shfl_up(eh.hR, 1, 64);
+                const float aHv = __shfl_up(eh.huR, 1, 64);
+                const float sx = carryH + ev.hL, su = carryHu + ev.huL, sy = aH + eh.hL, sv = aHv + eh.huL;
+                if (owned) {
+                    const size_t c = (size_t)x * v.pitch;
+                    const unsigned ry = lane_bytes(y);
+                    col_set(io.sOut.sx, c, ry, sx);
+                    col_set(io.sOut.su, c, ry, su);
+                    col_set(io.sOut.sy, c, ry, sy);
+                    col_set(io.sOut.sv, c, ry, sv);
+                }
+                if constexpr (kRecord) {
+                    const bool nonzero =
+                        (__float_as_uint(sx) | __float_as_uint(su) | __float_as_uint(sy) | __float_as_uint(sv)) != 0u;
+                    loudLast = __ballot(owned && nonzero);
+                    loudAll |= loudLast;
+                    if (((x - 1) & (kQuietCols - 1)) == 0) loudFirst = loudLast;
+                }
+                carryH = ev.hR;
+                carryHu = ev.huR;
+                cur = nxt;
+                cq = nq;
+                // the end of a record tile: its parts' flags and its maximum.  A tile
+                // reports its right edge (x | x+1) and, first in a run, its left halo
+                // edge; the tile of column 1 always starts a run, so every x-edge is
+                // in some record, and each record's edges lie in its tile's footprint.
+                // A deferred edge at the boundary touches both tiles.
+                if (kRecord && ((x & (kQuietCols - 1)) == 0 || x == x1)) {  // uniform per wave
+                    const float tileMax = tile_max();
+                    smaxRun = max(smaxRun, __builtin_amdgcn_readfirstlane(__float_as_uint(tileMax)));
+                    if (io.quiet) {
+                        unsigned quiet = (loudAll == 0u ? kQuietAll : 0u) |
+                                         ((loudAll >> 1 & 1u) == 0u ? kQuietBottom : 0u) |
+                                         ((loudAll >> kStripRows & 1u) == 0u ? kQuietTop : 0u) |
+                                         (loudFirst == 0u ? kQuietLeft : 0u) | (loudLast == 0u ? kQuietRight : 0u);
+                        if (__any(loud)) quiet = 0u;
+                        if (lane == 0) {
+                            const int rec = slotNow + yt + nyt * ((x - 1) / kQuietCols);
+                            io.quiet[rec] = quiet;
+                            io.speed[rec] = tileMax;
+                        }
+                    }
+                    smaxX = smaxY = 0.f;
+                    loud = loudEdge;
+                    loudAll = loudFirst = 0u;
+                }
+            }
+
+            if (N && __any(outside)) return false;
+            if constexpr (!kRecord) smaxRun = __float_as_uint(tile_max());
+            if (lane == 0) raise_max(ctl->smax[slotOut], smaxRun);
+            return true;
+        };
+        run_tile<dev::SolverCtx<S>, V>(threadIdx.x & 63, tile);
+        if (!(kRecord && io.list)) return;
+    }
 }
 
 }  // namespace swe

@@ -42,7 +42,6 @@ enum SweepMode : int { MODE_MAX = 0, MODE_STORE = 1, MODE_UPDATE = 2 };
 constexpr int kStripRows = 62;  // owned rows per wavefront
 constexpr int kWavesPerGroup = 4;
 constexpr int kPlanGroup = 1024;  // wave segments per workgroup of the quiet-tile plan
-constexpr int kPlanPieces = 8;    // list entries per segment at most (32 columns in runs of 4)
 
 // ---- strip tiles of the batched engine --------------------------------------
 // The strips of kStripRows rows below a block's last strip are cut into
@@ -259,6 +258,20 @@ __device__ __forceinline__ float wave_max(float v) {
         for (int off = 32; off >= 1; off >>= 1) v = dev::smax(v, __shfl_xor(v, off, 64));
         return v;
     }
+}
+
+// Inclusive sums over the wave's lanes, by data-parallel-primitive moves.
+template <int Ctrl, int RowMask>
+__device__ __forceinline__ unsigned dpp_add_step(unsigned v) {
+    return v + (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, Ctrl, RowMask, 0xf, false);
+}
+__device__ __forceinline__ unsigned wave_scan(unsigned v) {
+    v = dpp_add_step<0x111, 0xf>(v);  // row_shr:1, 2, 4, 8
+    v = dpp_add_step<0x112, 0xf>(v);
+    v = dpp_add_step<0x114, 0xf>(v);
+    v = dpp_add_step<0x118, 0xf>(v);
+    v = dpp_add_step<0x142, 0xa>(v);  // row_bcast:15 into rows 1 and 3
+    return dpp_add_step<0x143, 0xc>(v);  // row_bcast:31 into rows 2 and 3
 }
 
 // Raise a maximum of the running launch (float bits of a non-negative number)

@@ -81,7 +81,7 @@ __global__ void apply_bc_bathymetry_kernel(float* b, int nx, int ny, int pitch, 
 // slotOut.  The record tiles of a segment from its first to its last busy
 // one are listed in pieces of at most `piece` tiles,
 // (segment << 6) | (first << 3) | (length - 1); workgroup g keeps its
-// entries in segment order at list[g * kPlanGroup * kPlanPieces ...] and
+// entries in segment order at list[g * kPlanGroup ...] and
 // their number in count[g].  piece adapts to the load: busy tiles found by
 // the previous launch's plan over kPlanWaves, between 1 and `fine` (with few
 // busy tiles short pieces spread them over more waves, the busiest wave sets
@@ -137,12 +137,7 @@ __global__ __launch_bounds__(kPlanGroup) void quiet_plan_kernel(const unsigned* 
     const int runLen = leader ? 32 - __builtin_clz(segBits) - firstBusy : 0;
     const unsigned pieces = (unsigned)((runLen + piece - 1) / piece);
     // exclusive prefix of the pieces over the wave, then over the workgroup
-    unsigned incl = pieces;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-        const unsigned o = __shfl_up(incl, off, 64);
-        incl += (lane >= off) ? o : 0u;
-    }
+    const unsigned incl = wave_scan(pieces);
     sp = wave_max(sp);
     if (lane == 63) wavePieces[w] = incl;
     if (lane == 0) {
@@ -158,11 +153,11 @@ __global__ __launch_bounds__(kPlanGroup) void quiet_plan_kernel(const unsigned* 
         nbusy += waveBusy[k];
         mx = max(mx, waveMax[k]);
     }
-    const unsigned pos = (unsigned)blockIdx.x * kPlanGroup * kPlanPieces + before + incl - pieces;
+    const unsigned pos = (unsigned)blockIdx.x * kPlanGroup + before + incl - pieces;
     for (unsigned p = 0; p < pieces; ++p) {
         const int f0 = firstBusy + (int)p * piece;
         const int len = min(piece, runLen - (int)p * piece);
-        list[pos + p] = ((unsigned)seg << 6) | ((unsigned)f0 << 3) | (unsigned)(len - 1);
+        list[pos + p] = ((unsigned)seg << (2 * kEntryBits)) | ((unsigned)f0 << kEntryBits) | (unsigned)(len - 1);
     }
     if (threadIdx.x == 0) {
         count[blockIdx.x] = total;

@@ -67,8 +67,7 @@ int launch_fused_defer(int xseg, StateView v, FusedIO io, BoundaryInfo bi, Devic
     auto go = [&](auto xsTag) {
         constexpr int XS = decltype(xsTag)::value;
         const int nxs = (v.nx + XS - 1) / XS;
-        // list mode may list up to one piece per record tile
-        const int waves = io.list ? nyt * ((v.nx + kQuietCols - 1) / kQuietCols) : nyt * nxs;
+        const int waves = io.list ? list_waves(nyt, nxs, v.nx) : nyt * nxs;
         const int groups = (waves + kWavesPerGroup - 1) / kWavesPerGroup;
         hipLaunchKernelGGL((fused_u_kernel<SOLVER_AUGRIE_DEFER, XS, 0>), dim3(groups), dim3(64 * kWavesPerGroup), 0,
                            stream, v, io, bi, ctl, slotIn, slotOut, slotClear, dtLog, logIdx);

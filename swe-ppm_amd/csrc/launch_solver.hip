@@ -101,8 +101,7 @@ int launch_fused_u_solver(int xseg, StateView v, FusedIO io, BoundaryInfo bi, De
     auto go = [&](auto xsTag) {
         constexpr int XS = decltype(xsTag)::value;
         const int nxs = (v.nx + XS - 1) / XS;
-        // list mode may list up to one piece per record tile
-        const int waves = io.list ? nyt * ((v.nx + kQuietCols - 1) / kQuietCols) : nyt * nxs;
+        const int waves = io.list ? list_waves(nyt, nxs, v.nx) : nyt * nxs;
         const int groups = (waves + kWavesPerGroup - 1) / kWavesPerGroup;
         if (g_fusedTimer.start) {
             hipExtLaunchKernelGGL((fused_u_kernel<S, XS, V>), dim3(groups), dim3(64 * kWavesPerGroup), 0, stream,

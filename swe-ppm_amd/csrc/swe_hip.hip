@@ -207,8 +207,8 @@ int advance_width(const swe_hip_block* k) {
     return 8;
 }
 
-// Strip width of the fused strategy on a block that does not fill the GPU at
-// default_xseg's widths, or 0.  One wave's columns are a chain of dependent
+// Strip width of the fused strategy where a narrower one than default_xseg's
+// pays, or 0.  One wave's columns are a chain of dependent
 // operations, about 1 us per column for the light solvers and 3 for the
 // augmented one, so a launch of few waves lasts as long as its widest strip;
 // once a SIMD has a few waves the halo column per strip costs more than
@@ -219,24 +219,25 @@ int advance_width(const swe_hip_block* k) {
 //   Hybrid 64x50    13.9 / 16.9 / 21.6 / 25.1     256^2   18.3 / 20.4 / 31.6 / 47.6
 //          512^2    27.0 / 24.5 / 34.4 / 53.7     1500x901 47.3 / 48.9 / 45.2 / 54.6
 //          2048^2   90.8 / 80.3 / 77.9 / 79.7     4096^2   341 / 306 / 274 / 280
-//   AugRie 64x50    11.9 / 16.2 / 27.6 / 28.3     256^2   15.5 / 17.6 / 31.1 / 32.2
-//          512^2    26.7 / 21.2 / 32.8 / 33.7     1000x500 36.0 / 29.8 / 33.2 / 34.0
-//          1024^2   42.3 / 42.2 / 33.8 / 34.4
-// (AugRie's 4 and 8 columns record and skip quiet tiles, which the narrower
-// ones do not: there a lake at rest is solved edge by edge, and on larger
-// blocks that costs more.)
+//   AugRie, islands and (after the bar) every cell moving
+//          64x50    11.4 / 15.7 / 21.6 / 21.7     256^2   12.5 / 16.9 / 23.3 / 24.1 | 13.6 / 16.8 / 23.2 / 23.5
+//          512^2    20.1 / 19.3 / 24.8 / 24.9 | 20.8 / 21.4 / 28.7 / 28.9
+//          1000x500 35.3 / 26.8 / 25.2 / 25.7 | 30.3 / 26.9 / 34.5 / 35.3
+//          1024^2   41.0 / 37.7 / 26.6 / 27.0 | 42.0 / 40.4 / 48.7 / 48.4
+//          2048^2     -  /   -  / 30.7 / 31.0 |   -  /   -  /  112 / 105   (12 columns: 31.1 | 115)
+// (AugRie's 4 columns and more record and skip quiet tiles, which the narrower
+// ones do not: there a lake at rest is solved edge by edge.)
 int narrow_width(int nx, int ny, int solver, int cus) {
     struct Limit {
         int width;
         double waves;  // per SIMD
     };
     static const Limit light[] = {{1, 0.625}, {2, 1.0}, {4, 2.25}}, hybrid[] = {{1, 2.0}, {2, 4.5}, {4, 1e30}},
-                       augrie[] = {{1, 2.0}, {2, 4.5}, {0, 1e30}};
+                       augrie[] = {{1, 4.5}, {2, 4.5}, {8, 16.0}};
     const Limit* t = solver == SOLVER_AUGRIE ? augrie : solver == SOLVER_HYBRID ? hybrid : light;
     const double strips = (double)((ny + kStripRows - 1) / kStripRows);
     for (int i = 0; i < 3; ++i)
-        if (strips * ((nx + std::max(t[i].width, 1) - 1) / std::max(t[i].width, 1)) <= t[i].waves * 4.0 * cus)
-            return t[i].width;
+        if (strips * ((nx + t[i].width - 1) / t[i].width) <= t[i].waves * 4.0 * cus) return t[i].width;
     return 0;
 }
 
@@ -365,7 +366,13 @@ int ensure_defer_queue(swe_hip_block* k) {
 
 // Strip tiles of the narrowest width: the most any width needs.
 size_t max_tiles(const swe_hip_block* k) {
-    return (size_t)((k->ny + kStripRows - 1) / kStripRows) * (size_t)((k->nx + 3) / 4);
+    return (size_t)((k->ny + kStripRows - 1) / kStripRows) * (size_t)((k->nx + kQuietCols - 1) / kQuietCols);
+}
+
+// Whether quiet tiles can be skipped at strip width xseg.
+bool records_quiet(const swe_hip_block* k, int xseg) {
+    const long strips = (k->ny + kStripRows - 1) / kStripRows;
+    return xseg % kRecordWidth == 0 && strips * ((k->nx + xseg - 1) / xseg) < kMaxSegments;
 }
 
 // Workgroups the quiet-tile plan can use at any width of whole record tiles.
@@ -382,7 +389,7 @@ int ensure_quiet_record(swe_hip_block* k) {
     HIP_TRY(hipMalloc(&k->quiet, n * sizeof(unsigned)));
     HIP_TRY(hipMalloc(&k->tspeed, n * sizeof(float)));
     const size_t groups = plan_groups_max(k);
-    HIP_TRY(hipMalloc(&k->tlist, groups * kPlanGroup * kPlanPieces * sizeof(unsigned)));
+    HIP_TRY(hipMalloc(&k->tlist, groups * kPlanGroup * sizeof(unsigned)));
     HIP_TRY(hipMalloc(&k->tcount, groups * sizeof(unsigned)));
     return 0;
 }
@@ -409,7 +416,7 @@ int pc_fused(swe_hip_block* k, int slotIn, int out, float dtFixed, unsigned rbSe
     io.dtFixed = dtFixed;
     const int step = k->pcStep + 1;
     const int es = eff_solver(k);
-    if (k->skipQuiet && es == SOLVER_AUGRIE && launch_width(k) % kQuietCols == 0) {
+    if (k->skipQuiet && es == SOLVER_AUGRIE && records_quiet(k, launch_width(k))) {
         if (int r = ensure_quiet_record(k)) return r;
         io.quiet = k->quiet;
         io.speed = k->tspeed;
@@ -586,7 +593,7 @@ int run_u_device_loop(swe_hip_block* k, int nsteps, float* t_inout, float* dt_lo
             io.step = s;
             // (only the augmented solver keeps a record, at widths of whole record tiles)
             const int es = defer ? SOLVER_AUGRIE_DEFER : eff_solver(k);
-            const bool record = (es == SOLVER_AUGRIE || es == SOLVER_AUGRIE_DEFER) && xseg % kQuietCols == 0;
+            const bool record = (es == SOLVER_AUGRIE || es == SOLVER_AUGRIE_DEFER) && records_quiet(k, xseg);
             if (k->skipQuiet && s >= 3 && record) {
                 if (tm && tm->perKernel && !extTimed) HIP_TRY(tm->mark(k->stream, 0));
                 if (tm) ++tm->plans;
@@ -1867,7 +1874,7 @@ size_t noalloc_layout(const swe_hip_block& k, size_t off[7]) {
     off[4] = at;
     at += align256(2 * tiles * sizeof(float));
     off[5] = at;
-    at += align256(groups * kPlanGroup * kPlanPieces * sizeof(unsigned));
+    at += align256(groups * kPlanGroup * sizeof(unsigned));
     off[6] = at;
     at += align256(groups * sizeof(unsigned));
     return at;

@@ -1,4 +1,4 @@
-"""Small blocks run strips of 1, 2 or 4 columns (narrow_width in swe_hip.hip)
+"""Small blocks run strips of 1, 2, 4 or 8 columns (narrow_width in swe_hip.hip)
 until the caller sets a width: the device loop and the per-call loop at the
 edges of the strips, and across the sizes where the width changes."""
 import numpy as np
