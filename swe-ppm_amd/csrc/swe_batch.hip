@@ -426,12 +426,14 @@ int enqueue_iteration(swe_hip_batch* k) {
     const bool defer = k->fused && solver == SOLVER_AUGRIE_MLP && k->deferQ;
     // groups == 0: the direct form (one wave per possible item) for the fused
     // sweep; the store strategy's persistent grids then take the default size
-    const bool direct = k->groups == 0;
+    const int direct = k->groups != 0 ? 0 : k->mode == BATCH_LTS ? 1 : kWavesPerGroup;  // waves per workgroup
     const int persistent = direct ? default_groups(k) : k->groups;
-    const int directGrid = (int)((k->itemsMost + kWavesPerGroup - 1) / kWavesPerGroup);
-    int rc = k->fused ? launch_fused(defer ? SOLVER_AUGRIE_DEFER : solver, k->xs,
-                                     direct ? std::max(1, directGrid) : k->groups, direct ? 1 : 0, k->A, k->dDesc,
-                                     k->dState, k->dG, k->dItems, k->deferQ, k->dJobs, k->dGeom, k->stream)
+    const int round = direct == 1 ? kDirectRound : kWavesPerGroup;  // items the grid is rounded up to
+    const long long directGrid =
+        direct ? std::max<long long>(1, (k->itemsMost + round - 1) / round) * round / direct : 0;
+    int rc = k->fused ? launch_fused(defer ? SOLVER_AUGRIE_DEFER : solver, k->xs, direct ? (int)directGrid : k->groups,
+                                     direct, k->A, k->dDesc, k->dState, k->dG, k->dItems, k->deferQ, k->dJobs,
+                                     k->dGeom, k->stream)
                       : launch_sweep(solver, k->xs, persistent, k->A, k->dDesc, k->dState, k->dG, k->dItems, k->stream);
     if (rc) return rc;
     if (defer) {
