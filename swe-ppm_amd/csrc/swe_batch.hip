@@ -12,6 +12,7 @@
 
 #include "../../include/swe_hip_batch.h"
 #include "../../include/swe_hip_mlp.h"
+#include "host_stage.hpp"
 #include "kernels_batch.hpp"
 #include "swe_internal.h"
 
@@ -366,6 +367,7 @@ struct swe_hip_batch {
     long long itemsMost = 0;  // the longest queue an iteration can have (the direct grid)
     int cus = 256;
     hipStream_t stream = nullptr;
+    HostStage stage;  // uploads and downloads of large batches
     hipGraphExec_t exec = nullptr;
     bool uploaded = false;
     const unsigned* mlp = nullptr;  // attached learned middle state (weight fragments), or null
@@ -742,6 +744,7 @@ int swe_hip_batch_create(int nblocks, const int* nx, const int* ny, const float*
         swe_hip_batch_destroy(k);
         return rc;
     }
+    k->stage.create(3 * bytes);
     k->groups = 0;  // the direct form: fastest on the LTS tiling and the ensemble (swe_hip_batch_autotune)
     *out = k;
     return SWE_HIP_OK;
@@ -767,6 +770,7 @@ int swe_hip_batch_destroy(swe_hip_batch* k) {
     if (k->dDtLog) (void)hipFree(k->dDtLog);
     if (k->dIterLog) (void)hipFree(k->dIterLog);
     if (k->hostStat) (void)hipHostFree(k->hostStat);
+    k->stage.destroy();
     if (k->stream) (void)hipStreamDestroy(k->stream);
     delete k;
     return SWE_HIP_OK;
@@ -778,10 +782,11 @@ int swe_hip_batch_upload(swe_hip_batch* k, const float* h, const float* hu, cons
         return SWE_HIP_EINVAL;
     }
     const size_t bytes = sizeof(float) * (size_t)k->total;
-    HIP_TRY(hipMemcpyAsync(k->A.h[0], h, bytes, hipMemcpyHostToDevice, k->stream));
-    HIP_TRY(hipMemcpyAsync(k->A.hu[0], hu, bytes, hipMemcpyHostToDevice, k->stream));
-    HIP_TRY(hipMemcpyAsync(k->A.hv[0], hv, bytes, hipMemcpyHostToDevice, k->stream));
-    HIP_TRY(hipMemcpyAsync(k->A.b, b, bytes, hipMemcpyHostToDevice, k->stream));
+    const HostCopy copies[4] = {{const_cast<float*>(h), k->A.h[0], bytes},
+                                {const_cast<float*>(hu), k->A.hu[0], bytes},
+                                {const_cast<float*>(hv), k->A.hv[0], bytes},
+                                {const_cast<float*>(b), k->A.b, bytes}};
+    HIP_TRY(k->stage.to_device(copies, 4, k->stream));
     std::vector<BatchBlockState> st(k->nblocks);
     for (auto& s : st) {
         std::memset(&s, 0, sizeof(s));
@@ -814,10 +819,9 @@ int swe_hip_batch_download(swe_hip_batch* k, float* h, float* hu, float* hv, flo
         return SWE_HIP_EINVAL;
     }
     const size_t bytes = sizeof(float) * (size_t)k->total;
-    HIP_TRY(hipMemcpyAsync(h, k->A.h[0], bytes, hipMemcpyDeviceToHost, k->stream));
-    HIP_TRY(hipMemcpyAsync(hu, k->A.hu[0], bytes, hipMemcpyDeviceToHost, k->stream));
-    HIP_TRY(hipMemcpyAsync(hv, k->A.hv[0], bytes, hipMemcpyDeviceToHost, k->stream));
-    if (b) HIP_TRY(hipMemcpyAsync(b, k->A.b, bytes, hipMemcpyDeviceToHost, k->stream));
+    const HostCopy copies[4] = {
+        {h, k->A.h[0], bytes}, {hu, k->A.hu[0], bytes}, {hv, k->A.hv[0], bytes}, {b, k->A.b, bytes}};
+    HIP_TRY(k->stage.to_host(copies, b ? 4 : 3, k->stream));
     HIP_TRY(hipStreamSynchronize(k->stream));
     return SWE_HIP_OK;
 }
