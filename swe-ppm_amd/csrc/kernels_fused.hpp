@@ -17,6 +17,9 @@
 // Work decomposition and edge order are those of the strip sweep
 // (kernels_u.hpp), so S(k) and M(k) are bit-identical to the two-kernel step.
 //
+// Flavour S (V == kSplit) takes its own dt rule, update and CFL maximum through
+// the same launch and keeps no quiet record.
+//
 // Quiet tiles.  The quiet record works on tiles of one strip (62 rows) by
 // kQuietCols columns.  Launch k records per tile which of its parts had all
 // four sums of every owned cell +0 (bit pattern 0) with no deferred edge --
@@ -191,7 +194,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(fused_waves
     const int nxs = (v.nx + XS - 1) / XS;
     const int nx = v.nx, ny = v.ny;
 
-    const float dt = io.dtFixed >= 0.f ? io.dtFixed : timestep_from_max(ctl->smax[slotIn].value(), v.dx, v.dy);
+    float dt = io.dtFixed;
+    if (!(dt >= 0.f)) {
+        const float s = ctl->smax[slotIn].value();
+        dt = V == kSplit ? split_timestep(s, v.dx) : timestep_from_max(s, v.dx, v.dy);
+    }
     if (blockIdx.x == 0) {
         ctl->smax[slotClear].clear();
         if (threadIdx.x == 0) {
@@ -203,7 +210,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(fused_waves
             if (dtLog) dtLog[logIdx] = dt;
         }
     }
-    constexpr bool kRecord = quiet_record<S>(XS);
+    constexpr bool kRecord = V != kSplit && quiet_record<S>(XS);
     const int items = nyt * nxs;
     // list mode: entry after entry until the list ends (the grid covers the
     // usual lists once)
@@ -259,7 +266,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(fused_waves
             auto updated = [&](const Raw& r, int x) -> Q3 {
                 Q3 q{r.h, r.hu, r.hv};
                 if (x >= 1 && x <= nx && rowInterior) {
-                    const Cell u = update_cell(q.h, q.hu, q.hv, dtdx, dtdy, r.sx, r.sy, r.su, r.sv);
+                    const Cell u = step_cell<V>(q.h, q.hu, q.hv, dtdx, dtdy, r.sx, r.sy, r.su, r.sv);
                     q = Q3{u.h, u.hu, u.hv};
                 }
                 return q;
@@ -321,8 +328,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(fused_waves
             // x-edges count on owned rows (each interior row is owned by one strip),
             // so a record tile's maximum depends on its footprint only; which lanes
             // count is the same in every column, so they are masked at the tile's end.
-            float smaxX = e.speed, smaxY = 0.f;
+            // Flavour S counts the x-edges of every row: edge (0 | 1) by the
+            // first segment, any other halo edge by the segment left of it (the column
+            // loaded as halo lacks its ghost rows' boundary condition, as do lanes past
+            // the top ghost row).
+            float smaxX = V != kSplit ? e.speed : x0 == 1 ? dev::smax(0.f, e.speed) : 0.f, smaxY = 0.f;
             auto tile_max = [&] {
+                if constexpr (V == kSplit) return wave_max<N>(rowValid ? smaxX : 0.f);
                 return wave_max<N>(dev::smax(owned ? smaxX : 0.f, hEdgeValid ? smaxY : 0.f));
             };
             // the segment's maximum over its record tiles, wave-uniform (float bits:
@@ -357,7 +369,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(fused_waves
                     eh = defer_edge(eh, owned || y == 0, make_uint2((unsigned)x | kDeferY, (unsigned)y), io.deferQ,
                                     &ctl->defer[slotOut]);
                 }
-                smaxY = A::max(smaxY, eh.speed);
+                if constexpr (V != kSplit) smaxY = A::max(smaxY, eh.speed);
                 const float aH = __shfl_up(eh.hR, 1, 64);
                 const float aHv = __shfl_up(eh.huR, 1, 64);
                 const float sx = carryH + ev.hL, su = carryHu + ev.huL, sy = aH + eh.hL, sv = aHv + eh.huL;

@@ -234,6 +234,18 @@ __device__ __forceinline__ float timestep_from_max(float s, float dx, float dy) 
     return FLT_MAX;
 }
 
+// Variant of the sweep, fused and apply kernels (template parameter V): 0 and 1
+// are flavour U in IEEE and fast arithmetic, kSplit is flavour S, swe_simple's
+// split step (src/blocks/SWE_DimensionalSplitting.cpp:105-210) in IEEE
+// arithmetic.  Its y-sweep reads the old state, as flavour U's edges do, so the
+// edges, sums and their layout are the same; what differs is
+//   the CFL maximum: over the x-edges of all rows, ghost rows included, none of
+//                    the y-edges', and dt = 0.4 dx / max without a guard;
+//   the update:      Q* = Q - dt/dx (x sums), then h and hv of it - dt/dx (y
+//                    sums) -- the y part uses dx too -- without the dry clamp.
+constexpr int kSplit = 2;
+__host__ __device__ __forceinline__ float split_timestep(float s, float dx) { return kCfl * (dx / s); }
+
 // The maximum over the wave's lanes.  Dpp: by data-parallel-primitive moves
 // (within rows of 16 lanes, then across rows), valid in lane 63 and returned as a
 // uniform value; for non-negative numbers without NaN.  It takes about a tenth
@@ -424,6 +436,17 @@ __device__ __forceinline__ Cell update_cell(float h, float hu, float hv, float d
     return c;
 }
 
+// Variant V's update: flavour S takes dt/dx in both directions and clamps nothing
+// (SWE_DimensionalSplitting.cpp:150-168, 196-206).
+template <int V>
+__device__ __forceinline__ Cell step_cell(float h, float hu, float hv, float dtdx, float dtdy, float sx, float sy,
+                                          float su, float sv) {
+    if constexpr (V == kSplit)
+        return Cell{(h - dtdx * sx) - dtdx * sy, hu - dtdx * su, hv - dtdx * sv};
+    else
+        return update_cell(h, hu, hv, dtdx, dtdy, sx, sy, su, sv);
+}
+
 // One loaded cell: state plus the quantities its edges share.
 struct CellQ {
     float h, hu, hv, b, u, v, c, sq, inv, fx, fy;
@@ -476,7 +499,7 @@ __device__ __forceinline__ CellQ cell_q(float h, float hu, float hv, float b) {
 // if every cell was in the range.
 template <class Ctx, int V, class Body>
 __device__ __forceinline__ void run_tile(int lane, const Body& body) {
-    if constexpr (V == 0 && Ctx::kNormalForm) {
+    if constexpr (V != 1 && Ctx::kNormalForm) {
         if (body(std::true_type(), lane)) return;
         asm volatile("" : "+v"(lane));  // nothing of the general form is computed before
     }
@@ -572,7 +595,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MODE == MOD
         // halo vertical edge (x0-1 | x0)
         const dev::EdgeOut e = solver.template solve<A>(cq.xside(), nq.xside());
         float carryH = e.hR, carryHu = e.huR;
-        float smaxv = rowInterior ? e.speed : 0.f;
+        const bool xCounts = V == kSplit ? rowValid : rowInterior;
+        float smaxv = !xCounts ? 0.f : V == kSplit ? dev::smax(0.f, e.speed) : e.speed;
 
         for (int x = x0; x <= x1; ++x) {
             ch = nh;
@@ -604,11 +628,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MODE == MOD
 
             // vertical edge (x | x+1)
             const dev::EdgeOut ev = solver.template solve<A>(cq.xside(), nq.xside());
-            if (rowInterior) smaxv = dev::smax(smaxv, ev.speed);
+            if (xCounts) smaxv = dev::smax(smaxv, ev.speed);
 
             // horizontal edge (y | y+1): upper cell from lane+1
             const dev::EdgeOut eh = solver.template solve<A>(cq.yside(), cq.yside_from_lane_above());
-            if (hEdgeValid) smaxv = dev::smax(smaxv, eh.speed);
+            if (V != kSplit && hEdgeValid) smaxv = dev::smax(smaxv, eh.speed);
             // up-going part of edge (y-1 | y) from lane-1
             const float aH = __shfl_up(eh.hR, 1, 64);
             const float aHv = __shfl_up(eh.huR, 1, 64);

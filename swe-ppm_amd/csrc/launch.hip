@@ -1,7 +1,6 @@
 // launch.hip -- solver-independent launches and the solver dispatch.
 #include <hip/hip_runtime.h>
 
-#include "kernels_s.hpp"
 #include "kernels_u.hpp"
 #include "swe_internal.h"
 
@@ -172,7 +171,9 @@ __global__ __launch_bounds__(kPlanGroup) void quiet_plan_kernel(const unsigned* 
 // A kernel of its own after the flux pass: it needs no event in the stream
 // (an event there costs the stream a pause before its next kernel), and
 // the host learns the maximum while the stream runs on.
-__global__ void readback_kernel(const DeviceCtl* ctl, int slot, unsigned seq) {
+// slotClear >= 0: the next pass's slot, cleared on the way.
+__global__ void readback_kernel(DeviceCtl* ctl, int slot, unsigned seq, int slotClear) {
+    if (slotClear >= 0) ctl->smax[slotClear].clear();
     if (threadIdx.x == 0) {
         const unsigned long long w = ((unsigned long long)seq << 32) | ctl->smax[slot].bits();
         __hip_atomic_store(&ctl->ring[seq % kReadbackRing], w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
@@ -187,22 +188,38 @@ __global__ void ctl_reset_kernel(DeviceCtl* ctl, int par) {
     }
 }
 
-__global__ __launch_bounds__(256) void apply_s_kernel(StateView v, SumsView sums, float dt) {
-    const int y = blockIdx.x * 64 + (threadIdx.x & 63) + 1;
-    const int x0 = 1 + (blockIdx.y * 4 + (threadIdx.x >> 6)) * kSplitXSeg;
-    if (y > v.ny || x0 > v.nx) return;
-    const int x1 = min(x0 + kSplitXSeg - 1, v.nx);
-    const float dtdx = dt / v.dx;
-    for (int x = x0; x <= x1; ++x) {
+// Applies flavour S's sums to state v with dtFixed or (ctl given) the dt of CFL
+// slot `slot`, which is logged.  In place or, where o is another buffer, into
+// it: then the ghost cells go over unchanged.  One cell per thread, every load
+// in flight at once: the pass streams 40 bytes per cell (1024^2: 13.8 us with 16
+// cells a thread).
+__global__ __launch_bounds__(256) void apply_s_kernel(StateView v, SumsView sums, StateView o, float dtFixed,
+                                                      DeviceCtl* ctl, int slot, float* dtLog, int logIdx) {
+    const int y = blockIdx.x * 64 + (threadIdx.x & 63);
+    const int x = blockIdx.y * kWavesPerGroup + (threadIdx.x >> 6);
+    const float dt = ctl ? split_timestep(ctl->smax[slot].value(), v.dx) : dtFixed;
+    if (x <= v.nx + 1 && y <= v.ny + 1) {
         const size_t c = idx(v, x, y);
-        const float hStar = v.h[c] - dtdx * sums.sx[c];
-        const float huStar = v.hu[c] - dtdx * sums.su[c];
-        v.h[c] = hStar - dtdx * sums.sy[c];
-        v.hu[c] = huStar;
-        v.hv[c] = v.hv[c] - dtdx * sums.sv[c];
+        if (x >= 1 && x <= v.nx && y >= 1 && y <= v.ny) {
+            const float dtdx = dt / v.dx;
+            const Cell n = step_cell<kSplit>(v.h[c], v.hu[c], v.hv[c], dtdx, dtdx, sums.sx[c], sums.sy[c],
+                                             sums.su[c], sums.sv[c]);
+            o.h[c] = n.h;
+            o.hu[c] = n.hu;
+            o.hv[c] = n.hv;
+        } else if (o.h != v.h) {
+            o.h[c] = v.h[c];
+            o.hu[c] = v.hu[c];
+            o.hv[c] = v.hv[c];
+        }
+    }
+    if (ctl && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) {
+        ctl->dt = dt;
+        ctl->t += dt;
+        ctl->steps += 1;
+        if (dtLog) dtLog[logIdx] = dt;
     }
 }
-
 
 template <int V>
 static int sweep_u_v(int solver, int mode, int xseg, StateView v, SumsView sums, float* hn, float* hun, float* hvn,
@@ -234,6 +251,9 @@ static int sweep_u_v(int solver, int mode, int xseg, StateView v, SumsView sums,
 int launch_sweep_u(int solver, int variant, int mode, int xseg, StateView v, SumsView sums, float* hn, float* hun,
                    float* hvn, BoundaryInfo bi, DeviceCtl* ctl, Slots sl, float dtFixed, int fuseBc, float* dtLog,
                    int logIdx, hipStream_t stream) {
+    if (variant == kSplit)
+        return sweep_u_v<kSplit>(solver, mode, xseg, v, sums, hn, hun, hvn, bi, ctl, sl, dtFixed, fuseBc, dtLog,
+                                 logIdx, stream);
     if (variant == 1)
         return sweep_u_v<1>(solver, mode, xseg, v, sums, hn, hun, hvn, bi, ctl, sl, dtFixed, fuseBc, dtLog, logIdx,
                             stream);
@@ -285,6 +305,8 @@ static int fused_u_v(int solver, int xseg, StateView v, FusedIO io, BoundaryInfo
 
 int launch_fused_u(int solver, int variant, int xseg, StateView v, FusedIO io, BoundaryInfo bi, DeviceCtl* ctl,
                    int slotIn, int slotOut, int slotClear, float* dtLog, int logIdx, hipStream_t stream) {
+    if (variant == kSplit)
+        return fused_u_v<kSplit>(solver, xseg, v, io, bi, ctl, slotIn, slotOut, slotClear, dtLog, logIdx, stream);
     if (variant == 1) return fused_u_v<1>(solver, xseg, v, io, bi, ctl, slotIn, slotOut, slotClear, dtLog, logIdx, stream);
     return fused_u_v<0>(solver, xseg, v, io, bi, ctl, slotIn, slotOut, slotClear, dtLog, logIdx, stream);
 }
@@ -301,31 +323,6 @@ int launch_advance_u(int solver, int xseg, StateView v, float* hn, float* hun, f
 
 int launch_solve_edges(int solver, int variant, int64_t n, const float* in, float* out, hipStream_t stream) {
     return variant == 1 ? solve_edges_v<1>(solver, n, in, out, stream) : solve_edges_v<0>(solver, n, in, out, stream);
-}
-
-static int dispatch_s(int solver, int dir, StateView v, SumsView sums, DeviceCtl* ctl, int par,
-                      hipStream_t stream) {
-    switch (solver) {
-        case SOLVER_HLLE:
-            return launch_sweep_s_solver<SOLVER_HLLE>(dir, v, sums, ctl, par, stream);
-        case SOLVER_FWAVE:
-            return launch_sweep_s_solver<SOLVER_FWAVE>(dir, v, sums, ctl, par, stream);
-        case SOLVER_AUGRIE:
-            return launch_sweep_s_solver<SOLVER_AUGRIE>(dir, v, sums, ctl, par, stream);
-        case SOLVER_HYBRID:
-            return launch_sweep_s_solver<SOLVER_HYBRID>(dir, v, sums, ctl, par, stream);
-        default:
-            set_error("unknown solver %d", solver);
-            return -1;
-    }
-}
-
-int launch_sweep_s_x(int solver, StateView v, SumsView sums, DeviceCtl* ctl, int par, hipStream_t stream) {
-    return dispatch_s(solver, 0, v, sums, ctl, par, stream);
-}
-
-int launch_sweep_s_y(int solver, StateView v, SumsView sums, hipStream_t stream) {
-    return dispatch_s(solver, 1, v, sums, nullptr, 0, stream);
 }
 
 int launch_apply_bc(StateView v, BoundaryInfo bi, hipStream_t stream) {
@@ -357,8 +354,8 @@ int launch_quiet_plan(const unsigned* quiet, float* speed, int nx, int ny, int x
     return 0;
 }
 
-int launch_readback(const DeviceCtl* ctl, int slot, unsigned seq, hipStream_t stream) {
-    hipLaunchKernelGGL(readback_kernel, dim3(1), dim3(64), 0, stream, ctl, slot, seq);
+int launch_readback(DeviceCtl* ctl, int slot, unsigned seq, int slotClear, hipStream_t stream) {
+    hipLaunchKernelGGL(readback_kernel, dim3(1), dim3(64), 0, stream, ctl, slot, seq, slotClear);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return hip_fail(e, "readback_kernel launch");
     return 0;
@@ -371,10 +368,11 @@ int launch_ctl_reset(DeviceCtl* ctl, int par, hipStream_t stream) {
     return 0;
 }
 
-int launch_apply_s(StateView v, SumsView sums, float dt, hipStream_t stream) {
-    const int nxs = (v.nx + kSplitXSeg - 1) / kSplitXSeg;
-    dim3 grid((v.ny + 63) / 64, (nxs + 3) / 4);
-    hipLaunchKernelGGL(apply_s_kernel, grid, dim3(256), 0, stream, v, sums, dt);
+int launch_apply_s(StateView v, SumsView sums, StateView o, float dtFixed, DeviceCtl* ctl, int slot, float* dtLog,
+                   int logIdx, hipStream_t stream) {
+    const dim3 grid((v.ny + 2 + 63) / 64, (v.nx + 2 + kWavesPerGroup - 1) / kWavesPerGroup);
+    hipLaunchKernelGGL(apply_s_kernel, grid, dim3(64 * kWavesPerGroup), 0, stream, v, sums, o, dtFixed, ctl, slot,
+                       dtLog, logIdx);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return hip_fail(e, "apply_s_kernel launch");
     return 0;

@@ -1,11 +1,12 @@
 // launch_solver.hip -- per-solver, per-math-variant kernel instantiations.
 // Compiled once per (solver, variant) with -DSWE_SOLVER_ID=<id> and
-// -DSWE_VARIANT=<0|1>, so that the big device solvers build in parallel
+// -DSWE_VARIANT=<0|1|2>, so that the big device solvers build in parallel
 // translation units and the two arithmetic variants get their own compile
 // flags:
 //   variant 0 (IEEE): no contraction, correctly rounded division and square
 //                     root -- bit-compatible with an IEEE CPU evaluation;
-//   variant 1 (fast): FMA contraction, hardware reciprocal / square root.
+//   variant 1 (fast): FMA contraction, hardware reciprocal / square root;
+//   variant 2 (kSplit): flavour S, compiled like variant 0.
 // The variant is also a template parameter of every kernel, so the two
 // instantiations never share a symbol.
 #include <hip/hip_ext.h>
@@ -13,7 +14,6 @@
 
 #include "kernels_advance.hpp"
 #include "kernels_fused.hpp"
-#include "kernels_s.hpp"
 #include "kernels_u.hpp"
 #include "swe_internal.h"
 
@@ -45,9 +45,19 @@ int go_u(StateView v, SumsView sums, float* hn, float* hun, float* hvn, Boundary
 template <int S, int MODE, int V>
 int go_u_xs(int xseg, StateView v, SumsView sums, float* hn, float* hun, float* hvn, BoundaryInfo bi,
             DeviceCtl* ctl, Slots sl, float dtFixed, int fuseBc, float* dtLog, int logIdx, hipStream_t stream) {
-    if constexpr (V == 0 && MODE == MODE_STORE)
-        if (xseg <= 2)  // the first pass of a small block (narrow_width)
+    // the narrow widths (narrow_width): the first pass of a loop, flavour S's sweep
+    // (Hybrid 1024^2 at 4 / 8 columns 35 / 50 us)
+    if constexpr (V != 1 && MODE == MODE_STORE) {
+        if (xseg <= 2)
             return go_u<S, MODE, 2, V>(v, sums, hn, hun, hvn, bi, ctl, sl, dtFixed, fuseBc, dtLog, logIdx, stream);
+        if (xseg == 4)
+            return go_u<S, MODE, 4, V>(v, sums, hn, hun, hvn, bi, ctl, sl, dtFixed, fuseBc, dtLog, logIdx, stream);
+    }
+    if constexpr (V == kSplit) {  // flavour S: 2, 4, 8 and 16 columns
+        if (xseg < 16)
+            return go_u<S, MODE, 8, V>(v, sums, hn, hun, hvn, bi, ctl, sl, dtFixed, fuseBc, dtLog, logIdx, stream);
+        return go_u<S, MODE, 16, V>(v, sums, hn, hun, hvn, bi, ctl, sl, dtFixed, fuseBc, dtLog, logIdx, stream);
+    }
     switch (xseg) {
         case 8:
         case 10:  // width 10 runs the sweeps at 8
@@ -81,6 +91,9 @@ template <int S, int V>
 int launch_sweep_u_solver(int mode, int xseg, StateView v, SumsView sums, float* hn, float* hun, float* hvn,
                           BoundaryInfo bi, DeviceCtl* ctl, Slots sl, float dtFixed, int fuseBc, float* dtLog,
                           int logIdx, hipStream_t stream) {
+    if constexpr (V == kSplit)
+        return go_u_xs<S, MODE_STORE, V>(xseg, v, sums, hn, hun, hvn, bi, ctl, sl, dtFixed, fuseBc, dtLog, logIdx,
+                                         stream);
     switch (mode) {
         case MODE_MAX:
             return go_u_xs<S, MODE_MAX, V>(xseg, v, sums, hn, hun, hvn, bi, ctl, sl, dtFixed, fuseBc, dtLog, logIdx,
@@ -113,20 +126,21 @@ int launch_fused_u_solver(int xseg, StateView v, FusedIO io, BoundaryInfo bi, De
                                bi, ctl, slotIn, slotOut, slotClear, dtLog, logIdx);
         }
     };
-    if (V == 0 && xseg == 1)  // narrow widths of small blocks (narrow_width)
-        go(std::integral_constant<int, V == 0 ? 1 : 8>());
-    else if (V == 0 && xseg == 2)
-        go(std::integral_constant<int, V == 0 ? 2 : 8>());
+    constexpr bool kNarrow = V != 1, kWide = V != kSplit;  // flavour S: 1, 2, 4, 8 and 16 columns
+    if (kNarrow && xseg == 1)  // narrow widths of small blocks (narrow_width)
+        go(std::integral_constant<int, kNarrow ? 1 : 8>());
+    else if (kNarrow && xseg == 2)
+        go(std::integral_constant<int, kNarrow ? 2 : 8>());
     else if (xseg == 4)
         go(std::integral_constant<int, 4>());
-    else if (xseg == 10)
-        go(std::integral_constant<int, 10>());
-    else if (xseg == 12)
-        go(std::integral_constant<int, 12>());
-    else if (xseg == 16)
+    else if (kWide && xseg == 10)
+        go(std::integral_constant<int, kWide ? 10 : 8>());
+    else if (kWide && xseg == 12)
+        go(std::integral_constant<int, kWide ? 12 : 8>());
+    else if (kWide && xseg == 32)
+        go(std::integral_constant<int, kWide ? 32 : 16>());
+    else if (xseg >= 16)
         go(std::integral_constant<int, 16>());
-    else if (xseg == 32)
-        go(std::integral_constant<int, 32>());
     else
         go(std::integral_constant<int, 8>());
     hipError_t e = hipGetLastError();
@@ -146,7 +160,7 @@ int launch_solve_edges_solver(int64_t n, const float* in, float* out, hipStream_
 template int launch_sweep_u_solver<SWE_SOLVER_ID, SWE_VARIANT>(int, int, StateView, SumsView, float*, float*,
                                                                float*, BoundaryInfo, DeviceCtl*, Slots, float, int,
                                                                float*, int, hipStream_t);
-#if SWE_SOLVER_ID != 4
+#if SWE_SOLVER_ID != 4 && SWE_VARIANT != 2
 template int launch_solve_edges_solver<SWE_SOLVER_ID, SWE_VARIANT>(int64_t, const float*, float*, hipStream_t);
 #endif
 template int launch_fused_u_solver<SWE_SOLVER_ID, SWE_VARIANT>(int, StateView, FusedIO, BoundaryInfo, DeviceCtl*, int,
@@ -177,27 +191,6 @@ int launch_advance_u_solver(int xseg, StateView v, float* hn, float* hun, float*
 }
 template int launch_advance_u_solver<SWE_SOLVER_ID>(int, StateView, float*, float*, float*, BoundaryInfo, DeviceCtl*,
                                                     int, int, int, int, float*, int, hipStream_t);
-#endif
-
-#if SWE_VARIANT == 0 && SWE_SOLVER_ID != 4
-template <int S>
-int launch_sweep_s_solver(int dir, StateView v, SumsView sums, DeviceCtl* ctl, int par, hipStream_t stream) {
-    if (dir == 0) {
-        const int nyt = (v.ny + 2 + 63) / 64;
-        const int nxs = (v.nx + 1 + kSplitXSeg - 1) / kSplitXSeg;
-        const int groups = (nyt * nxs + kWavesPerGroup - 1) / kWavesPerGroup;
-        hipLaunchKernelGGL((sweep_s_x_kernel<S>), dim3(groups), dim3(256), 0, stream, v, sums, ctl, par);
-    } else {
-        const int nyt = (v.ny + kStripRows - 1) / kStripRows;
-        const int nxs = (v.nx + kSplitXSeg - 1) / kSplitXSeg;
-        const int groups = (nyt * nxs + kWavesPerGroup - 1) / kWavesPerGroup;
-        hipLaunchKernelGGL((sweep_s_y_kernel<S>), dim3(groups), dim3(256), 0, stream, v, sums);
-    }
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return hip_fail(e, "sweep_s kernel launch");
-    return 0;
-}
-template int launch_sweep_s_solver<SWE_SOLVER_ID>(int, StateView, SumsView, DeviceCtl*, int, hipStream_t);
 #endif
 
 }  // namespace swe

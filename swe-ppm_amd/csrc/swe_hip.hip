@@ -15,7 +15,6 @@
 #include "../../include/swe_hip.h"
 #include "../../include/swe_hip_mlp.h"
 #include "kernels_advance.hpp"
-#include "kernels_s.hpp"
 #include "kernels_u.hpp"
 #include "swe_internal.h"
 
@@ -89,6 +88,7 @@ struct swe_hip_block {
     int pcSums = 0;  // sums set holding the last flux pass's sums (0: sums, 1: sums2)
     bool fluxValid = false;  // those sums belong to the current state (swe_hip_update may use them)
     int pcSlot = 0;  // CFL slot of the next flux pass (0, 1, 2 in turn)
+    bool slotClear = false;  // flavour S: the last report cleared slot pcSlot
     int pcStep = 0;  // fused flux passes since the last plain one: the quiet record's step
     // look-ahead (swe_hip_set_lookahead): once a caller has gone through
     // update(the dt returned) -> apply_bc -> fluxes, each flux pass queues
@@ -330,23 +330,36 @@ int check(swe_hip_block* k) {
     return 0;
 }
 
+// `count` arrays of the block's size, all of them or none.
+int alloc_fields(swe_hip_block* k, float** f, int count) {
+    const size_t bytes = field_elems(k) * sizeof(float);
+    for (int i = 0; i < count; ++i) {
+        const hipError_t e = hipMalloc(&f[i], bytes);
+        if (e == hipSuccess) continue;
+        for (int j = 0; j <= i; ++j) {
+            if (j < i) (void)hipFree(f[j]);
+            f[j] = nullptr;
+        }
+        return hip_fail(e, "hipMalloc of a second state buffer or sums set");
+    }
+    return 0;
+}
+
 int ensure_second_buffer(swe_hip_block* k) {
     const int o = k->cur ^ 1;
     if (k->h[o]) return 0;
-    const size_t bytes = field_elems(k) * sizeof(float);
-    HIP_TRY(hipMalloc(&k->h[o], bytes));
-    HIP_TRY(hipMalloc(&k->hu[o], bytes));
-    HIP_TRY(hipMalloc(&k->hv[o], bytes));
+    float* f[3];
+    if (int r = alloc_fields(k, f, 3)) return r;
+    k->h[o] = f[0];
+    k->hu[o] = f[1];
+    k->hv[o] = f[2];
     return 0;
 }
 
 int ensure_second_sums(swe_hip_block* k) {
     if (k->sums2[0]) return 0;
-    const size_t bytes = field_elems(k) * sizeof(float);
-    for (int i = 0; i < 4; ++i) {
-        HIP_TRY(hipMalloc(&k->sums2[i], bytes));
-        HIP_TRY(hipMemsetAsync(k->sums2[i], 0, bytes, k->stream));
-    }
+    if (int r = alloc_fields(k, k->sums2, 4)) return r;
+    for (int i = 0; i < 4; ++i) HIP_TRY(hipMemsetAsync(k->sums2[i], 0, field_elems(k) * sizeof(float), k->stream));
     return 0;
 }
 
@@ -431,7 +444,7 @@ int pc_fused(swe_hip_block* k, int slotIn, int out, float dtFixed, unsigned rbSe
         }
     }
     if (rbSeq != 0u)
-        if (int r = launch_readback(k->ctl, slotIn, rbSeq, k->stream)) return r;
+        if (int r = launch_readback(k->ctl, slotIn, rbSeq, -1, k->stream)) return r;
     if (int r = launch_fused_u(es, k->math, launch_width(k), view(k, k->cur), io, k->bi, k->ctl, slotIn, out, (out + 1) % 3,
                                nullptr, 0, k->stream))
         return r;
@@ -498,6 +511,7 @@ int ensure_dtlog(swe_hip_block* k, int n) {
     if (n <= k->dtlogCap) return 0;
     if (k->dtlog) HIP_TRY(hipFree(k->dtlog));
     k->dtlog = nullptr;
+    k->dtlogCap = 0;
     HIP_TRY(hipMalloc(&k->dtlog, sizeof(float) * n));
     k->dtlogCap = n;
     return 0;
@@ -660,6 +674,50 @@ int run_u_device_loop(swe_hip_block* k, int nsteps, float* t_inout, float* dt_lo
     HIP_TRY(hipMemcpyAsync(&t1, &k->ctl->t, sizeof(float), hipMemcpyDeviceToHost, k->stream));
     HIP_TRY(hipStreamSynchronize(k->stream));
     if (t_inout) *t_inout = t1;
+    return SWE_HIP_OK;
+}
+
+// Flavour S's step loop on the device: sweep on Q(0), then one launch per step
+// that applies the previous update on load (kernels_fused.hpp), then the last
+// update, which brings the state back to the buffer it came from (pointers that
+// a caller holds to a flavour-S state stay good).  Hybrid 1024^2, us per step:
+// boundary conditions, sweep, report to the host and update as launches of
+// their own 60 (120 with a sweep per direction), this loop 27.  The sums of the
+// last step end in k->sums and its dt in k->fluxDt, as the per-call API leaves
+// them.
+int run_s_device_loop(swe_hip_block* k, int nsteps, float* t_inout, float* dt_log) {
+    const int xseg = launch_width(k), home = k->cur;
+    k->slotClear = false;
+    const float t0 = t_inout ? *t_inout : 0.f;
+    HIP_TRY(hipMemcpyAsync(&k->ctl->t, &t0, sizeof(float), hipMemcpyHostToDevice, k->stream));
+    for (int slot = 0; slot < 3; ++slot)
+        if (int r = launch_ctl_reset(k->ctl, slot, k->stream)) return r;
+    if (int r = launch_apply_bc(view(k, home), k->bi, k->stream)) return r;
+    SumsView set[2] = {sums_view(k), sums2_view(k)};
+    if (int r = launch_sweep_u(k->solver, kSplit, MODE_STORE, xseg, view(k, home), set[0], nullptr, nullptr, nullptr,
+                               k->bi, k->ctl, Slots{0, 1}, -1.f, 0, nullptr, 0, k->stream))
+        return r;
+    int cur = home;
+    for (int s = 1; s < nsteps; ++s) {
+        const int o = cur ^ 1;
+        const FusedIO io{k->h[cur], k->hu[cur], k->hv[cur], k->b, k->h[o], k->hu[o], k->hv[o], set[(s - 1) & 1],
+                         set[s & 1]};
+        if (int r = launch_fused_u(k->solver, kSplit, xseg, view(k, cur), io, k->bi, k->ctl, (s - 1) % 3, s % 3,
+                                   (s + 1) % 3, k->dtlog, s - 1, k->stream))
+            return r;
+        cur = o;
+    }
+    if (int r = launch_apply_s(view(k, cur), set[(nsteps - 1) & 1], view(k, home), -1.f, k->ctl, (nsteps - 1) % 3,
+                               k->dtlog, nsteps - 1, k->stream))
+        return r;
+    if ((nsteps - 1) & 1) std::swap(k->sums, k->sums2);
+    if (dt_log) HIP_TRY(hipMemcpyAsync(dt_log, k->dtlog, sizeof(float) * nsteps, hipMemcpyDeviceToHost, k->stream));
+    float t1 = 0.f, dt = 0.f;
+    HIP_TRY(hipMemcpyAsync(&t1, &k->ctl->t, sizeof(float), hipMemcpyDeviceToHost, k->stream));
+    HIP_TRY(hipMemcpyAsync(&dt, &k->ctl->dt, sizeof(float), hipMemcpyDeviceToHost, k->stream));
+    HIP_TRY(hipStreamSynchronize(k->stream));
+    if (t_inout) *t_inout = t1;
+    k->fluxDt = dt;
     return SWE_HIP_OK;
 }
 
@@ -1138,7 +1196,7 @@ int swe_hip_fluxes(swe_hip_block* k, float* max_timestep) {
             if (int r = pc_fused(k, out, next, -1.f, want)) return r;
             k->spec = true;
             k->specOut = next;
-        } else if (int r = launch_readback(k->ctl, out, want, k->stream)) {
+        } else if (int r = launch_readback(k->ctl, out, want, -1, k->stream)) {
             return r;
         }
         if (int r = wait_readback(k, want, &bits)) return r;
@@ -1149,15 +1207,23 @@ int swe_hip_fluxes(swe_hip_block* k, float* max_timestep) {
         k->pcClean = true;
         *max_timestep = dt;
     } else {
-        if (int r = launch_ctl_reset(k->ctl, 0, k->stream)) return r;
-        if (int r = launch_sweep_s_x(k->solver, view(k, k->cur), sums_view(k), k->ctl, 0, k->stream)) return r;
+        // one sweep for both directions; the report clears the next pass's slot
+        const int slot = k->pcSlot;
+        if (!k->slotClear)
+            if (int r = launch_ctl_reset(k->ctl, slot, k->stream)) return r;
+        k->slotClear = false;
+        if (int r = launch_sweep_u(k->solver, kSplit, MODE_STORE, launch_width(k), view(k, k->cur), sums_view(k),
+                                   nullptr, nullptr, nullptr, k->bi, k->ctl, Slots{slot, (slot + 1) % 3}, -1.f, 0,
+                                   nullptr, 0, k->stream))
+            return r;
         if (++k->rbSeq == 0u) k->rbSeq = 1u;  // 0 means "no report"
-        if (int r = launch_readback(k->ctl, 0, k->rbSeq, k->stream)) return r;
+        k->pcSlot = (slot + 1) % 3;
+        if (int r = launch_readback(k->ctl, slot, k->rbSeq, k->pcSlot, k->stream)) return r;
+        k->slotClear = true;
         if (int r = wait_readback(k, k->rbSeq, &bits)) return r;
         float s;
         std::memcpy(&s, &bits, sizeof(s));
-        const float dt = (float).4 * (k->dx / s);  // SWE_DimensionalSplitting.cpp:221, no zero guard
-        if (int r = launch_sweep_s_y(k->solver, view(k, k->cur), sums_view(k), k->stream)) return r;
+        const float dt = split_timestep(s, k->dx);  // SWE_DimensionalSplitting.cpp:221, no zero guard
         k->fluxDt = dt;
         *max_timestep = dt;
     }
@@ -1189,7 +1255,7 @@ int swe_hip_update(swe_hip_block* k, float dt) {
         set_error("swe_hip_update: flavour S needs swe_hip_fluxes first");
         return SWE_HIP_ESTATE;
     }
-    return launch_apply_s(view(k, k->cur), sums_view(k), k->fluxDt, k->stream);
+    return launch_apply_s(view(k, k->cur), sums_view(k), view(k, k->cur), k->fluxDt, nullptr, 0, nullptr, 0, k->stream);
 }
 
 int swe_hip_run(swe_hip_block* k, int nsteps, float* t_inout, float* dt_log) {
@@ -1202,7 +1268,11 @@ int swe_hip_run(swe_hip_block* k, int nsteps, float* t_inout, float* dt_log) {
     }
     if (nsteps == 0) return SWE_HIP_OK;
     if (k->flavour != FLAVOUR_U) {
-        // flavour S keeps its host-visible dt (swe_simple reads it every step)
+        const bool room = ensure_dtlog(k, nsteps) == 0 &&
+                          (nsteps == 1 || (ensure_second_buffer(k) == 0 && ensure_second_sums(k) == 0));
+        if (room) return run_s_device_loop(k, nsteps, t_inout, dt_log);
+        // no memory for a second state and sums set: step by step through the per-call API
+        (void)hipGetLastError();
         float t = t_inout ? *t_inout : 0.f;
         for (int s = 0; s < nsteps; ++s) {
             float dt;

@@ -59,7 +59,7 @@ struct LaunchTimer {
 extern thread_local LaunchTimer g_fusedTimer;
 // Words of the host ring the readback kernel writes (slot seq % kReadbackRing).
 constexpr unsigned kReadbackRing = 4;
-int launch_readback(const DeviceCtl* ctl, int slot, unsigned seq, hipStream_t stream);
+int launch_readback(DeviceCtl* ctl, int slot, unsigned seq, int slotClear, hipStream_t stream);
 // Quiet-tile plan of fused launch `step` at strip width xseg (a multiple of
 // kQuietCols; kernels_fused.hpp): skipped tiles carry their speeds, the busy
 // runs are listed for the launch.  slotPrev is the CFL slot of the previous
@@ -68,10 +68,11 @@ int launch_readback(const DeviceCtl* ctl, int slot, unsigned seq, hipStream_t st
 int launch_quiet_plan(const unsigned* quiet, float* speed, int nx, int ny, int xseg, int step, DeviceCtl* ctl,
                       int slotPrev, int slotOut, unsigned* list, unsigned* count, unsigned rbSeq, hipStream_t stream);
 
-// Flavour S.
-int launch_sweep_s_x(int solver, StateView v, SumsView sums, DeviceCtl* ctl, int par, hipStream_t stream);
-int launch_sweep_s_y(int solver, StateView v, SumsView sums, hipStream_t stream);
-int launch_apply_s(StateView v, SumsView sums, float dt, hipStream_t stream);
+// Flavour S's update with dtFixed or, with ctl, the dt of its CFL slot, into o
+// (the block's own state or another buffer).  Its sweep and fused launches are
+// launch_sweep_u (MODE_STORE) and launch_fused_u with variant kSplit.
+int launch_apply_s(StateView v, SumsView sums, StateView o, float dtFixed, DeviceCtl* ctl, int slot, float* dtLog,
+                   int logIdx, hipStream_t stream);
 
 template <int V>
 int launch_apply_u_variant(StateView v, SumsView sums, BoundaryInfo bi, DeviceCtl* ctl, Slots sl, float dtFixed,
@@ -119,8 +120,6 @@ int launch_defer_solve(StateView vNew, SumsView sums, DeviceCtl* ctl, int slot, 
                        int groups, hipStream_t stream);
 template <int S, int V>
 int launch_solve_edges_solver(int64_t n, const float* in, float* out, hipStream_t stream);
-template <int S>
-int launch_sweep_s_solver(int dir, StateView v, SumsView sums, DeviceCtl* ctl, int par, hipStream_t stream);
 
 // Batched engine: strip sweep over the queued tiles (one translation unit per solver).
 template <int S>
