@@ -171,10 +171,22 @@ struct DeviceCtl {
     const unsigned* mlp;  // weight fragments of the learned middle state (solver SOLVER_AUGRIE_MLP)
     unsigned int defer[3];  // edges queued by the deferring sweep, per CFL slot (SOLVER_AUGRIE_DEFER)
     unsigned int busy[3];   // busy record tiles found by the quiet-tile plan of each CFL slot's launch
-    // coherent host ring the readback kernel writes (kept here rather than
-    // passed as a kernel argument, so the launch is an ordinary one)
+    // coherent host ring of report_max (kept here rather than passed as a kernel
+    // argument, so the launch is an ordinary one)
     unsigned long long* ring;
 };
+
+// The CFL maximum of a slot to the host, by one thread: one 64-bit word
+// (sequence number above, float bits below) stored at system scope into
+// coherent host memory, ctl->ring[seq % kReadbackRing], which the host polls for
+// that number.  It needs no event in the stream (an event there costs the
+// stream a pause before its next kernel), and the host learns the maximum
+// while the stream runs on.
+constexpr unsigned kReadbackRing = 4;
+__device__ __forceinline__ void report_max(const DeviceCtl* ctl, int slot, unsigned seq) {
+    __hip_atomic_store(&ctl->ring[seq % kReadbackRing], ((unsigned long long)seq << 32) | ctl->smax[slot].bits(),
+                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
 
 // Which CFL-maximum slot a launch reads or accumulates into, and which slot
 // it clears for a later step (the last reader of that slot has finished).

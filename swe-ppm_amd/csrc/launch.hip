@@ -102,8 +102,7 @@ __global__ __launch_bounds__(kPlanGroup) void quiet_plan_kernel(const unsigned* 
     const int slotNow = (step & 1) * tiles, slotPrev = ((step - 1) & 1) * tiles;
     const unsigned prevBusy = ctl->busy[slotPrev3];
     if (rbSeq != 0u && blockIdx.x == 0 && threadIdx.x == 0)  // the previous launch's maximum to the host
-        __hip_atomic_store(&ctl->ring[rbSeq % kReadbackRing], ((unsigned long long)rbSeq << 32) | ctl->smax[slotPrev3].bits(),
-                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        report_max(ctl, slotPrev3, rbSeq);
     const int piece = prevBusy == 0u ? fine : (int)min((unsigned)fine, max(1u, (prevBusy + kPlanWaves - 1) / kPlanWaves));
     const int yt = seg % nyt, xs = seg / nyt;
     const int f = xs * fine + i;
@@ -165,19 +164,11 @@ __global__ __launch_bounds__(kPlanGroup) void quiet_plan_kernel(const unsigned* 
     }
 }
 
-// The CFL maximum of a slot to the host: one 64-bit word (sequence number
-// above, float bits below) stored at system scope into coherent host memory,
-// ctl->ring[seq % kReadbackRing], which the host polls for that number.
-// A kernel of its own after the flux pass: it needs no event in the stream
-// (an event there costs the stream a pause before its next kernel), and
-// the host learns the maximum while the stream runs on.
-// slotClear >= 0: the next pass's slot, cleared on the way.
+// report_max after a flux pass that no further launch follows.  slotClear >= 0:
+// the next pass's slot, cleared on the way.
 __global__ void readback_kernel(DeviceCtl* ctl, int slot, unsigned seq, int slotClear) {
     if (slotClear >= 0) ctl->smax[slotClear].clear();
-    if (threadIdx.x == 0) {
-        const unsigned long long w = ((unsigned long long)seq << 32) | ctl->smax[slot].bits();
-        __hip_atomic_store(&ctl->ring[seq % kReadbackRing], w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-    }
+    if (threadIdx.x == 0) report_max(ctl, slot, seq);
 }
 
 __global__ void ctl_reset_kernel(DeviceCtl* ctl, int par) {

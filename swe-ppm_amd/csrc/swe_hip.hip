@@ -419,7 +419,7 @@ int ensure_quiet_record(swe_hip_block* k) {
 // writing the state (every call that could resets pcStep).  rbSeq != 0:
 // slot slotIn (the pass before, complete by then) is reported to the host
 // under that sequence number first, by the quiet-tile plan where there is
-// one, else by a readback kernel.
+// one, else by the fused launch as it starts.
 int pc_fused(swe_hip_block* k, int slotIn, int out, float dtFixed, unsigned rbSeq) {
     if (int r = ensure_second_buffer(k)) return r;
     if (int r = ensure_second_sums(k)) return r;
@@ -443,8 +443,7 @@ int pc_fused(swe_hip_block* k, int slotIn, int out, float dtFixed, unsigned rbSe
             io.count = k->tcount;
         }
     }
-    if (rbSeq != 0u)
-        if (int r = launch_readback(k->ctl, slotIn, rbSeq, -1, k->stream)) return r;
+    io.rbSeq = rbSeq;
     if (int r = launch_fused_u(es, k->math, launch_width(k), view(k, k->cur), io, k->bi, k->ctl, slotIn, out, (out + 1) % 3,
                                nullptr, 0, k->stream))
         return r;

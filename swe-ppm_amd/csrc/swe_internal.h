@@ -57,8 +57,6 @@ struct LaunchTimer {
     hipEvent_t start = nullptr, stop = nullptr;
 };
 extern thread_local LaunchTimer g_fusedTimer;
-// Words of the host ring the readback kernel writes (slot seq % kReadbackRing).
-constexpr unsigned kReadbackRing = 4;
 int launch_readback(DeviceCtl* ctl, int slot, unsigned seq, int slotClear, hipStream_t stream);
 // Quiet-tile plan of fused launch `step` at strip width xseg (a multiple of
 // kQuietCols; kernels_fused.hpp): skipped tiles carry their speeds, the busy
