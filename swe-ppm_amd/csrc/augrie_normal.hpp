@@ -18,10 +18,11 @@
 //     operation: the product is exact, so the sum is rounded once either way;
 //   * in a wave whose lanes are all subcritical wave 1 goes left and wave 3
 //     right, so only wave 2 chooses its side, as a weight of 0, 1/2 or 1.
-// On the 2048^2 islands with every cell moving a fused launch issues 56.9 M
-// vector instructions (83.6 M in the general form) and takes 130 us (156),
-// bound by vector issue; a lone wave (a 64 x 50 block) takes 29 us for 8 columns
-// (36), bound by its chain of dependent operations.
+//   * where both sides are calm (calm_edge) the middle state is not computed.
+// On the 2048^2 islands with every cell moving a fused launch issues 83.6 M vector
+// instructions in the general form, 61 M with all of the above but the last and
+// 35.6 M with it, and takes 156, 103 and 75 us: at the first two bound by vector
+// issue, now by half and for the rest by waits for memory.
 #pragma once
 
 #include "solvers_dev.hpp"
@@ -64,6 +65,29 @@ __device__ __forceinline__ float wall_depth(float h, float un, float c, float in
         invX = A::rcp(x);
         g = A::sqrt(0.5f * kGravity * (invX + inv));
     }
+}
+
+// True where the middle state is certain to have s1m <= 0 <= s2m, so that it need
+// not be computed: with U = max(|uL|, |uR|), cMin and cMax the two celerities,
+//   U + 2 cMax < 2.99 cMin   (U < 0.99 cMin and cMax < 1.5 cMin).
+// In each of its three forms the middle depth's celerity cm and velocity um bound
+// s1m = um - cm from above (s2m = um + cm from below by the mirrored edge):
+//   two rarefactions  cm = (2 (cL + cR) - du) / 4, so s1m = uL + 2 cL - 3 cm =
+//                     (uL + 3 uR) / 4 + cL / 2 - 3 cR / 2 <= U + cMax / 2 - 3 cMin / 2
+//                     (du <= 2 U < 4 cMin: the depth is not cut off at 0);
+//   two shocks        cm >= cMax and um <= uL, so s1m <= U - cMax;
+//   one of each       cMin <= cm <= cMax.  Left side deep: s1m = uL + 2 cL - 3 cm
+//                     <= U + 2 cMax - 3 cMin; right side deep: s1m = uR - 2 cR +
+//                     cm <= U - cMax.
+// Newton's iterates do not leave these bounds: the depth function is concave and
+// increases, so they rise to the root from the start, hMax for two shocks and
+// hMin for one of each, whose root lies below hMax.  All operands are normal
+// numbers, so rounding moves either side by less than 1e-5 cMin; the test leaves
+// 0.01 cMin.  uLm < 0 < uRp follow as well, so min(.., s2m) and max(.., s1m)
+// change neither l1 nor l3.  A dry side has c = 0 and fails the test.
+__device__ __forceinline__ bool calm_edge(float uL, float uR, float cL, float cR) {
+    const float u = vmax(fabsf(uL), fabsf(uR));
+    return __builtin_fmaf(2.f, vmax(cL, cR), u) < 2.99f * vmin(cL, cR);
 }
 
 // Speeds s1m, s2m of the middle state (middle_state's, whose depth the
@@ -183,8 +207,11 @@ __device__ __forceinline__ EdgeOut augrie_normal(const Side& L, const Side& R) {
     const float cHat = A::sqrt(gh);
     const float uHat = A::div(cL * uL + cR * uR, cL + cR);
     const float uLm = uL - cL, uRp = uR + cR;
-    float s1m, s2m;
-    middle_speeds(hL, hR, uL, uR, cL, cR, invL, invR, anyDry, s1m, s2m);
+    // The middle state enters through the signs of s1m and s2m alone where both
+    // sides run well below their celerity and differ little in depth (calm_edge):
+    // any values with s1m <= 0 <= s2m leave l1, l3 and the sonic test as they are.
+    float s1m = 0.f, s2m = 0.f;
+    if (!calm_edge(uL, uR, cL, cR)) middle_speeds(hL, hR, uL, uR, cL, cR, invL, invR, anyDry, s1m, s2m);
     const float l1 = vmin(vmin(uLm, uHat - cHat), s2m);
     const float l3 = vmax(vmax(uRp, uHat + cHat), s1m);
     const float l2 = 0.5f * (l1 + l3);
