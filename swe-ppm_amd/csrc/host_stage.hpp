@@ -35,8 +35,9 @@ class HostStage {
     // 0.73 / 0.54, 48 3.05 / 1.45, 96 10.5 / 3.2, 343 36 / 8.0; to the device 64 MiB
     // 2.35 / 2.05, 128 4.55 / 3.55, 456 14.9 / 10.3, but the first time (the slots'
     // own page faults) 64 MiB 2.6 / 4.9, 128 4.9 / 6.3, 456 18.1 / 17.0.  Slots of
-    // 1 / 2 / 4 / 8 MiB: 11.1 / 9.0 / 8.0 / 7.7 ms for 343 MB to the host.
-    static constexpr size_t kLeastToHost = size_t(16) << 20, kLeastToDevice = size_t(256) << 20;
+    // 1 / 2 / 4 / 8 MiB: 11.1 / 9.0 / 8.0 / 7.7 ms for 343 MB to the host.  Making the
+    // ring takes about 5 ms, which a download of 48 MiB does not win back.
+    static constexpr size_t kLeastToHost = size_t(64) << 20, kLeastToDevice = size_t(256) << 20;
 
     // Pinned memory and events for transfers of `bytes` in all to the host; without
     // them (too small, no memory, too few CPUs) copies go straight.
