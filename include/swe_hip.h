@@ -289,8 +289,8 @@ int swe_hip_solve_edges(int solver, int math, int64_t n, const float* hL, const 
 /* Tuning of the device loop (swe_hip_run): strategy 0 = recompute (max pass
  * + update pass), 1 = store (flux pass writing 4 net-update sums + apply
  * pass), 2 = fused (one launch per step that applies the previous update on
- * load, or, for HLLE and f-wave with the IEEE arithmetic on blocks of 2^19
- * cells and more, one that updates and takes the new state's CFL maximum; the
+ * load, or, with the IEEE arithmetic, for HLLE and f-wave on blocks of 2^19
+ * cells and more and for Hybrid from 6 * 2^20, one that updates and takes the new state's CFL maximum; the
  * default); xseg = x columns per wavefront strip (4, 8, 10, 12,
  * 16 or 32; the sweeps of strategies 0 and 1 run 4 as 16); -1 keeps the
  * current value.  All strategies and widths give
@@ -299,8 +299,8 @@ int swe_hip_solve_edges(int solver, int math, int64_t n, const float* hL, const 
  * threshold (nyt = ceil(ny/62); AugRie 12, 4; with a learned middle state
  * attached 5, 3; HLLE, f-wave, Hybrid 2, 1), else 8 (swe_hip_set_surrogate
  * re-picks it); with strategy 2 a block that does not fill the GPU at that
- * width runs strips of 1 to 8 columns instead (HLLE and f-wave on larger
- * blocks: their one-pass launch picks 8, 16 or 32).  The fused loop skips quiet tiles (swe_hip_set_quiet_skip)
+ * width runs strips of 1 to 8 columns instead (the one-pass launch picks 8, 16
+ * or 32).  The fused loop skips quiet tiles (swe_hip_set_quiet_skip)
  * at widths that are multiples of 4. */
 int swe_hip_set_tuning(swe_hip_block* blk, int strategy, int xseg);
 int swe_hip_get_tuning(swe_hip_block* blk, int* strategy, int* xseg);

@@ -46,6 +46,19 @@ __device__ __forceinline__ EdgeOut solve_edge(const Side& L, const Side& R) {
     }
 }
 
+// The speed alone that solver S reports for an edge (the light solvers; Hybrid
+// takes the augmented solver's from its whole edge, on the few shallow lanes).
+template <int S, class A>
+__device__ __forceinline__ float solver_speed(const Side& L, const Side& R) {
+    if constexpr (S == SOLVER_HYBRID) {
+        float speed = edge_speed<SOLVER_FWAVE, A>(L, R);
+        if (!(L.h >= kHybridTol && R.h >= kHybridTol)) speed = solve_edge<SOLVER_AUGRIE, A>(L, R).speed;
+        return speed;
+    } else {
+        return edge_speed<S, A>(L, R);
+    }
+}
+
 // Solver with per-kernel state, built once at kernel start from an optional
 // parameter block (the learned middle state keeps its network weights in
 // registers; the exact solvers have no state).  kNormalForm: the sweeps solve

@@ -1,5 +1,5 @@
-// kernels_advance.hpp -- flavour-U step of the light solvers (HLLE, f-wave) in
-// one pass over the state: one launch per time step, no sums in memory.
+// kernels_advance.hpp -- flavour-U step of the light solvers (HLLE, f-wave, and on
+// larger blocks Hybrid) in one pass over the state: one launch per time step, no sums in memory.
 //
 // Launch k reads Q(k) (ghost cells as setGhostLayer leaves them) and M(k), the
 // CFL maximum of its edges, solves the edges of Q(k), updates the cells with
@@ -157,8 +157,8 @@ advance_u_kernel(StateView v, float* hn, float* hun, float* hvn, BoundaryInfo bi
                 const CellQ uq = cell_q<A>(q.h, q.hu, q.hv, cq.b);
                 outside = outside || outside_range<N>(uq);
                 if (mine) {  // uniform; column x0 - 1 only lends its right edge
-                    smaxX = A::max(smaxX, dev::edge_speed<S, A>(wq.xside(), uq.xside()));
-                    smaxY = A::max(smaxY, dev::edge_speed<S, A>(uq.yside(), uq.yside_from_lane_above()));
+                    smaxX = A::max(smaxX, dev::solver_speed<S, A>(wq.xside(), uq.xside()));
+                    smaxY = A::max(smaxY, dev::solver_speed<S, A>(uq.yside(), uq.yside_from_lane_above()));
                 }
                 wq = uq;
             }
@@ -168,7 +168,7 @@ advance_u_kernel(StateView v, float* hn, float* hun, float* hvn, BoundaryInfo bi
                 if (!last) {
                     const CellQ rq = cell_q<A>(edge.h, edge.hu, edge.hv, nq.b);
                     outside = outside || outside_range<N>(rq);
-                    smaxX = A::max(smaxX, dev::edge_speed<S, A>(wq.xside(), rq.xside()));
+                    smaxX = A::max(smaxX, dev::solver_speed<S, A>(wq.xside(), rq.xside()));
                 }
             }
             cq = nq;

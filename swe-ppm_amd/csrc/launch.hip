@@ -308,6 +308,9 @@ int launch_advance_u(int solver, int xseg, StateView v, float* hn, float* hun, f
     if (solver == SOLVER_HLLE)
         return launch_advance_u_solver<SOLVER_HLLE>(xseg, v, hn, hun, hvn, bi, ctl, slotIn, slotOut, slotClear, last,
                                                     dtLog, logIdx, stream);
+    if (solver == SOLVER_HYBRID)
+        return launch_advance_u_solver<SOLVER_HYBRID>(xseg, v, hn, hun, hvn, bi, ctl, slotIn, slotOut, slotClear, last,
+                                                      dtLog, logIdx, stream);
     return launch_advance_u_solver<SOLVER_FWAVE>(xseg, v, hn, hun, hvn, bi, ctl, slotIn, slotOut, slotClear, last,
                                                  dtLog, logIdx, stream);
 }

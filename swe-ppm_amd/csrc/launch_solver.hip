@@ -166,7 +166,7 @@ template int launch_solve_edges_solver<SWE_SOLVER_ID, SWE_VARIANT>(int64_t, cons
 template int launch_fused_u_solver<SWE_SOLVER_ID, SWE_VARIANT>(int, StateView, FusedIO, BoundaryInfo, DeviceCtl*, int,
                                                                int, int, float*, int, hipStream_t);
 
-#if SWE_VARIANT == 0 && (SWE_SOLVER_ID == 0 || SWE_SOLVER_ID == 1)
+#if SWE_VARIANT == 0 && (SWE_SOLVER_ID == 0 || SWE_SOLVER_ID == 1 || SWE_SOLVER_ID == 3)
 template <int S>
 int launch_advance_u_solver(int xseg, StateView v, float* hn, float* hun, float* hvn, BoundaryInfo bi, DeviceCtl* ctl,
                             int slotIn, int slotOut, int slotClear, int last, float* dtLog, int logIdx,

@@ -148,7 +148,10 @@ int device_cus() {
 // against one pass): 512^2 21 / 17 against 20 / 17, 768^2 25 / 21 against 21 /
 // 19, 1024^2 28 / 22 against 23 / 22, 2048^2 59 / 54 against 46 / 44, 3000^2 154 /
 // 152 against 77 / 77, 4096^2 276 / 275 against 141 / 140.
-constexpr long kAdvanceCells = 1l << 19;
+// Hybrid solves the speeds of its shallow edges whole, so its line lies higher,
+// and it takes 8 columns: 2300^2 93 against 90, 2600^2 128 / 104, 3000^2 163 / 119,
+// 4096^2 282 / 195 (16 columns 203; 1500 x 901 42 / 78, 2048^2 72 / 85).
+constexpr long kAdvanceCells = 1l << 19, kAdvanceCellsHybrid = 3l << 21;
 
 // Default strip width of a flavour-U block.  A wider segment loads and solves
 // fewer halo columns per owned column and pays a wave's fixed start fewer
@@ -189,11 +192,11 @@ int default_xseg(int nx, int ny, int solver, int cus) {
 }
 
 // Whether the fused strategy's device loop takes the one-pass form
-// (kernels_advance.hpp): the light solvers on blocks whose state and sums pass
+// (kernels_advance.hpp): HLLE, f-wave and Hybrid on blocks whose state and sums pass
 // through memory every step.
 bool advance_pays(const swe_hip_block* k) {
-    return k->strategy == 2 && k->math == 0 && (k->solver == SOLVER_HLLE || k->solver == SOLVER_FWAVE) &&
-           (long)k->nx * k->ny >= kAdvanceCells;
+    if (k->strategy != 2 || k->math != 0 || k->solver == SOLVER_AUGRIE) return false;
+    return (long)k->nx * k->ny >= (k->solver == SOLVER_HYBRID ? kAdvanceCellsHybrid : kAdvanceCells);
 }
 // Its strip width until the caller sets one: the widest that still gives every
 // SIMD eight waves.  Measured at 8 / 16 / 32 columns (f-wave, us per step):
@@ -201,6 +204,7 @@ bool advance_pays(const swe_hip_block* k) {
 // 144.
 int advance_width(const swe_hip_block* k) {
     if (k->xsegSet) return k->xseg;
+    if (k->solver == SOLVER_HYBRID) return 8;
     const double strips = (double)((k->ny + kAdvanceRows - 1) / kAdvanceRows), simds = 4.0 * k->cus;
     for (int w : {32, 16})
         if (strips * ((k->nx + w - 1) / w) / simds >= 8.0) return w;
@@ -218,7 +222,7 @@ int advance_width(const swe_hip_block* k) {
 //          512^2    22.1 / 16.9 / 15.7 / 19.2     1000x500 34.1 / 25.6 / 19.2 / 21.1
 //   Hybrid 64x50    13.9 / 16.9 / 21.6 / 25.1     256^2   18.3 / 20.4 / 31.6 / 47.6
 //          512^2    27.0 / 24.5 / 34.4 / 53.7     1500x901 47.3 / 48.9 / 45.2 / 54.6
-//          2048^2   90.8 / 80.3 / 77.9 / 79.7     4096^2   341 / 306 / 274 / 280
+//          2048^2   90.8 / 80.3 / 75.0 / 71.5     4096^2   341 / 306 / 282 / 280
 //   AugRie, islands and (after the bar) every cell moving
 //          64x50    11.4 / 15.7 / 21.6 / 21.7     256^2   12.5 / 16.9 / 23.3 / 24.1 | 13.6 / 16.8 / 23.2 / 23.5
 //          512^2    20.1 / 19.3 / 24.8 / 24.9 | 20.8 / 21.4 / 28.7 / 28.9
@@ -229,14 +233,15 @@ int advance_width(const swe_hip_block* k) {
 // ones do not: there a lake at rest is solved edge by edge.)
 int narrow_width(int nx, int ny, int solver, int cus) {
     struct Limit {
-        int width;
-        double waves;  // per SIMD
+        int width = 0;  // 0: end of the list
+        double waves = 0;  // per SIMD
     };
-    static const Limit light[] = {{1, 0.625}, {2, 1.0}, {4, 2.25}}, hybrid[] = {{1, 2.0}, {2, 4.5}, {4, 1e30}},
-                       augrie[] = {{1, 4.5}, {2, 4.5}, {8, 16.0}};
+    static const Limit light[4] = {{1, 0.625}, {2, 1.0}, {4, 2.25}, {}},
+                       hybrid[4] = {{1, 2.0}, {2, 4.5}, {4, 12.0}, {8, 1e30}},
+                       augrie[4] = {{1, 4.5}, {2, 4.5}, {8, 16.0}, {}};
     const Limit* t = solver == SOLVER_AUGRIE ? augrie : solver == SOLVER_HYBRID ? hybrid : light;
     const double strips = (double)((ny + kStripRows - 1) / kStripRows);
-    for (int i = 0; i < 3; ++i)
+    for (int i = 0; i < 4 && t[i].width; ++i)
         if (strips * ((nx + t[i].width - 1) / t[i].width) <= t[i].waves * 4.0 * cus) return t[i].width;
     return 0;
 }

@@ -39,3 +39,29 @@ def test_one_pass_matches_oracle_and_store_strategy(swe, oracle, solver, nx, ny)
             for name, a, c in zip(("h", "hu", "hv"), got[2, widths[0]], ref):
                 assert same_bits(a[1:-1, 1:-1], c[1:-1, 1:-1]), (bnd, name)
             assert same_bits(got[2, widths[0]][3], ref[3])
+
+
+# Hybrid takes it from 6 Mi cells on, with both kinds of edge among the cells
+@pytest.mark.parametrize("nx,ny", [(103200, 61), (31, 203000), (2510, 2511)])
+def test_one_pass_hybrid_matches_oracle_and_store_strategy(swe, oracle, nx, ny):
+    rng = np.random.default_rng(nx)
+    shape = (nx + 2, ny + 2)
+    h = rng.uniform(0.5, 4.0, shape).astype(np.float32)
+    h[rng.random(shape) < 0.02] = 0.0
+    hu, hv = [(h * rng.uniform(-2.0, 2.0, shape)).astype(np.float32) for _ in range(2)]
+    state, bnd = (h, hu, hv, rng.uniform(-0.5, 0.5, shape).astype(np.float32)), [1, 0, 0, 1]
+    got = {}
+    for strategy, width in ((1, -1), (2, -1), (2, 16)):
+        with swe.SweBlock(nx, ny, 1.0, 1.5, solver=3) as blk:
+            blk.set_boundaries(bnd)
+            blk.set_tuning(strategy, width)
+            blk.upload(*state)
+            _, dts = blk.run(3)
+            got[strategy, width] = (*blk.download(), dts)
+    for key, out in got.items():  # ghosts included
+        for name, a, c in zip(("h", "hu", "hv", "dt"), out, got[1, -1]):
+            assert same_bits(a, c), (key, name)
+    ref = oracle.run_u(*state, 1.0, 1.5, bnd, 3, 3)
+    for name, a, c in zip(("h", "hu", "hv"), got[2, -1], ref):
+        assert same_bits(a[1:-1, 1:-1], c[1:-1, 1:-1]), name
+    assert same_bits(got[2, -1][3], ref[3])
