@@ -13,8 +13,8 @@
 // written) against the fused step's 60 (four sums written and read besides),
 // and solves the speeds of every edge a second time.  The light solvers are
 // bound by memory, so that pays where the state and sums do not stay in the
-// caches near the SIMDs (advance_pays); the augmented solver's speeds cost
-// most of its edge.
+// caches near the SIMDs (advance_pays); the augmented solver keeps its sums, whose
+// zeros are the record that lets quiet tiles be skipped.
 //
 // Work decomposition: the strip sweep's, with a deeper halo.  A wave owns 61
 // rows (lanes 1..61); lane 62 updates the row above too, for the speed of the

@@ -161,10 +161,10 @@ constexpr long kAdvanceCells = 1l << 19, kAdvanceCellsHybrid = 3l << 21;
 // still holds at least the solver's threshold of waves (waves per SIMD =
 // ceil(ny/62) * ceil(nx/xs) / (CUs x 4)), else 8:
 //                                      16     12
-//   AugRie (5 waves per SIMD)          12      4
+//   AugRie (6 waves per SIMD)          12      4
 //   learned middle state (deferring)    5      3   lighter, even waves
 //   HLLE, f-wave, Hybrid                2      1   light edges
-// Widths are whole numbers of the quiet record's 4-column tiles, so that
+// Widths are whole numbers of kRecordWidth columns (two record tiles), so that
 // quiet tiles can be skipped (10 columns, the old third choice, measured
 // within 1% of 8 where it won).  4, 10 and 32 stay available through
 // swe_hip_set_tuning.  Measured without skipping, radial dam break over
@@ -1814,7 +1814,8 @@ int swe_hip_autotune(swe_hip_block* k, int steps, float* ms_per_step) {
         copy_state(false);
     }
     // the light solvers on HBM-resident blocks: the recompute strategy moves
-    // 44 B per cell against the fused step's ~70 and can win at wide strips
+    // 44 B per cell and won at wide strips before the one-pass step (28 B); it is still
+    // timed, for blocks below that step's line and the fast arithmetic
     const int oldStrategy = k->strategy;
     int bestStrategy = oldStrategy;
     const int es = eff_solver(k);
