@@ -306,22 +306,23 @@ __device__ __forceinline__ int next_items(int* head, int* sBase) {
     return base;
 }
 
-// The direct form's item of a wave.  With local time stepping the workgroups are
-// single waves (direct == 1): a queue holds about as many waves as fit the chip,
-// and a finished tile's slot takes the next item while its neighbours still
-// run.  Consecutive workgroups go to the eight dies in turn, so runs of
-// kDirectRun consecutive items (strips one above the other, which share halo
-// rows) are given to one die's L2.  28-block LTS tiling, ms on the GPU for 6
+// The direct form's item of a wave, in workgroups of `direct` waves.  With local
+// time stepping they are single waves: a queue holds about as many waves as fit
+// the chip, and a finished tile's slot takes the next item while its neighbours
+// still run.  Where every block computes the launch has many rounds of waves and
+// four to a workgroup share their halo rows in one CU's cache.  Consecutive
+// workgroups go to the eight dies in turn, so runs of kDirectRun consecutive
+// ones (strips one above the other and the segments next to them, which share
+// halo cells) are given to one die's L2.  28-block LTS tiling, ms on the GPU for 6
 // macro steps: workgroups of four waves 103.4, single waves 108.8 without the
-// runs and 101.9 with them.  Where every block computes the launch has many
-// rounds of waves and four to a workgroup (direct == 4) share their halo rows
-// in one CU's cache: 512 instances, 150 steps, 81.9 against 82.3.
+// runs and 101.9 with them; 512 instances, 150 steps, 81.9 with four waves, 82.3
+// with one, and, with cheaper edges since, 78.2 without the runs and 76.8 with
+// them (runs of 64 workgroups 77.2).
 constexpr int kDirectRun = 4, kDirectDies = 8;
-constexpr int kDirectRound = kDirectRun * kDirectDies;  // the grid of single waves is a multiple of this
+constexpr int kDirectRound = kDirectRun * kDirectDies;  // the grid is a multiple of this
 __device__ __forceinline__ int direct_item(int direct, int group, int wave) {
-    if (direct != 1) return group * direct + wave;
     const int in = group % kDirectRound;
-    return group - in + in % kDirectDies * kDirectRun + in / kDirectDies;
+    return (group - in + in % kDirectDies * kDirectRun + in / kDirectDies) * direct + wave;
 }
 
 template <int S>
@@ -603,14 +604,14 @@ __device__ __forceinline__ void fused_tile(const BatchSolver<S>& solver, const S
         float carryH = e.hR, carryHu = e.huR;
         float smaxv = owned ? e.speed : 0.f;
         // Column x+1's loads are issued one column ahead (a software pipeline),
-        // as in the single-block fused kernel; past the tile they read column
-        // nx + 1 at most (a packed item's segments are inner ones) and are not
-        // used.  Not for the deferring sweep, which has no registers to spare.
+        // as in the single-block fused kernel; past the tile they read its right
+        // halo column again (the caches hold it) and are not used.  Not for the
+        // deferring sweep, which has no registers to spare.
         struct Raw {
             float h, hu, hv, sx, sy, su, sv, b;
         };
         auto load_raw = [&](int x) -> Raw {
-            const size_t c = col(min(x, nx + 1));
+            const size_t c = col(min(x, x0 + n));
             const unsigned ro = lane_bytes(rowC);
             return Raw{col_get(v.h, c, ro),    col_get(v.hu, c, ro),   col_get(v.hv, c, ro),   col_get(sIn.sx, c, ro),
                        col_get(sIn.sy, c, ro), col_get(sIn.su, c, ro), col_get(sIn.sv, c, ro), col_get(v.b, c, ro)};

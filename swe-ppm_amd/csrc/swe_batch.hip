@@ -430,9 +430,8 @@ int enqueue_iteration(swe_hip_batch* k) {
     // sweep; the store strategy's persistent grids then take the default size
     const int direct = k->groups != 0 ? 0 : k->mode == BATCH_LTS ? 1 : kWavesPerGroup;  // waves per workgroup
     const int persistent = direct ? default_groups(k) : k->groups;
-    const int round = direct == 1 ? kDirectRound : kWavesPerGroup;  // items the grid is rounded up to
-    const long long directGrid =
-        direct ? std::max<long long>(1, (k->itemsMost + round - 1) / round) * round / direct : 0;
+    const long long round = (long long)kDirectRound * std::max(direct, 1);  // items the grid is rounded up to
+    const long long directGrid = direct ? std::max<long long>(1, (k->itemsMost + round - 1) / round) * kDirectRound : 0;
     int rc = k->fused ? launch_fused(defer ? SOLVER_AUGRIE_DEFER : solver, k->xs, direct ? (int)directGrid : k->groups,
                                      direct, k->A, k->dDesc, k->dState, k->dG, k->dItems, k->deferQ, k->dJobs,
                                      k->dGeom, k->stream)
