@@ -6,8 +6,8 @@
 // itself moves 55 GB/s to and from pinned memory.  Here the calling thread
 // queues the DMA transfers of one slot after the other and the workers copy
 // between the slots and the arrays, faults included.
-// The calling thread alone talks to the GPU.  Every wait ends: a failed
-// transfer raises `stop`, which each waiting loop tests.
+// The calling thread alone talks to the GPU.  Every wait ends: there is at least
+// one worker, and a failed transfer raises `stop`, which each waiting loop tests.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -152,8 +152,10 @@ class HostStage {
             for (const int want = std::min(kWorkers, cpus() - 1); started < want; ++started)
                 workers[started] = std::thread(work);
         } catch (...) {  // as many as the system gives
-            if (started == 0) return straight(copies, count, stream, toDevice);
         }
+        // none, or this thread is bound to one CPU (create() may have run on another
+        // thread): nobody would fill or empty the slots
+        if (started == 0) return straight(copies, count, stream, toDevice);
 
         // done(i): the workers have finished piece i (pieces of a slot in order)
         auto done = [&](int i) {
