@@ -310,8 +310,10 @@ int swe_hip_get_tuning(swe_hip_block* blk, int* strategy, int* xseg);
  * the device loop (swe_hip_run, current strategy) from the block's current
  * state at each of the SWE_HIP_TUNE_WIDTHS widths 4, 8, 10, 12, 16, 32, restores
  * the state (h, hu, hv, the simulated time and step count), and keeps the
- * fastest width as if set with swe_hip_set_tuning.  ms_per_step (may be
- * null) receives the per-step times in that order.  With the fused strategy
+ * fastest width as if set with swe_hip_set_tuning (a small block whose width
+ * the caller has not set keeps its narrow strips where these are faster than
+ * all six).  ms_per_step (may be null) receives the per-step times in that
+ * order.  With the fused strategy
  * and the HLLE or f-wave solver it also times the recompute strategy (0) at
  * 16 and 32 columns and keeps it if faster: on blocks that do not fit the
  * GPU's caches recompute moves fewer bytes per cell (swe_hip_get_tuning

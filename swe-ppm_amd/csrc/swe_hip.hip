@@ -1784,22 +1784,25 @@ int swe_hip_autotune(swe_hip_block* k, int steps, float* ms_per_step) {
     }
     const int widths[SWE_HIP_TUNE_WIDTHS] = {4, 8, 10, 12, 16, 32};
     const int oldXseg = k->xseg;
-    const bool oldNarrowOk = k->narrowOk;
+    const bool oldNarrowOk = k->narrowOk, oldXsegSet = k->xsegSet;
     int best = oldXseg, rc = 0;
     float bestMs = 0.f;
     // one untimed run first (first launches of the process, allocations)
     if (e == hipSuccess) rc = swe_hip_run_timed(k, 2, nullptr, nullptr, nullptr, nullptr);
     if (e == hipSuccess && rc == 0) copy_state(false);
     // the narrow width of a small block, where the caller has not chosen one
-    bool narrowBest = false;
+    bool narrowTimed = false;
     float narrowMs = 0.f;
-    if (e == hipSuccess && rc == 0 && k->narrowOk && launch_width(k) != k->xseg) {
+    if (e == hipSuccess && rc == 0 && !advance_pays(k) && launch_width(k) != k->xseg) {
         rc = swe_hip_run_timed(k, steps, nullptr, &narrowMs, nullptr, nullptr);
         narrowMs /= steps;
-        narrowBest = rc == 0;
+        narrowTimed = rc == 0;
         if (rc == 0) copy_state(false);
     }
+    // every launch at the width that is timed, the one-pass step's included (its
+    // own choice, advance_width, is among them)
     k->narrowOk = false;
+    k->xsegSet = true;
     for (int i = 0; i < SWE_HIP_TUNE_WIDTHS && e == hipSuccess && rc == 0; ++i) {
         k->xseg = widths[i];
         float total = 0.f;
@@ -1819,6 +1822,8 @@ int swe_hip_autotune(swe_hip_block* k, int steps, float* ms_per_step) {
     const int oldStrategy = k->strategy;
     int bestStrategy = oldStrategy;
     const int es = eff_solver(k);
+    const bool narrowBest = narrowTimed && narrowMs < bestMs;
+    if (narrowBest) bestMs = narrowMs;
     if (oldStrategy == 2 && (es == SOLVER_HLLE || es == SOLVER_FWAVE)) {
         k->strategy = 0;
         for (int xs : {16, 32}) {
@@ -1850,13 +1855,13 @@ int swe_hip_autotune(swe_hip_block* k, int steps, float* ms_per_step) {
     if (rc || e != hipSuccess) {
         k->xseg = oldXseg;
         k->narrowOk = oldNarrowOk;
+        k->xsegSet = oldXsegSet;
         k->strategy = oldStrategy;
         return rc ? rc : hip_fail(e, "swe_hip_autotune");
     }
     k->xseg = best;
     k->strategy = bestStrategy;
-    k->xsegSet = true;
-    k->narrowOk = narrowBest && narrowMs < bestMs;
+    k->narrowOk = narrowBest && bestStrategy == oldStrategy;
     return SWE_HIP_OK;
 }
 
