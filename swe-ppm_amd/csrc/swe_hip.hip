@@ -1272,11 +1272,13 @@ int swe_hip_run(swe_hip_block* k, int nsteps, float* t_inout, float* dt_log) {
     }
     if (nsteps == 0) return SWE_HIP_OK;
     if (k->flavour != FLAVOUR_U) {
-        const bool room = ensure_dtlog(k, nsteps) == 0 &&
-                          (nsteps == 1 || (ensure_second_buffer(k) == 0 && ensure_second_sums(k) == 0));
-        if (room) return run_s_device_loop(k, nsteps, t_inout, dt_log);
-        // no memory for a second state and sums set: step by step through the per-call API
-        (void)hipGetLastError();
+        if (nsteps > 1) {
+            if (ensure_dtlog(k, nsteps) == 0 && ensure_second_buffer(k) == 0 && ensure_second_sums(k) == 0)
+                return run_s_device_loop(k, nsteps, t_inout, dt_log);
+            (void)hipGetLastError();
+        }
+        // a single step, or no memory for a second state and sums set: step by step
+        // through the per-call API
         float t = t_inout ? *t_inout : 0.f;
         for (int s = 0; s < nsteps; ++s) {
             float dt;
