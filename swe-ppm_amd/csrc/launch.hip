@@ -1,6 +1,8 @@
 // launch.hip -- solver-independent launches and the solver dispatch.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "kernels_u.hpp"
 #include "swe_internal.h"
 
@@ -183,13 +185,14 @@ __global__ void ctl_reset_kernel(DeviceCtl* ctl, int par) {
 // slot `slot`, which is logged.  In place or, where o is another buffer, into
 // it: then the ghost cells go over unchanged.  One cell per thread, every load
 // in flight at once: the pass streams 40 bytes per cell (1024^2: 13.8 us with 16
-// cells a thread).
+// cells a thread).  (Blocks of more columns than a grid's second dimension holds
+// at kWavesPerGroup each go round again.)
 __global__ __launch_bounds__(256) void apply_s_kernel(StateView v, SumsView sums, StateView o, float dtFixed,
                                                       DeviceCtl* ctl, int slot, float* dtLog, int logIdx) {
     const int y = blockIdx.x * 64 + (threadIdx.x & 63);
-    const int x = blockIdx.y * kWavesPerGroup + (threadIdx.x >> 6);
     const float dt = ctl ? split_timestep(ctl->smax[slot].value(), v.dx) : dtFixed;
-    if (x <= v.nx + 1 && y <= v.ny + 1) {
+    for (int x = blockIdx.y * kWavesPerGroup + (threadIdx.x >> 6); x <= v.nx + 1 && y <= v.ny + 1;
+         x += gridDim.y * kWavesPerGroup) {
         const size_t c = idx(v, x, y);
         if (x >= 1 && x <= v.nx && y >= 1 && y <= v.ny) {
             const float dtdx = dt / v.dx;
@@ -364,7 +367,7 @@ int launch_ctl_reset(DeviceCtl* ctl, int par, hipStream_t stream) {
 
 int launch_apply_s(StateView v, SumsView sums, StateView o, float dtFixed, DeviceCtl* ctl, int slot, float* dtLog,
                    int logIdx, hipStream_t stream) {
-    const dim3 grid((v.ny + 2 + 63) / 64, (v.nx + 2 + kWavesPerGroup - 1) / kWavesPerGroup);
+    const dim3 grid((v.ny + 2 + 63) / 64, std::min((v.nx + 2 + kWavesPerGroup - 1) / kWavesPerGroup, 65535));
     hipLaunchKernelGGL(apply_s_kernel, grid, dim3(64 * kWavesPerGroup), 0, stream, v, sums, o, dtFixed, ctl, slot,
                        dtLog, logIdx);
     hipError_t e = hipGetLastError();
