@@ -63,6 +63,12 @@ def measured_valu(xseg: int):
     return profile_field("valu_wave_instructions_per_launch")
 
 
+def width_name(xseg: int):
+    """Columns per strip as asked for.  Left to the block (-1), a launch may run
+    narrower strips than swe_hip_get_tuning reports."""
+    return "automatic" if xseg == -1 else xseg
+
+
 def cpu_threads() -> int:
     try:
         return len(os.sched_getaffinity(0))
@@ -378,7 +384,7 @@ def every_tile_line(swe, state, steps: int, xseg: int):
     n = h.shape[0] - 2
     with swe.SweBlock(n, n, dx, dy, solver=swe.AUGRIE) as blk:
         blk.set_boundaries(bnd)
-        blk.set_tuning(-1, xseg)
+        blk.set_tuning(-1, xseg)  # -1: the block's own choice, as on the headline
         blk.set_quiet_skip(False)
         blk.upload(h, hu, hv, b)
         blk.run(10, want_dts=False)  # warm-up
@@ -387,7 +393,7 @@ def every_tile_line(swe, state, steps: int, xseg: int):
     v = n * n * steps / (total_ms * 1e-3) / 1e6
     return {"workload": "the headline workload with every strip tile computed every step (quiet-tile skipping off)",
             "value": round(v, 3), "unit": "MCell-updates/s", "ms_per_step": round(total_ms / steps, 6),
-            "fused_kernel_avg_us": round(kms[1] / max(kl[1], 1) * 1e3, 3), "xseg": xseg}
+            "fused_kernel_avg_us": round(kms[1] / max(kl[1], 1) * 1e3, 3), "xseg": width_name(xseg)}
 
 
 def per_call_line(state, steps: int, warmup: int):
@@ -444,13 +450,12 @@ def disturbed_line(swe, scenarios, n: int, seed: int, steps: int, noise: float =
         blk.run(10, want_dts=False)  # warm-up
         blk.upload(h, hu, hv, b)
         _, total_ms, kms, kl = timed_run(swe, blk, steps, per_kernel=True)
-        xseg = blk.get_tuning()[1]
     v = n * n * steps / (total_ms * 1e-3) / 1e6
     fused_us = kms[1] / max(kl[1], 1) * 1e3
     return {"workload": f"{n}x{n} islands dam break (seed {seed}) with uniform surface noise +-{noise} m on every "
                         f"cell (seed {seed + 1}), AugRie FP32, {steps} steps from t=0",
             "value": round(v, 3), "unit": "MCell-updates/s", "ms_per_step": round(total_ms / steps, 6),
-            "fused_kernel_avg_us": round(fused_us, 3), "xseg": xseg,
+            "fused_kernel_avg_us": round(fused_us, 3), "xseg": width_name(-1),
             "hbm_frac_algorithmic": round(BYTES_PER_CELL * n * n / (fused_us * 1e-6) / 1e9 / HBM_PEAK_GBS, 5)}
 
 
@@ -672,7 +677,7 @@ def main() -> int:
                         f"outflow boundaries, {args.steps} steps from t=0",
             "cells": cells,
             "strategy": ["recompute", "store", "fused"][strategy],
-            "xseg": xseg,
+            "xseg": width_name(args.xseg),
             "simulated_s": round(t_sim, 6),
             "wall_s_incl_sync": round(wall_s, 4),
         },
@@ -702,7 +707,7 @@ def main() -> int:
         print(json.dumps(line))
         return 0
     line["init"] = seeded_init_line(swe, scenarios, n, args.seed, (h, hu, hv, b), dx, bnd, host_gen_s)
-    line["every_tile"] = every_tile_line(swe, (h, hu, hv, b, dx, dy, bnd), args.steps, xseg)
+    line["every_tile"] = every_tile_line(swe, (h, hu, hv, b, dx, dy, bnd), args.steps, args.xseg)
     line["every_tile"]["vs_headline"] = round(line["every_tile"]["value"] / mcells, 4)
     line["per_call"] = per_call_line((h, hu, hv, b, dx, dy, bnd), args.steps, args.warmup)
     if "value" in line["per_call"]:

@@ -290,18 +290,24 @@ int swe_hip_solve_edges(int solver, int math, int64_t n, const float* hL, const 
  * + update pass), 1 = store (flux pass writing 4 net-update sums + apply
  * pass), 2 = fused (one launch per step that applies the previous update on
  * load, or, with the IEEE arithmetic, for HLLE and f-wave on blocks of 2^19
- * cells and more and for Hybrid from 6 * 2^20, one that updates and takes the new state's CFL maximum; the
- * default); xseg = x columns per wavefront strip (4, 8, 10, 12,
- * 16 or 32; the sweeps of strategies 0 and 1 run 4 as 16); -1 keeps the
- * current value.  All strategies and widths give
- * identical results.  Until the caller sets xseg, a block uses the widest of
- * 16 and 12 for which nyt * ceil(nx/xseg) / (CUs * 4) reaches the solver's
- * threshold (nyt = ceil(ny/62); AugRie 12, 4; with a learned middle state
- * attached 5, 3; HLLE, f-wave, Hybrid 2, 1), else 8 (swe_hip_set_surrogate
- * re-picks it); with strategy 2 a block that does not fill the GPU at that
- * width runs strips of 1 to 8 columns instead (the one-pass launch picks 8, 16
- * or 32).  The fused loop skips quiet tiles (swe_hip_set_quiet_skip)
- * at widths that are multiples of 4. */
+ * cells and more and for Hybrid from 6 * 2^20, one that updates and takes the
+ * new state's CFL maximum, the one-pass step; the default); xseg = x columns
+ * per wavefront strip (4, 8, 10, 12, 16 or 32); -1 keeps the current value.  A
+ * pass without a kernel of the width runs another: the sweeps 8 for 10 and,
+ * but for the IEEE store pass, 16 for 4; the one-pass step (8, 16, 32) and
+ * flavour S (4, 8, 16) the next narrower one, at least their narrowest.  All
+ * strategies and widths give identical results.
+ *
+ * Until the caller sets xseg, a block uses the widest of 16 and 12 for which
+ * nyt * ceil(nx/xseg) / (CUs * 4) reaches the solver's threshold (nyt =
+ * ceil(ny/62); AugRie 12, 4; with a learned middle state attached 5, 3; HLLE,
+ * f-wave, Hybrid 2, 1), else 8 (swe_hip_set_surrogate re-picks it).  That is the
+ * width swe_hip_get_tuning reports; what a launch of strategy 2 runs then may
+ * be less: the one-pass step picks 8, 16 or 32 by its own rule, a block that
+ * does not fill the GPU runs strips of 1 to 8 columns, and Hybrid never more
+ * than 8.  Passing the reported width to swe_hip_set_tuning makes every launch
+ * run it.  The fused loop skips quiet tiles (swe_hip_set_quiet_skip) at widths
+ * that are multiples of 4. */
 int swe_hip_set_tuning(swe_hip_block* blk, int strategy, int xseg);
 int swe_hip_get_tuning(swe_hip_block* blk, int* strategy, int* xseg);
 
@@ -315,9 +321,9 @@ int swe_hip_get_tuning(swe_hip_block* blk, int* strategy, int* xseg);
  * all six).  ms_per_step (may be null) receives the per-step times in that
  * order.  With the fused strategy
  * and the HLLE or f-wave solver it also times the recompute strategy (0) at
- * 16 and 32 columns and keeps it if faster: on blocks that do not fit the
- * GPU's caches recompute moves fewer bytes per cell (swe_hip_get_tuning
- * reports the strategy kept).  Results of later runs do not depend on the
+ * 16 and 32 columns and keeps it if faster (swe_hip_get_tuning reports the
+ * strategy kept); with the fast arithmetic, which has no one-pass step, that
+ * moves fewer bytes per cell on blocks that do not fit the GPU's caches.  Results of later runs do not depend on the
  * choice.  Allocates and frees 3 fields of scratch. */
 #define SWE_HIP_TUNE_WIDTHS 6
 int swe_hip_autotune(swe_hip_block* blk, int steps, float* ms_per_step);
@@ -375,7 +381,11 @@ int swe_hip_run_noalloc(int nx, int ny, float dx, float dy, int solver, const in
  *   1 = fast: FMA contraction, hardware reciprocal and square root; results
  *       differ from the IEEE variant by rounding only (about 1e-2 relative
  *       L-infinity after 500 steps of a wet/dry dam break, the same order as
- *       the difference between FP32 and FP64 runs of the scheme). */
+ *       the difference between FP32 and FP64 runs of the scheme).  It keeps the
+ *       general form of the solvers and the wider strips, so it is not the
+ *       faster one any more: 2048^2 AugRie 34 against 30 us per step on the
+ *       islands dam break and 137 against 85 with every cell moving, HLLE 56
+ *       against 46, Hybrid 101 against 71. */
 int swe_hip_set_math(swe_hip_block* blk, int math);
 
 #ifdef __cplusplus

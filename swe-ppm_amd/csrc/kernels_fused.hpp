@@ -68,10 +68,10 @@ constexpr unsigned kQuietAll = 1u, kQuietBottom = 2u, kQuietTop = 4u, kQuietLeft
 // Record tiles are kQuietCols columns wide; a wave's segment of XS columns
 // spans XS / kQuietCols of them.  A launch with few busy tiles lasts as long as
 // one of them, whose columns are a chain of dependent operations.  us per step
-// with tiles of 4 / 2 / 1 columns: 1024^2 islands 33.8 / 26.8 / 24.4, 2048^2 islands
-// from the start 37.0 / 31.1 / 31.7 and from step 400 67 / 55 / 60, 4096^2 trench
-// from the start 35.8 / 32.0 / 35.6 and from step 600 48.7 / 49.3 / 53.9, every cell
-// moving 2048^2 104 / 104 / 108, 4096^2 332 / 341 / 351: one column solves an edge
+// with tiles of 4 / 2 / 1 columns: 1024^2 islands 34.4 / 26.6 / 24.7, 2048^2 islands
+// from the start 36.4 / 30.0 / 30.7 and from step 400 56.3 / 55.7 / 56.8, 4096^2 trench
+// from the start 37.5 / 37.8 / 41.4 and from step 600 53.4 / 57.2 / 62.5, every cell
+// moving 2048^2 84.8 / 85.4 / 87.6, 4096^2 301 / 301 / 313: one column solves an edge
 // column twice per column and doubles the plan's work.
 constexpr int kQuietCols = 2;
 constexpr int kRecordWidth = 4;  // strip widths with a record are multiples of this
@@ -82,8 +82,8 @@ constexpr long kMaxSegments = 1l << (32 - 2 * kEntryBits);
 // Waves the quiet-tile plan aims to fill with busy record tiles before it
 // lengthens the pieces it lists: eight per SIMD of the chip.  Measured with 4096 /
 // 6144 / 8192 (us per step, strips of 8 columns at 2048^2, of 16 at 4096^2): 2048^2
-// islands from step 400 66 / 61 / 54, every cell moving 108 / 104 / 105; 4096^2
-// islands from step 300 105 / 90 / 90, trench from step 600 51 / 49 / 50.  Shorter
+// islands from step 400 61.9 / 62.3 / 55.7, every cell moving 84.5 / 84.7 / 85.4; 4096^2
+// islands from step 300 102 / 92.5 / 89.0, trench from step 600 55.3 / 56.9 / 57.2.  Shorter
 // pieces give more waves to hide the busy tiles' latency but solve more halo
 // edges.
 constexpr unsigned kPlanWaves = 8192;

@@ -17,7 +17,8 @@
 //     lane-1 the same way.
 // Each interior edge is solved once per strip (plus one halo x-edge per
 // segment), net updates never leave registers, and the CFL maximum is
-// reduced in-wave before one atomic per wave.
+// reduced in-wave; a wave raises its die's word of it only where its own is
+// larger (raise_max).
 //
 // Modes:
 //   MODE_MAX    edges -> max speed only (first half of the two-pass step);

@@ -81,15 +81,15 @@ __global__ void apply_bc_bathymetry_kernel(float* b, int nx, int ny, int pitch, 
 // carries its speed into slot step & 1 and into the CFL maximum of slot
 // slotOut.  The record tiles of a segment from its first to its last busy
 // one are listed in pieces of at most `piece` tiles,
-// (segment << 6) | (first << 3) | (length - 1); workgroup g keeps its
-// entries in segment order at list[g * kPlanGroup ...] and
+// (segment << 8) | (first << 4) | (length - 1) (kEntryBits); workgroup g keeps
+// its entries in segment order at list[g * kPlanGroup ...] and
 // their number in count[g].  piece adapts to the load: busy tiles found by
 // the previous launch's plan over kPlanWaves, between 1 and `fine` (with few
 // busy tiles short pieces spread them over more waves, the busiest wave sets
 // the launch time; with many, long pieces solve fewer halo edges).  The
 // number of busy tiles goes to ctl->busy[slotOut].  rbSeq != 0: the plan also
-// reports the previous launch's CFL maximum to the host, as readback_kernel
-// does (one kernel less between a flux pass and the next).
+// reports the previous launch's CFL maximum to the host, as the fused launch
+// does where no plan precedes it.
 __global__ __launch_bounds__(kPlanGroup) void quiet_plan_kernel(const unsigned* __restrict__ quiet, float* speed,
                                                                 int nyt, int nxs, int nxf, int fine, int lanes,
                                                                 int step, DeviceCtl* ctl, int slotPrev3, int slotOut,

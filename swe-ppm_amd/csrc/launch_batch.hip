@@ -43,7 +43,7 @@ template <int S>
 int launch_batch_fused_solver(int xs, int groups, int direct, BatchArena A, const BatchBlockDesc* D,
                               BatchBlockState* st, BatchGlobals* G, const int* items, uint2* deferQ,
                               const GhostJob* jobs, const GhostGeom* geo, hipStream_t stream) {
-        const dim3 grid(groups), block(64 * (direct ? direct : kWavesPerGroup));
+    const dim3 grid(groups), block(64 * (direct ? direct : kWavesPerGroup));
     switch (xs) {
         case 4:
             hipLaunchKernelGGL((batch_fused_kernel<S, 4>), grid, block, 0, stream, A, D, st, G, items, direct, deferQ,

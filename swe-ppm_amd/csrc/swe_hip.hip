@@ -167,15 +167,19 @@ constexpr long kAdvanceCells = 1l << 19, kAdvanceCellsHybrid = 3l << 21;
 // Widths are whole numbers of kRecordWidth columns (two record tiles), so that
 // quiet tiles can be skipped (10 columns, the old third choice, measured
 // within 1% of 8 where it won).  4, 10 and 32 stay available through
-// swe_hip_set_tuning.  Measured without skipping, radial dam break over
-// bathymetry, us per step at 8/10/12/16/32 columns:
-//   AugRie 1024^2  73.5 / 72.7 / 80.2 / 99.9 / 176   (picks 10)
-//          2048^2   156 /  145 /  143 /  161 / 215   (12)
-//          3000^2   299 /  266 /  259 /  268 / 309   (12)
-//          4096^2   514 /  423 /  413 /  414 / 467   (16; the trench 4096^2: 424 at 12, 416 at 16)
-//          8192^2  1879 / 1417 / 1387 / 1346 / 1360  (16)
-//   learned 2048^2  181 /  174 /  166 /  172 / 220   (12); 3000^2: 285 at 12, 280 at 16 (16)
-//   HLLE 2048^2     129 /  116 /  105 /   95 /  90   (16); f-wave 134 / 122 / 104 / 96 / 100 (16)
+// swe_hip_set_tuning.  Measured without skipping, islands dam break, after the
+// bar with every cell moving, us per step at 8/10/12/16/32 columns:
+//   AugRie 1024^2    48 /   52 /   64 /   80 / 149  |   49 /   53 /   64 /   80 / 147   (picks 8)
+//          2048^2    71 /   72 /   77 /   86 / 146  |   81 /   81 /   84 /   95 / 147   (12)
+//          3000^2   152 /  152 /  158 /  169 / 204  |  165 /  160 /  164 /  172 / 199   (12)
+//          4096^2   266 /  267 /  274 /  283 / 323  |  286 /  280 /  290 /  297 / 319   (16)
+//          8192^2  1009 / 1050 / 1054 / 1068 / 1113                                     (16)
+//   learned 2048^2   98 /  113 /  122 /  139 / 226   (12); 3000^2: 187 / 186 / 205 / 211 / 289 (16)
+// The thresholds date from edges about twice as dear, when 12 and 16 columns won
+// from 2048^2 on; where narrow_width does not step in they now cost up to 8%, with
+// the learned middle state up to 25% (not re-tuned yet).  The light solvers'
+// widths matter for the fast arithmetic alone, which takes them from 2048^2 on
+// (HLLE 58 / 58 / 58 / 55 / 57, f-wave 59 / 58 / 57 / 58 / 66: 16).
 int default_xseg(int nx, int ny, int solver, int cus) {
     if (cus <= 0) return 8;
     const double strips = (double)((ny + kStripRows - 1) / kStripRows);
@@ -218,19 +222,23 @@ int advance_width(const swe_hip_block* k) {
 // once a SIMD has a few waves the halo column per strip costs more than
 // that saves.  The narrowest width is taken whose waves per SIMD stay below
 // the solver's limit.  Measured, us per step at 1 / 2 / 4 / 8 columns:
-//   f-wave 64x50     7.1 /  8.7 / 10.7 / 14.3     256^2   13.2 / 11.1 / 12.7 / 18.0
-//          512^2    22.1 / 16.9 / 15.7 / 19.2     1000x500 34.1 / 25.6 / 19.2 / 21.1
-//   Hybrid 64x50    13.9 / 16.9 / 21.6 / 25.1     256^2   18.3 / 20.4 / 31.6 / 47.6
-//          512^2    27.0 / 24.5 / 34.4 / 53.7     1500x901 47.3 / 48.9 / 45.2 / 54.6
-//          2048^2   90.8 / 80.3 / 75.0 / 71.5     4096^2   341 / 306 / 282 / 280
+//   f-wave 64x50     6.5 /  8.0 / 10.8 / 15.9     256^2   10.4 /  9.2 / 11.6 / 17.1
+//          512^2    21.6 / 16.0 / 15.4 / 18.7     1000x500 31.2 / 22.3 / 17.8 / 20.2
+//   HLLE   64x50     5.7 /  7.1 /  8.6 / 12.4     256^2    9.4 /  9.3 /  9.6 / 13.2
+//          512^2    23.1 / 17.1 / 14.7 / 15.2     1000x500 29.8 / 22.7 / 16.8 / 17.5
+//   Hybrid 64x50    15.4 / 20.3 / 28.8 / 41.8     256^2   13.2 / 18.0 / 28.4 / 48.1
+//          512^2    22.0 / 20.4 / 29.9 / 50.8     1500x901 44.7 / 40.6 / 37.7 / 48.7
+//          2048^2   83.3 / 70.2 / 70.2 / 73.2     4096^2   313 / 289 / 270 / 271
 //   AugRie, islands and (after the bar) every cell moving
-//          64x50    11.4 / 15.7 / 21.6 / 21.7     256^2   12.5 / 16.9 / 23.3 / 24.1 | 13.6 / 16.8 / 23.2 / 23.5
-//          512^2    20.1 / 19.3 / 24.8 / 24.9 | 20.8 / 21.4 / 28.7 / 28.9
-//          1000x500 35.3 / 26.8 / 25.2 / 25.7 | 30.3 / 26.9 / 34.5 / 35.3
-//          1024^2   41.0 / 37.7 / 26.6 / 27.0 | 42.0 / 40.4 / 48.7 / 48.4
-//          2048^2     -  /   -  / 30.7 / 31.0 |   -  /   -  /  112 / 105   (12 columns: 31.1 | 115)
+//          64x50    12.2 / 16.4 / 21.5 / 21.8 | 11.9 / 16.3 / 21.2 / 22.2
+//          256^2    12.5 / 16.3 / 22.9 / 24.0 | 13.0 / 16.7 / 22.8 / 23.8
+//          512^2    19.9 / 18.9 / 24.0 / 25.0 | 20.2 / 20.5 / 27.1 / 28.9
+//          1000x500 30.7 / 24.2 / 24.7 / 26.0 | 29.6 / 24.5 / 30.3 / 34.4
+//          1024^2   39.7 / 34.4 / 25.8 / 26.8 | 36.0 / 35.9 / 42.1 / 42.6
+//          2048^2     -  / 64.5 / 31.1 / 31.9 |   -  / 83.0 / 86.5 / 86.7   (12 columns: 32.8 | 98.2)
 // (AugRie's 4 columns and more record and skip quiet tiles, which the narrower
-// ones do not: there a lake at rest is solved edge by edge.)
+// ones do not: there a lake at rest is solved edge by edge, which is why 1024^2
+// takes 8 columns although 2 win once every cell moves.)
 int narrow_width(int nx, int ny, int solver, int cus) {
     struct Limit {
         int width = 0;  // 0: end of the list

@@ -101,7 +101,7 @@ int launch_fused_u_solver(int xseg, StateView v, FusedIO io, BoundaryInfo bi, De
                           int slotClear, float* dtLog, int logIdx, hipStream_t stream);
 int launch_fused_u(int solver, int variant, int xseg, StateView v, FusedIO io, BoundaryInfo bi, DeviceCtl* ctl,
                    int slotIn, int slotOut, int slotClear, float* dtLog, int logIdx, hipStream_t stream);
-// One-pass step of the light solvers (kernels_advance.hpp; HLLE or f-wave).
+// One-pass step of the light solvers (kernels_advance.hpp; HLLE, f-wave, Hybrid).
 template <int S>
 int launch_advance_u_solver(int xseg, StateView v, float* hn, float* hun, float* hvn, BoundaryInfo bi, DeviceCtl* ctl,
                             int slotIn, int slotOut, int slotClear, int last, float* dtLog, int logIdx,
