@@ -185,14 +185,15 @@ __global__ void ctl_reset_kernel(DeviceCtl* ctl, int par) {
 // slot `slot`, which is logged.  In place or, where o is another buffer, into
 // it: then the ghost cells go over unchanged.  One cell per thread, every load
 // in flight at once: the pass streams 40 bytes per cell (1024^2: 13.8 us with 16
-// cells a thread).  (Blocks of more columns than a grid's second dimension holds
-// at kWavesPerGroup each go round again.)
+// cells a thread).  Columns go over the grid's second dimension, kSplitGroups
+// workgroups of kWavesPerGroup (it holds 65536), and from there over the third.
+constexpr int kSplitGroups = 32768;
 __global__ __launch_bounds__(256) void apply_s_kernel(StateView v, SumsView sums, StateView o, float dtFixed,
                                                       DeviceCtl* ctl, int slot, float* dtLog, int logIdx) {
     const int y = blockIdx.x * 64 + (threadIdx.x & 63);
     const float dt = ctl ? split_timestep(ctl->smax[slot].value(), v.dx) : dtFixed;
-    for (int x = blockIdx.y * kWavesPerGroup + (threadIdx.x >> 6); x <= v.nx + 1 && y <= v.ny + 1;
-         x += gridDim.y * kWavesPerGroup) {
+    const int x = (blockIdx.z * kSplitGroups + blockIdx.y) * kWavesPerGroup + (threadIdx.x >> 6);
+    if (x <= v.nx + 1 && y <= v.ny + 1) {
         const size_t c = idx(v, x, y);
         if (x >= 1 && x <= v.nx && y >= 1 && y <= v.ny) {
             const float dtdx = dt / v.dx;
@@ -207,7 +208,7 @@ __global__ __launch_bounds__(256) void apply_s_kernel(StateView v, SumsView sums
             o.hv[c] = v.hv[c];
         }
     }
-    if (ctl && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) {
+    if (ctl && blockIdx.x == 0 && blockIdx.y == 0 && blockIdx.z == 0 && threadIdx.x == 0) {
         ctl->dt = dt;
         ctl->t += dt;
         ctl->steps += 1;
@@ -367,7 +368,8 @@ int launch_ctl_reset(DeviceCtl* ctl, int par, hipStream_t stream) {
 
 int launch_apply_s(StateView v, SumsView sums, StateView o, float dtFixed, DeviceCtl* ctl, int slot, float* dtLog,
                    int logIdx, hipStream_t stream) {
-    const dim3 grid((v.ny + 2 + 63) / 64, std::min((v.nx + 2 + kWavesPerGroup - 1) / kWavesPerGroup, 65535));
+    const int groups = (v.nx + 2 + kWavesPerGroup - 1) / kWavesPerGroup;
+    const dim3 grid((v.ny + 2 + 63) / 64, std::min(groups, kSplitGroups), (groups + kSplitGroups - 1) / kSplitGroups);
     hipLaunchKernelGGL(apply_s_kernel, grid, dim3(64 * kWavesPerGroup), 0, stream, v, sums, o, dtFixed, ctl, slot,
                        dtLog, logIdx);
     hipError_t e = hipGetLastError();

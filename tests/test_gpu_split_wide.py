@@ -8,7 +8,7 @@ from helpers import same_bits
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("nx", [4 * 65535 - 2, 4 * 65535 - 1, 600_001])
+@pytest.mark.parametrize("nx", [4 * 32768 - 2, 4 * 32768 - 1, 4 * 65535 - 2, 4 * 65535 - 1, 600_001])
 def test_wide_block(swe, oracle, nx):
     ny, steps, bnd = 3, 2, [0, 1, 0, 0]
     rng = np.random.default_rng(nx)
